@@ -87,10 +87,11 @@ struct Carver {
     }
 };
 
-// t_emb = linear_2(silu(linear_1(t_sin))) and the three consumers' inputs
+// silu(t_emb), t_emb = linear_2(silu(linear_1(t_sin))): its consumers (modulation.1,
+// norm_out.linear) all take silu(t_emb)
 int time_embed(qimm_model *m, const float *t_sin, int64_t batch, float *tmp, float *temb, hipStream_t s) {
     const int64_t hid = m->cfg.hidden;
-    QIMM_HIP(m->ctx, qimm::launch_linear_f32(t_sin, kTimeDim, m->t1, batch, hid, kTimeDim, qimm::ACT_NONE, tmp, hid, s));
+    QIMM_HIP(m->ctx, qimm::launch_linear_f32(t_sin, kTimeDim, m->t1, batch, hid, kTimeDim, qimm::ACT_SILU, tmp, hid, s));
     QIMM_HIP(m->ctx, qimm::launch_linear_f32(tmp, hid, m->t2, batch, hid, hid, qimm::ACT_SILU, temb, hid, s));
     return QIMM_OK;
 }
@@ -192,7 +193,7 @@ int qimm_model_forward(qimm_model *m, const float *latents, int64_t batch, int64
     float *modv = c.take<float>(batch * 4 * hid), *scale = c.take<float>(batch * hid);
     // time embedding and modulation (:537-539)
     if ((rc = time_embed(m, t_sin, batch, tmp, temb, s))) return rc;
-    QIMM_HIP(ctx, qimm::launch_linear_f32(temb, hid, m->mod, batch, 4 * hid, hid, qimm::ACT_SILU, modv, 4 * hid, s));
+    QIMM_HIP(ctx, qimm::launch_linear_f32(temb, hid, m->mod, batch, 4 * hid, hid, qimm::ACT_NONE, modv, 4 * hid, s));
     // target = img_in(latents) (:483)
     QIMM_HIP(ctx, qimm::launch_linear_f32(latents, ch, m->img_in, rows, hid, ch, qimm::ACT_NONE, h, hid, s));
     // the blocks, in place (:538-543)
@@ -205,7 +206,7 @@ int qimm_model_forward(qimm_model *m, const float *latents, int64_t batch, int64
         if (rc) return rc;
     }
     // norm_out and proj_out (:545, 300-309)
-    QIMM_HIP(ctx, qimm::launch_linear_f32(temb, hid, m->norm_out, batch, hid, hid, qimm::ACT_SILU, scale, hid, s));
+    QIMM_HIP(ctx, qimm::launch_linear_f32(temb, hid, m->norm_out, batch, hid, hid, qimm::ACT_NONE, scale, hid, s));
     QIMM_HIP(ctx, qimm::launch_rows_ln_scale(h, scale, rows, hid, seq, kEps, h, s));
     QIMM_HIP(ctx, qimm::launch_linear_f32(h, hid, m->proj_out, rows, ch, hid, qimm::ACT_NONE, pred, ch, s));
     return QIMM_OK;
@@ -251,8 +252,8 @@ int qimm_model_prefix_fill(qimm_model *m, const float *txt, int64_t text_len, co
     if (text_len) {
         if (jd) {
             QIMM_HIP(ctx, qimm::launch_rows_rmsnorm(txt, m->txt_norm, trows, jd, kEps, tn, s));
-            QIMM_HIP(ctx, qimm::launch_linear_f32(tn, jd, m->txt_in, trows, hid, jd, qimm::ACT_NONE, tmid, hid, s));
-            QIMM_HIP(ctx, qimm::launch_linear_f32(tmid, hid, m->txt_out, trows, hid, hid, qimm::ACT_GELU_TANH, tx, hid, s));
+            QIMM_HIP(ctx, qimm::launch_linear_f32(tn, jd, m->txt_in, trows, hid, jd, qimm::ACT_GELU_TANH, tmid, hid, s));
+            QIMM_HIP(ctx, qimm::launch_linear_f32(tmid, hid, m->txt_out, trows, hid, hid, qimm::ACT_NONE, tx, hid, s));
             txt_h = tx;
         }
     }
@@ -271,15 +272,9 @@ int qimm_model_prefix_fill(qimm_model *m, const float *txt, int64_t text_len, co
         at += len;
     }
     // zero_modulation: the t = 0 sinusoid [1 .. 1, 0 .. 0] through the embedder (:334-343)
-    {
-        std::vector<float> z((size_t)batch * kTimeDim, 0.f);
-        for (int64_t b = 0; b < batch; b++)
-            for (int i = 0; i < kTimeDim / 2; i++) z[(size_t)b * kTimeDim + i] = 1.0f;
-        QIMM_HIP(ctx, hipMemcpyAsync(tsin, z.data(), z.size() * 4, hipMemcpyHostToDevice, s));
-        QIMM_HIP(ctx, hipStreamSynchronize(s));
-    }
+    QIMM_HIP(ctx, qimm::launch_zero_sinusoid(tsin, batch, kTimeDim, s));
     if ((rc = time_embed(m, tsin, batch, tmp, temb, s))) return rc;
-    QIMM_HIP(ctx, qimm::launch_linear_f32(temb, hid, m->mod, batch, 4 * hid, hid, qimm::ACT_SILU, modv, 4 * hid, s));
+    QIMM_HIP(ctx, qimm::launch_linear_f32(temb, hid, m->mod, batch, 4 * hid, hid, qimm::ACT_NONE, modv, 4 * hid, s));
     // every block under the block-causal mask, keeping its k, v (:383-391)
     qimm_attn_mask mask{image_ids, key_valid};
     for (int64_t i = 0; i < m->cfg.layers; i++) {

@@ -211,9 +211,11 @@ hipError_t launch_transpose_sd(const uint16_t *in, int64_t bh, int64_t s, uint16
 
 // ---- the denoising step around the blocks (step.hip), all f32 ----
 enum : int { ACT_NONE = 0, ACT_SILU = 1, ACT_GELU_TANH = 2 };
-// y[m][n] (row stride ldy) = sum_k act(x[m][k]) * w[n][k]; x row stride ldx, w [n][k] dense.
+// y[m][n] (row stride ldy) = act(sum_k x[m][k] * w[n][k]); x row stride ldx, w [n][k] dense.
 hipError_t launch_linear_f32(const float *x, int64_t ldx, const float *w, int64_t m, int64_t n, int64_t k,
-                             int act_in, float *y, int64_t ldy, hipStream_t stream);
+                             int act_out, float *y, int64_t ldy, hipStream_t stream);
+// out[rows][width] = 1 in each row's first half, 0 in its second (the t = 0 timestep embedding)
+hipError_t launch_zero_sinusoid(float *out, int64_t rows, int64_t width, hipStream_t stream);
 // y = x / sqrt(mean(x^2) + eps) * w, per row of d values
 hipError_t launch_rows_rmsnorm(const float *x, const float *w, int64_t rows, int64_t d, float eps, float *y,
                                hipStream_t stream);

@@ -343,3 +343,38 @@ def test_model_full_size_prefix_fill_and_forward(torch_cuda, qctx):
     c, m = cos_sim(got[rows], ref), max_abs_rel(got[rows], ref)
     print(f"prediction rows: cos {c:.7f} mar {m:.2e}", flush=True)
     assert c >= 0.9999 and m <= 2e-2
+
+
+@pytest.mark.parametrize("ch,hid,b,sh,sw", [
+    (64, 256, 1, 4, 8),      # one timestep row; tiles with one wave per column tile (K < 512)
+    (64, 768, 3, 5, 7),      # three rows in one pass; K shared by eight waves, 16-token tiles, ragged tokens
+    (48, 1056, 9, 3, 5),     # nine rows: matrix instructions; 33 runs of k, 48 output columns of a 64-column tile
+    (16, 4608, 5, 2, 3),     # two passes of rows, two LDS chunks of k
+    (20, 256, 2, 3, 3),      # K % 16 != 0: the kernel for any sizes
+    (1024, 2048, 2, 8, 16),  # 32-token tiles with K shared by eight waves
+])
+def test_global_linears_by_size(torch_cuda, qctx, ch, hid, b, sh, sw):
+    """The f32 global linears over the sizes that pick their kernels, through a
+    model without blocks, against the f64 oracle: f32 sums of up to 4608 terms
+    through five products and a LayerNorm stay within 1e-4 of the largest value
+    (2^-24 sqrt(K) per product is 4e-6)."""
+    torch = torch_cuda
+    rng = np.random.default_rng(ch + hid)
+    g = {n: synth.weight(rng, synth.F32, r, k, std=k ** -0.5) for n, r, k in (
+        ("img_in", hid, ch), ("t_linear_1", hid, 256), ("t_linear_2", hid, hid), ("modulation", 4 * hid, hid),
+        ("norm_out", hid, hid), ("proj_out", ch, hid))}
+    keep, T = [], qimm.ModelTensors()
+    for name, (t, data, rows, cols) in g.items():
+        setattr(T, name, qimm.make_tensor(t, rows, cols, data.tobytes(), keep))
+    mdl = qctx.model_create(qimm.ModelConfig(ch, 0, hid, 0), T, [])
+    s = sh * sw
+    latents = rng.standard_normal((b, s, ch)).astype(np.float32)
+    ts = [0.9 - 0.07 * i for i in range(b)]
+    lat_d, tsd, pe_d = dev(torch, latents), t_sin_dev(torch, qctx, ts), dev(torch, np.zeros((s, 128), np.float32))
+    pred = torch.full((b, s, ch), float("nan"), dtype=torch.float32, device="cuda")
+    mdl.forward(lat_d.data_ptr(), b, s, tsd.data_ptr(), pe_d.data_ptr(), None, pred.data_ptr(), None, stream(torch))
+    got = host(pred)
+    temb = OM.time_embed(g, O.timestep_embedding(np.array(ts, np.float32)))
+    want = OM.final_layer(g, OM.linear(g["img_in"], latents), temb)
+    assert max_abs_rel(got, want) <= 1e-4, max_abs_rel(got, want)
+    mdl.free()
