@@ -213,7 +213,7 @@ WsLayout ws_layout(const qimm_block *blk, int64_t batch, int64_t seq, int64_t mo
     L.xn = off; off += align_up((size_t)(M * hid) * 2);
     L.q = off; off += align_up((size_t)(M * hid) * 2);
     L.k = off; off += align_up((size_t)(M * hid) * 2);
-    L.vt = off; off += align_up((size_t)(M * hid) * 2);
+    L.vt = off; off += align_up((size_t)(batch * qimm::vt_ld(seq) * hid) * 2);
     L.att = off; off += align_up((size_t)(M * hid) * 2);
     L.h = off; off += align_up((size_t)(M * F) * 2);
     L.lim = off; off += align_up((size_t)seq * 4);  // per-query key limits of the block-causal mask
@@ -247,12 +247,10 @@ int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t ba
     if (!aligned16(x) || !aligned16(x_out) || !aligned16(mod) || !aligned16(pe) ||
         (k_out && !aligned16(k_out)) || (v_out && !aligned16(v_out)))
         return set_err(ctx, QIMM_ERR_ARG, "block forward: device pointers must be 16-byte aligned");
-    int64_t P = 0;
     if (kv) {
         if (kv->batch != batch || kv->heads != H)
             return set_err(ctx, QIMM_ERR_SHAPE, "block forward: cache batch/heads differ from the block call");
         if (layer < 0 || layer >= kv->layers) return set_err(ctx, QIMM_ERR_SHAPE, "block forward: cache layer out of range");
-        P = kv->prefix;
     }
     const int64_t M = batch * seq;
     hipStream_t s = (hipStream_t)stream;
@@ -296,6 +294,7 @@ int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t ba
     ep.q = qb;
     ep.k = kb;
     ep.vt = vt;
+    ep.vt_ld = qimm::vt_ld(seq);
     ep.v_bhsd = v_out;
     ep.norm_q = blk->norm_q;
     ep.norm_k = blk->norm_k;
@@ -325,9 +324,9 @@ int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t ba
     }
     STAGE_MARK(2);
     // attention over [prefix ; own]                            (:143-148)
-    const uint16_t *pk = nullptr, *pvt = nullptr;
+    qimm::KeySeg prefix{};
     if (kv) {
-        const int rc = kv_layer(kv, layer, s, &pk, &pvt);
+        const int rc = kv_layer(kv, layer, s, &prefix);
         if (rc) return rc;
     }
     // candle mode: to_out's activation rounding, done by the attention launch
@@ -337,14 +336,14 @@ int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t ba
     const bool round_sep = separate_rounding();
     const int att_q = round_sep ? 0 : qb_out;
     float *att_f32 = qb_out ? stage_f32 : nullptr;
+    const qimm::KeySeg own{kb, vt, seq, ep.vt_ld};
     // score bound: q and own k from the RmsNorm weights, prefix k from the cache
     const float *kpn = kv ? kv->knorm + layer : nullptr;
     if (img || kvalid)
-        QIMM_HIP(ctx, qimm::launch_attention_masked(qb, pk, pvt, P, kb, vt, seq, batch, H, seq, 1.0f, img, kvalid,
-                                                    (int32_t *)(ws + L.lim), att, s, att_f32, kpn,
+        QIMM_HIP(ctx, qimm::launch_attention_masked(qb, prefix, own, batch, H, seq, 1.0f, img, kvalid, (int32_t *)(ws + L.lim), att, s, att_f32, kpn,
                                                     blk->q_norm_bound, blk->k_norm_bound, att_q));
     else
-        QIMM_HIP(ctx, qimm::launch_attention_log2(qb, pk, pvt, P, kb, vt, seq, batch, H, seq, att, s, att_f32, kpn,
+        QIMM_HIP(ctx, qimm::launch_attention_log2(qb, prefix, own, batch, H, seq, att, s, att_f32, kpn,
                                                   blk->q_norm_bound, blk->k_norm_bound, att_q));
     if (kv) {
         const int rc = kv_release(kv, layer, s);
@@ -512,12 +511,12 @@ int qimm_attention(qimm_ctx *ctx, const uint16_t *q, int64_t batch, int64_t head
     }
     if (P + so == 0) return set_err(ctx, QIMM_ERR_SHAPE, "attention: no keys");
     const hipStream_t s = (hipStream_t)stream;
-    const uint16_t *pk = nullptr, *pvt = nullptr;
+    qimm::KeySeg prefix{};
     if (kv) {
-        const int rc = kv_layer(kv, layer, s, &pk, &pvt);
+        const int rc = kv_layer(kv, layer, s, &prefix);
         if (rc) return rc;
     }
-    QIMM_HIP(ctx, qimm::launch_attention(q, pk, pvt, P, k_own, vt_own, so, batch, heads, sq, scale, out, s));
+    QIMM_HIP(ctx, qimm::launch_attention(q, prefix, qimm::KeySeg{k_own, vt_own, so, so}, batch, heads, sq, scale, out, s));
     return kv ? kv_release(kv, layer, s) : QIMM_OK;
 }
 
@@ -548,13 +547,12 @@ int qimm_attention_masked(qimm_ctx *ctx, const uint16_t *q, int64_t batch, int64
         if (rc) return rc;
         lim = (int32_t *)ctx->ws;
     }
-    const uint16_t *pk = nullptr, *pvt = nullptr;
+    qimm::KeySeg prefix{};
     if (kv) {
-        const int rc = kv_layer(kv, layer, s, &pk, &pvt);
+        const int rc = kv_layer(kv, layer, s, &prefix);
         if (rc) return rc;
     }
-    QIMM_HIP(ctx, qimm::launch_attention_masked(q, pk, pvt, P, k_own, vt_own, so, batch, heads, sq,
-                                                scale * 1.4426950408889634f, mask->image_ids, mask->key_valid, lim,
+    QIMM_HIP(ctx, qimm::launch_attention_masked(q, prefix, qimm::KeySeg{k_own, vt_own, so, so}, batch, heads, sq, scale * 1.4426950408889634f, mask->image_ids, mask->key_valid, lim,
                                                 out, s));
     return kv ? kv_release(kv, layer, s) : QIMM_OK;
 }

@@ -221,9 +221,9 @@ qimm_kv::Slot *kv_claim(const qimm_kv *kv, int64_t layer, hipStream_t s, int &rc
 // Copies host layer `layer` into slot sl on s and records its ready event.
 int kv_stage(const qimm_kv *kv, qimm_kv::Slot *sl, int64_t layer, hipStream_t s) {
     qimm_ctx *ctx = kv->ctx;
-    const size_t bytes = (size_t)kv->layer_elems() * 2;
-    QIMM_HIP(ctx, hipMemcpyAsync(sl->k, kv->k + layer * kv->layer_elems(), bytes, hipMemcpyHostToDevice, s));
-    QIMM_HIP(ctx, hipMemcpyAsync(sl->vt, kv->vt + layer * kv->layer_elems(), bytes, hipMemcpyHostToDevice, s));
+    const int64_t n = kv->layer_elems(), nv = kv->vt_elems();
+    QIMM_HIP(ctx, hipMemcpyAsync(sl->k, kv->k + layer * n, (size_t)n * 2, hipMemcpyHostToDevice, s));
+    QIMM_HIP(ctx, hipMemcpyAsync(sl->vt, kv->vt + layer * nv, (size_t)nv * 2, hipMemcpyHostToDevice, s));
     QIMM_HIP(ctx, hipEventRecord(sl->ready, s));
     return QIMM_OK;
 }
@@ -232,16 +232,14 @@ int kv_stage(const qimm_kv *kv, qimm_kv::Slot *sl, int64_t layer, hipStream_t s)
 
 namespace qimm_host {
 
-int kv_layer(const qimm_kv *kv, int64_t layer, hipStream_t s, const uint16_t **k, const uint16_t **vt) {
+int kv_layer(const qimm_kv *kv, int64_t layer, hipStream_t s, qimm::KeySeg *seg) {
+    *seg = qimm::KeySeg{nullptr, nullptr, kv->prefix, qimm::vt_ld(kv->prefix)};
     if (!kv->host) {
-        *k = kv->k + layer * kv->layer_elems();
-        *vt = kv->vt + layer * kv->layer_elems();
+        seg->k = kv->k + layer * kv->layer_elems();
+        seg->vt = kv->vt + layer * kv->vt_elems();
         return QIMM_OK;
     }
-    if (!kv->layer_elems()) {
-        *k = *vt = nullptr;
-        return QIMM_OK;
-    }
+    if (!kv->layer_elems()) return QIMM_OK;
     qimm_kv::Slot *sl = nullptr;
     for (auto &x : kv->slot)
         if (x.layer == layer) sl = &x;
@@ -253,8 +251,8 @@ int kv_layer(const qimm_kv *kv, int64_t layer, hipStream_t s, const uint16_t **k
         if (!sl) return rc;
         if ((rc = kv_stage(kv, sl, layer, s))) return rc;
     }
-    *k = sl->k;
-    *vt = sl->vt;
+    seg->k = sl->k;
+    seg->vt = sl->vt;
     return QIMM_OK;
 }
 
@@ -280,7 +278,7 @@ int qimm_kv_create(qimm_ctx *ctx, int64_t layers, int64_t batch, int64_t heads, 
     if (bytes) {
         hipError_t e = hipSetDevice(ctx->device);
         if (e == hipSuccess) e = hipMalloc((void **)&kv->k, bytes);
-        if (e == hipSuccess) e = hipMalloc((void **)&kv->vt, bytes);
+        if (e == hipSuccess) e = hipMalloc((void **)&kv->vt, (size_t)(layers * kv->vt_elems()) * 2);
         if (e == hipSuccess) e = kv_alloc_norms(kv);
         if (e != hipSuccess) {
             kv_free(kv);
@@ -300,12 +298,13 @@ int qimm_kv_create_host(qimm_ctx *ctx, int64_t layers, int64_t batch, int64_t he
     if (rc) return rc;
     kv->host = true;
     const size_t lbytes = (size_t)kv->layer_elems() * 2, bytes = lbytes * (size_t)layers;
+    const size_t lvbytes = (size_t)kv->vt_elems() * 2, vbytes = lvbytes * (size_t)layers;
     hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess && bytes) e = hipHostMalloc((void **)&kv->k, bytes, hipHostMallocDefault);
-    if (e == hipSuccess && bytes) e = hipHostMalloc((void **)&kv->vt, bytes, hipHostMallocDefault);
+    if (e == hipSuccess && bytes) e = hipHostMalloc((void **)&kv->vt, vbytes, hipHostMallocDefault);
     for (auto &sl : kv->slot) {
         if (e == hipSuccess && lbytes) e = hipMalloc((void **)&sl.k, lbytes);
-        if (e == hipSuccess && lbytes) e = hipMalloc((void **)&sl.vt, lbytes);
+        if (e == hipSuccess && lbytes) e = hipMalloc((void **)&sl.vt, lvbytes);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&sl.ready, hipEventDisableTiming);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&sl.released, hipEventDisableTiming);
     }
@@ -335,7 +334,7 @@ int qimm_kv_store_layer(qimm_kv *kv, int64_t layer, const uint16_t *k_bhpd, cons
     if (!kv || !k_bhpd || !v_bhpd) return QIMM_ERR_ARG;
     qimm_ctx *ctx = kv->ctx;
     if (layer < 0 || layer >= kv->layers) return set_err(ctx, QIMM_ERR_SHAPE, "kv store: layer out of range");
-    const int64_t n = kv->layer_elems();
+    const int64_t n = kv->layer_elems(), nv = kv->vt_elems();
     if (!n) return QIMM_OK;
     hipStream_t s = (hipStream_t)stream;
     // the layer's largest key norm: the attention's score bound
@@ -343,7 +342,8 @@ int qimm_kv_store_layer(qimm_kv *kv, int64_t layer, const uint16_t *k_bhpd, cons
                                             kv->knorm + layer, s));
     if (!kv->host) {
         QIMM_HIP(ctx, hipMemcpyAsync(kv->k + layer * n, k_bhpd, (size_t)n * 2, hipMemcpyDeviceToDevice, s));
-        QIMM_HIP(ctx, qimm::launch_transpose_sd(v_bhpd, kv->batch * kv->heads, kv->prefix, kv->vt + layer * n, 0, s));
+        QIMM_HIP(ctx, qimm::launch_transpose_sd(v_bhpd, kv->batch * kv->heads, kv->prefix, qimm::vt_ld(kv->prefix),
+                                                kv->vt + layer * nv, 0, s));
         return QIMM_OK;
     }
     // transpose V into a slot, then both halves down to host memory; the slot
@@ -357,9 +357,9 @@ int qimm_kv_store_layer(qimm_kv *kv, int64_t layer, const uint16_t *k_bhpd, cons
     qimm_kv::Slot *sl = kv_claim(kv, layer, s, rc);
     if (!sl) return rc;
     QIMM_HIP(ctx, hipMemcpyAsync(sl->k, k_bhpd, (size_t)n * 2, hipMemcpyDeviceToDevice, s));
-    QIMM_HIP(ctx, qimm::launch_transpose_sd(v_bhpd, kv->batch * kv->heads, kv->prefix, sl->vt, 0, s));
+    QIMM_HIP(ctx, qimm::launch_transpose_sd(v_bhpd, kv->batch * kv->heads, kv->prefix, qimm::vt_ld(kv->prefix), sl->vt, 0, s));
     QIMM_HIP(ctx, hipMemcpyAsync(kv->k + layer * n, sl->k, (size_t)n * 2, hipMemcpyDeviceToHost, s));
-    QIMM_HIP(ctx, hipMemcpyAsync(kv->vt + layer * n, sl->vt, (size_t)n * 2, hipMemcpyDeviceToHost, s));
+    QIMM_HIP(ctx, hipMemcpyAsync(kv->vt + layer * nv, sl->vt, (size_t)nv * 2, hipMemcpyDeviceToHost, s));
     QIMM_HIP(ctx, hipEventRecord(sl->ready, s));
     QIMM_HIP(ctx, hipEventRecord(kv->written, s));
     return QIMM_OK;
@@ -372,11 +372,11 @@ int qimm_kv_load_layer(const qimm_kv *kv, int64_t layer, uint16_t *k_bhpd, uint1
     const int64_t n = kv->layer_elems();
     if (!n) return QIMM_OK;
     hipStream_t s = (hipStream_t)stream;
-    const uint16_t *k, *vt;
-    int rc = kv_layer(kv, layer, s, &k, &vt);
+    qimm::KeySeg seg;
+    int rc = kv_layer(kv, layer, s, &seg);
     if (rc) return rc;
-    QIMM_HIP(ctx, hipMemcpyAsync(k_bhpd, k, (size_t)n * 2, hipMemcpyDeviceToDevice, s));
-    QIMM_HIP(ctx, qimm::launch_transpose_sd(vt, kv->batch * kv->heads, kv->prefix, v_bhpd, 1, s));
+    QIMM_HIP(ctx, hipMemcpyAsync(k_bhpd, seg.k, (size_t)n * 2, hipMemcpyDeviceToDevice, s));
+    QIMM_HIP(ctx, qimm::launch_transpose_sd(seg.vt, kv->batch * kv->heads, kv->prefix, seg.ld, v_bhpd, 1, s));
     return kv_release(kv, layer, s);
 }
 

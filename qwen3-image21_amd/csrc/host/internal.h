@@ -34,8 +34,8 @@ struct qimm_weight {
 struct qimm_kv {
     qimm_ctx *ctx = nullptr;
     int64_t layers = 0, batch = 0, heads = 0, prefix = 0, head_dim = 0;
-    // device cache: k [L][B][H][P][128], vt [L][B][H][128][P]; host cache: the
-    // same layout in pinned host memory, staged one layer at a time into slots
+    // device cache: k [L][B][H][P][128], vt [L][B][H][128][vt_ld(P)] (rows on
+    // 16 B); host cache: the same layout in pinned host memory, staged one layer at a time into slots
     uint16_t *k = nullptr;
     uint16_t *vt = nullptr;
     bool host = false;
@@ -57,6 +57,7 @@ struct qimm_kv {
     mutable int next = 0;
     hipEvent_t written = nullptr;
     int64_t layer_elems() const { return batch * heads * prefix * head_dim; }
+    int64_t vt_elems() const { return batch * heads * qimm::vt_ld(prefix) * head_dim; }
 };
 
 struct qimm_block {
@@ -91,10 +92,10 @@ int upload_weight_rows(qimm_ctx *ctx, int type, int64_t rows, int64_t cols, cons
 int64_t row_bytes(int type, int64_t cols);
 int block_values(int type);
 
-// Device pointers of cache layer `layer` for kernels launched on stream s. A
+// The key segment of cache layer `layer` for kernels launched on stream s. A
 // host cache stages the layer into a slot first (or waits for a prefetch);
 // kv_release must follow the last kernel that reads the pointers.
-int kv_layer(const qimm_kv *kv, int64_t layer, hipStream_t s, const uint16_t **k, const uint16_t **vt);
+int kv_layer(const qimm_kv *kv, int64_t layer, hipStream_t s, qimm::KeySeg *seg);
 int kv_release(const qimm_kv *kv, int64_t layer, hipStream_t s);
 
 }  // namespace qimm_host

@@ -11,26 +11,25 @@
 // max / row sum need only the lane and its partner lane^32. The probabilities
 // stay in registers and are the B operand of O^T += V^T P^T.
 //
-// Two kernels:
-//  - attn_fast_kernel (both segment lengths multiples of 8): 8 waves x 32
-//    queries per workgroup; 64-key K and V^T tiles copied HBM -> LDS with
-//    global_load_lds (no staging registers) into XOR-swizzled, conflict-free
-//    layouts, double-buffered; the K rows of a 32-key half are read in a
-//    bit-swapped order so that each lane's P^T registers hold 8 consecutive
-//    keys and every V^T fragment is one 16 B LDS read; the running maximum is
-//    folded into the S accumulator start (C = -m) and only moves when it grew
-//    by more than 2^8, so the common path is p = exp2(s) (q pre-scaled by
-//    scale*log2 e) and the rescale of O is a rare wave-uniform branch; row
-//    sums use v_dot2_f32_bf16 over the packed bf16 probabilities, the same
-//    values the PV product uses.
-//    With MASKED it also applies the key mask of build_block_causal_mask
-//    (image ids) and key validity, per 64-key window and wave: a window whose
-//    keys all lie before the wave's first query, or all share the queries'
-//    image block, runs unmasked; one with no visible key is skipped; the
-//    others test each score. A workgroup stops at the last key any of its
-//    queries may see (key_limit_kernel).
-//  - attn_any_kernel (any lengths): 4 waves x 32 queries, K/V^T staged through
-//    registers with per-element bounds, the reference shape for ragged tails.
+// attn_fast_kernel: 8 (or 4) waves x 32 queries per workgroup; 64-key K and V^T
+// tiles copied HBM -> LDS with global_load_lds (no staging registers) into
+// XOR-swizzled, conflict-free layouts, double-buffered; the K rows of a 32-key
+// half are read in a bit-swapped order so that each lane's P^T registers hold 8
+// consecutive keys and every V^T fragment is one 16 B LDS read; the running
+// maximum is folded into the S accumulator start (C = -m) and only moves when it
+// grew by more than 2^8, so the common path is p = exp2(s) (q pre-scaled by
+// scale*log2 e) and the rescale of O is a rare wave-uniform branch; row sums use
+// v_dot2_f32_bf16 over the packed bf16 probabilities, the same values the PV
+// product uses.
+// With MASKED it also applies the key mask of build_block_causal_mask (image
+// ids) and key validity, per 64-key window and wave: a window whose keys all lie
+// before the wave's first query, or all share the queries' image block, runs
+// unmasked; one with no visible key is skipped; the others test each score. A
+// workgroup stops at the last key any of its queries may see (key_limit_kernel).
+// Any segment length: the last window of a segment clamps its K rows and V^T
+// chunks to the segment and clears the V^T columns past its end. V^T rows of 16 B
+// aligned stride (KeySeg::ld) are copied straight into LDS; rows of any other
+// stride go through registers (RV).
 #include <type_traits>
 
 #include "device_common.h"
@@ -39,11 +38,7 @@
 namespace qimm {
 namespace {
 
-struct Seg {
-    const uint16_t *k;   // [BH][len][128]
-    const uint16_t *vt;  // [BH][128][len]
-    int64_t len;
-};
+using Seg = KeySeg;
 
 // Key mask of build_block_causal_mask (src/attention_mask.rs:18-66): query i
 // sees key j when key_valid[b][j] and (i >= j or i and j lie in the same
@@ -265,7 +260,10 @@ constexpr float RESCALE_TH = 8.0f;    // log2 units
 // bound (the prefix keys' norm is a device value); 1 = fixed reference, 2 =
 // running maximum, both decided on the host. A kernel with one form has only
 // that loop's registers to allocate.
-template <int NW, bool PRE, bool MASKED, int SMODE, bool PAIR>
+// RV: V^T rows whose stride is not a multiple of 16 B (a caller's dense V^T of
+// an odd length) cannot be copied 16 B at a time into LDS: their chunks are
+// loaded unaligned into registers one block ahead and written to the same slots.
+template <int NW, bool PRE, bool MASKED, int SMODE, bool PAIR, bool RV>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16_t *__restrict__ q, Seg s0, Seg s1,
                                                                     int64_t H, int64_t Sq, int64_t nq, int64_t B,
                                                                     float sl2, uint16_t *__restrict__ out,
@@ -332,7 +330,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             }
         }
 
-        const int len0 = (int)s0.len, len1 = (int)s1.len;
+        const int len0 = (int)s0.len, len1 = (int)s1.len, ld0 = (int)s0.ld, ld1 = (int)s1.ld;
         const int nb0 = (len0 + KB - 1) / KB, nb1 = (len1 + KB - 1) / KB;
         int nblk = nb0 + nb1;
 
@@ -362,8 +360,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
         }
         const char *kb0 = (const char *)(s0.k + bh * (int64_t)len0 * HD);
         const char *kb1 = (const char *)(s1.k + bh * (int64_t)len1 * HD);
-        const char *vb0 = (const char *)(s0.vt + bh * (int64_t)HD * len0);
-        const char *vb1 = (const char *)(s1.vt + bh * (int64_t)HD * len1);
+        const char *vb0 = (const char *)(s0.vt + bh * (int64_t)HD * ld0);
+        const char *vb1 = (const char *)(s1.vt + bh * (int64_t)HD * ld1);
 
         // DMA roles: instruction t = wave + NW i fills K rows 4t .. 4t+3 (lane at
         // row 4t + lane/16, slot lane%16) and V^T rows 8t .. 8t+7 (lane at row
@@ -377,59 +375,99 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             vrow[i] = (uint32_t)d;
             vcol[i] = (uint32_t)(((lane & 7) ^ ((d >> 1) & 7)) << 4);
         }
-        // Block j covers keys [start, start + 64) of its segment. The last block of
-        // a segment of at least 64 keys slides back to end at len (window [kv0,
-        // kv0 + 64), keys before `lo` already seen); a shorter segment clamps its
-        // rows and masks keys from `hi` on. Every load stays inside the segment.
+        // Block j covers keys [kv0, kv0 + 64) of its segment, of which the first hi
+        // exist. A short last block clamps its K rows and V^T chunks to the
+        // segment (scores from hi on are masked); every load stays inside it.
         struct Blk {
             const char *kb, *vb;
-            int len, kv0, lo, hi, kbase;  // kbase: index of the segment's first key in [s0 ; s1]
+            int len, ld, kv0, hi, kbase;  // kbase: index of the segment's first key in [s0 ; s1]
         };
         auto blk_of = [&](int j) __attribute__((always_inline)) {
             Blk b;
             const bool first = j < nb0;
             b.kbase = first ? 0 : len0;
             b.len = first ? len0 : len1;
+            b.ld = first ? ld0 : ld1;
             b.kb = first ? kb0 : kb1;
             b.vb = first ? vb0 : vb1;
-            const int start = (first ? j : j - nb0) * KB;
-            if (b.len >= KB) {
-                b.kv0 = min(start, b.len - KB);
-                b.lo = start - b.kv0;
-                b.hi = KB;
-            } else {
-                b.kv0 = 0;
-                b.lo = 0;
-                b.hi = b.len;
-            }
+            b.kv0 = (first ? j : j - nb0) * KB;
+            b.hi = min(KB, b.len - b.kv0);
             return b;
+        };
+        u32x4 vreg[DI];  // RV: the next block's V^T chunks of this lane
+        auto load_v = [&](const Blk &b) __attribute__((always_inline)) {
+            const char *vg = b.vb + (int64_t)b.kv0 * 2;
+#pragma unroll
+            for (int i = 0; i < DI; i++) {
+                const char *row = vg + vrow[i] * (uint32_t)(2 * b.ld);
+                if (b.hi == KB) {
+                    __builtin_memcpy(&vreg[i], row + vcol[i], 16);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int c = (int)(vcol[i] >> 1) + 2 * e;
+                        const uint32_t lo = c < b.hi ? ((const uint16_t *)row)[c] : 0u;
+                        const uint32_t hi = c + 1 < b.hi ? ((const uint16_t *)row)[c + 1] : 0u;
+                        vreg[i][e] = lo | (hi << 16);
+                    }
+                }
+            }
         };
         auto dma = [&](const Blk &b, int stage) __attribute__((always_inline)) {
             uint8_t *base = lds + stage * STAGE;
-            if (b.len >= KB) {
-                const char *kg = b.kb + (int64_t)b.kv0 * 256;
-                const char *vg = b.vb + (int64_t)b.kv0 * 2;
+            const char *kg = b.kb + (int64_t)b.kv0 * 256;
+            const char *vg = b.vb + (int64_t)b.kv0 * 2;
+            if (b.hi == KB) {
 #pragma unroll
                 for (int i = 0; i < DI; i++)
                     __builtin_amdgcn_global_load_lds((const void *)(kg + koff[i]),
                                                      (lds_ptr_t)(base + (wave + NW * i) * 1024), 16, 0, 0);
+                if constexpr (!RV) {
 #pragma unroll
-                for (int i = 0; i < DI; i++)
-                    __builtin_amdgcn_global_load_lds((const void *)(vg + (vrow[i] * (uint32_t)(2 * b.len) + vcol[i])),
-                                                     (lds_ptr_t)(base + TILE + (wave + NW * i) * 1024), 16, 0, 0);
+                    for (int i = 0; i < DI; i++)
+                        __builtin_amdgcn_global_load_lds((const void *)(vg + (vrow[i] * (uint32_t)(2 * b.ld) + vcol[i])),
+                                                         (lds_ptr_t)(base + TILE + (wave + NW * i) * 1024), 16, 0, 0);
+                }
             } else {
 #pragma unroll
                 for (int i = 0; i < DI; i++) {
                     const int r = 4 * (wave + NW * i) + (lane >> 4);
-                    const int gr = min(r, b.len - 1);
-                    __builtin_amdgcn_global_load_lds((const void *)(b.kb + (koff[i] - r * 256) + gr * 256),
+                    const int gr = min(r, b.hi - 1);
+                    __builtin_amdgcn_global_load_lds((const void *)(kg + (koff[i] - r * 256) + gr * 256),
                                                      (lds_ptr_t)(base + (wave + NW * i) * 1024), 16, 0, 0);
                 }
+                if constexpr (!RV) {
 #pragma unroll
+                    for (int i = 0; i < DI; i++) {
+                        const int gc = min((int)vcol[i] >> 1, ((b.hi + 7) & ~7) - 8);
+                        __builtin_amdgcn_global_load_lds((const void *)(vg + vrow[i] * (uint32_t)(2 * b.ld) + 2 * gc),
+                                                         (lds_ptr_t)(base + TILE + (wave + NW * i) * 1024), 16, 0, 0);
+                    }
+                }
+            }
+            if constexpr (RV && !MASKED) load_v(b);
+        };
+        // After this wave's copies of block b have landed, before the barrier that
+        // publishes them: the lane's own V^T chunks of a block whose end lies
+        // inside a chunk are cleared from the end on (a masked key's probability is
+        // 0, and the row padding may hold anything: 0 x NaN must not arise).
+        // RV writes its chunks here; the masked form has no registers to hold them
+        // over a step (132 spilled) and loads them here too.
+        auto seal = [&](const Blk &b, int stage) __attribute__((always_inline)) {
+            uint8_t *base = lds + stage * STAGE + TILE;
+            if constexpr (RV) {
+                if constexpr (MASKED) load_v(b);
+#pragma unroll
+                for (int i = 0; i < DI; i++) *(u32x4 *)(base + (wave + NW * i) * 1024 + 16 * lane) = vreg[i];
+            } else if (b.hi & 7) {
+#pragma unroll 1
                 for (int i = 0; i < DI; i++) {
-                    const int gc = min((int)vcol[i] >> 1, b.len - 8);
-                    __builtin_amdgcn_global_load_lds((const void *)(b.vb + vrow[i] * (uint32_t)(2 * b.len) + 2 * gc),
-                                                     (lds_ptr_t)(base + TILE + (wave + NW * i) * 1024), 16, 0, 0);
+                    u32x4 *p = (u32x4 *)(base + (wave + NW * i) * 1024 + 16 * lane);
+                    const int left = b.hi - (((lane & 7) ^ (((8 * (wave + NW * i) + (lane >> 3)) >> 1) & 7)) << 3);
+                    u32x4 v = *p;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] &= left > 2 * e + 1 ? 0xffffffffu : left > 2 * e ? 0xffffu : 0u;
+                    *p = v;
                 }
             }
         };
@@ -465,7 +503,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
         // kmask: visible keys of the window (bit kv), kid: lane kv holds the image
         // id of window key kv, kb0: index of the window's first key, partial: test
         // each score (MASKED only)
-        auto half_step = [&](const uint8_t *stg, int h, int lo, int hi, uint64_t kmask, int kid, int kb0,
+        auto half_step = [&](const uint8_t *stg, int h, int hi, uint64_t kmask, int kid, int kb0,
                              bool partial, auto stat) __attribute__((always_inline)) {
             constexpr bool STATIC = decltype(stat)::value;
             f32x16 st;
@@ -480,11 +518,11 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
                 const bf16x8 a = *(const bf16x8 *)(stg + h * 32 * 256 + kaddr[kk]);
                 st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[kk], st, 0, 0, 0);
             }
-            if (lo > h * 32 || hi < h * 32 + 32) {
+            if (hi < h * 32 + 32) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int kv = h * 32 + 16 * (r >> 3) + 8 * g + (r & 7);
-                    if (kv < lo || kv >= hi) st[r] = -INFINITY;
+                    if (kv >= hi) st[r] = -INFINITY;
                 }
             }
             if constexpr (MASKED) {
@@ -594,12 +632,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             }
             return st;
         };
-        auto pv_static = [&](const uint8_t *stg, int h, f32x16 st, int lo, int hi) __attribute__((always_inline)) {
-            if (lo > h * 32 || hi < h * 32 + 32) {
+        auto pv_static = [&](const uint8_t *stg, int h, f32x16 st, int hi) __attribute__((always_inline)) {
+            if (hi < h * 32 + 32) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int kv = h * 32 + 16 * (r >> 3) + 8 * g + (r & 7);
-                    if (kv < lo || kv >= hi) st[r] = -INFINITY;
+                    if (kv >= hi) st[r] = -INFINITY;
                 }
             }
             uint32_t pk[8];
@@ -626,7 +664,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
         constexpr int KEY_OFF = -0x7fffffff - 1;
         int mk = 0;
         auto mask_load = [&](const Blk &b) __attribute__((always_inline)) {
-            const int kv = min(lane, b.len - 1 - b.kv0);
+            const int kv = min(lane, b.hi - 1);
             const int64_t key = (int64_t)b.kbase + b.kv0 + kv;
             const bool valid = km.kvalid ? km.kvalid[bb * km.kv_len + key] != 0 : true;
             const int id = km.img ? km.img[key] : 0;
@@ -643,10 +681,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
                 // classify the window for this wave's queries (wave-uniform)
                 kid = mk;
                 kb0 = b.kbase + b.kv0;
-                const bool in = lane >= b.lo && lane < b.hi;
+                const bool in = lane < b.hi;
                 const uint64_t inm = __builtin_amdgcn_ballot_w64(in);
                 kmask = __builtin_amdgcn_ballot_w64(in && mk != KEY_OFF);
-                const int k_lo = kb0 + b.lo, k_hi = kb0 + b.hi - 1;
+                const int k_lo = kb0, k_hi = kb0 + b.hi - 1;
                 bool full = kmask == inm, empty = kmask == 0;
                 if (km.img) {
                     const uint64_t same = __builtin_amdgcn_ballot_w64(in && mk == qid_min);
@@ -662,13 +700,14 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             const uint8_t *stg = lds + cur * STAGE;
             if constexpr (decltype(stat)::value && !MASKED) {
                 const f32x16 s0 = qk_static(stg, 0), s1 = qk_static(stg, 1);
-                pv_static(stg, 0, s0, b.lo, b.hi);
-                pv_static(stg, 1, s1, b.lo, b.hi);
+                pv_static(stg, 0, s0, b.hi);
+                pv_static(stg, 1, s1, b.hi);
             } else if (!skip) {
-                half_step(stg, 0, b.lo, b.hi, kmask, kid, kb0, partial, stat);
-                half_step(stg, 1, b.lo, b.hi, kmask, kid, kb0, partial, stat);
+                half_step(stg, 0, b.hi, kmask, kid, kb0, partial, stat);
+                half_step(stg, 1, b.hi, kmask, kid, kb0, partial, stat);
             }
             __builtin_amdgcn_s_waitcnt(WAIT_VM0);  // vmcnt(0): block j+1 landed
+            if (j + 1 < nblk) seal(blk_of(j + 1), cur ^ 1);
             __syncthreads();
         };
 
@@ -677,6 +716,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             dma(blk_of(0), 0);
         }
         __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+        if (nblk > 0) seal(blk_of(0), 0);
         __syncthreads();
         // the fixed-reference form when the score bound allows it (wave-uniform)
         bool stat_ok = false;
@@ -779,232 +819,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
 
 }  // namespace fast
 
-namespace anylen {
-
-constexpr int QB = 128;     // queries per workgroup
-constexpr int KB = 64;      // keys per block
-constexpr int HD = 128;     // head dim
-constexpr int KP = 136;     // bf16 pitch of K tile rows (128 + 8)
-constexpr int VP = 68;      // bf16 pitch of V^T tile rows (64 + 4): conflict-free 8 B reads
-constexpr int KSTAGE = KB * KP;
-constexpr int VSTAGE = HD * VP;
-constexpr int STAGE = KSTAGE + VSTAGE;
-constexpr int OP = 136;     // bf16 pitch of the output staging rows
-
-// K and V^T tiles of 64 keys double-buffered in LDS through registers; the
-// 16-key K-slots of the PV MFMA use the key order of the S^T accumulator
-// layout, and V^T is read from LDS in the same order.
-template <bool MASKED>
-__global__ __launch_bounds__(256, 2) void attn_any_kernel(const uint16_t *__restrict__ q, Seg s0, Seg s1,
-                                                      int64_t H, int64_t Sq, int64_t nq, int64_t B,
-                                                      float sl2, uint16_t *__restrict__ out,
-                                                      float *__restrict__ outf, KeyMask km, int q8) {
-    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * STAGE];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, l32 = lane & 31;
-
-    // XCD-aware order: the hardware deals workgroups round-robin over 8 XCDs;
-    // give each XCD a contiguous range of (batch, head, query-tile) so the
-    // query tiles of one head share that XCD's L2 copy of its K/V.
-    const int64_t total = nq * H * B;
-    int64_t L = blockIdx.x;
-    if ((total & 7) == 0) L = (L & 7) * (total >> 3) + (L >> 3);
-    const int64_t qt = L % nq, hh = (L / nq) % H, bb = L / (nq * H);
-    const int64_t bh = bb * H + hh;
-    const int64_t q0 = qt * QB + wave * 32;
-
-    // Q^T fragments (B operand): lane holds query q0+l32, d = 16kk + 8g .. +8.
-    bf16x8 qf[8];
-    {
-        const int64_t qi = q0 + l32;
-        const uint16_t *qr = q + (bh * Sq + (qi < Sq ? qi : 0)) * HD;
-#pragma unroll
-        for (int kk = 0; kk < 8; kk++) {
-            u32x4 v = *(const u32x4 *)(qr + kk * 16 + g * 8);
-            if (qi >= Sq) v = u32x4{0u, 0u, 0u, 0u};
-            qf[kk] = __builtin_bit_cast(bf16x8, v);
-        }
-    }
-
-    const int64_t nb0 = (s0.len + KB - 1) / KB, nb1 = (s1.len + KB - 1) / KB;
-    const int64_t nblk = nb0 + nb1;
-
-    // loader roles
-    const int k_row = tid >> 4, k_col = (tid & 15) * 8;  // 4 x (16 rows apart)
-    const int v_row = tid >> 3, v_col = (tid & 7) * 8;   // 4 x (32 rows apart)
-    u32x4 rk[4], rv[4];
-
-    auto load_blk = [&](int64_t j) {
-        const Seg &sg = j < nb0 ? s0 : s1;
-        const int64_t kv0 = (j < nb0 ? j : j - nb0) * KB;
-        const int64_t len = sg.len;
-        const uint16_t *kb = sg.k + bh * len * HD;
-        const uint16_t *vb = sg.vt + bh * HD * len;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int64_t r = kv0 + k_row + 16 * i;
-            rk[i] = r < len ? *(const u32x4 *)(kb + r * HD + k_col) : u32x4{0u, 0u, 0u, 0u};
-        }
-        const bool vec = (len & 7) == 0;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint16_t *vr = vb + (int64_t)(v_row + 32 * i) * len;
-            const int64_t c = kv0 + v_col;
-            if (vec) {
-                rv[i] = c < len ? *(const u32x4 *)(vr + c) : u32x4{0u, 0u, 0u, 0u};
-            } else {
-                uint32_t w[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    uint32_t lo = c + 2 * e < len ? vr[c + 2 * e] : 0u;
-                    uint32_t hi = c + 2 * e + 1 < len ? vr[c + 2 * e + 1] : 0u;
-                    w[e] = lo | (hi << 16);
-                }
-                rv[i] = u32x4{w[0], w[1], w[2], w[3]};
-            }
-        }
-    };
-    auto store_blk = [&](uint16_t *st) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) *(u32x4 *)(st + (k_row + 16 * i) * KP + k_col) = rk[i];
-        uint16_t *vs = st + KSTAGE;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            uint16_t *p = vs + (v_row + 32 * i) * VP + v_col;
-            *(u32x2 *)p = u32x2{rv[i][0], rv[i][1]};
-            *(u32x2 *)(p + 4) = u32x2{rv[i][2], rv[i][3]};
-        }
-    };
-
-    f32x16 o[4];
-#pragma unroll
-    for (int dt = 0; dt < 4; dt++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f;
-
-    if (nblk > 0) {
-        load_blk(0);
-        store_blk(lds);
-    }
-    __syncthreads();
-
-    for (int64_t j = 0; j < nblk; j++) {
-        const int cur = (int)(j & 1);
-        const bool more = j + 1 < nblk;
-        if (more) load_blk(j + 1);
-        const uint16_t *ks = lds + cur * STAGE;
-        const uint16_t *vs = ks + KSTAGE;
-
-        const Seg &sg = j < nb0 ? s0 : s1;
-        const int64_t valid = sg.len - (j < nb0 ? j : j - nb0) * KB;  // keys of this block in range
-        // The 64-key block is processed as two 32-key halves so only one
-        // 32x32 S^T tile is live at a time.
-#pragma unroll
-        for (int half = 0; half < 2; half++) {
-            // S^T (32 keys x 32 queries) = K_half Q^T
-            f32x16 st;
-#pragma unroll
-            for (int r = 0; r < 16; r++) st[r] = 0.f;
-#pragma unroll
-            for (int kk = 0; kk < 8; kk++) {
-                bf16x8 a = *(const bf16x8 *)(ks + (half * 32 + l32) * KP + kk * 16 + g * 8);
-                st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[kk], st, 0, 0, 0);
-            }
-            // the prefetched tile goes to the other stage once its loads land,
-            // ending the live range of the staging registers early
-            if (half == 0 && more) store_blk(lds + (cur ^ 1) * STAGE);
-            if (valid < (half + 1) * 32) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int kv = half * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-                    if (kv >= valid) st[r] = -INFINITY;
-                }
-            }
-            if constexpr (MASKED) {
-                // key index in the concatenated [prefix ; own] sequence
-                const int64_t kb = (j < nb0 ? j * KB : s0.len + (j - nb0) * KB) + half * 32;
-                const int64_t qi = min(q0 + l32, Sq - 1);
-                const int32_t qimg = km.img ? km.img[qi] : -1;
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int64_t kidx = kb + 8 * (r >> 2) + 4 * g + (r & 3);
-                    if (kidx >= km.kv_len) continue;  // beyond the keys: masked above
-                    bool ok = km.kvalid ? km.kvalid[bb * km.kv_len + kidx] != 0 : true;
-                    if (km.img) ok = ok && (qi >= kidx || (qimg >= 0 && km.img[kidx] == qimg));
-                    if (!ok) st[r] = -INFINITY;
-                }
-            }
-            // online softmax in the log2 domain
-            float mx = st[0];
-#pragma unroll
-            for (int r = 1; r < 16; r++) mx = fmaxf(mx, st[r]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
-            const float m_new = fmaxf(m_run, mx * sl2);
-            const float m_use = m_new == -INFINITY ? 0.f : m_new;
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
-            float psum = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(st[r], sl2, -m_use));
-                st[r] = p;
-                psum += p;
-            }
-            l_run = l_run * alpha + psum;
-            m_run = m_new;
-#pragma unroll
-            for (int dt = 0; dt < 4; dt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
-            // P^T fragments: keys 32half + 16kk + {4g..4g+3, 8+4g..8+4g+3} are
-            // accumulator registers st[8kk .. 8kk+8) of this lane.
-#pragma unroll
-            for (int kk = 0; kk < 2; kk++) {
-                u32x4 w{pack_bf16x2(st[8 * kk + 0], st[8 * kk + 1]), pack_bf16x2(st[8 * kk + 2], st[8 * kk + 3]),
-                        pack_bf16x2(st[8 * kk + 4], st[8 * kk + 5]), pack_bf16x2(st[8 * kk + 6], st[8 * kk + 7])};
-                const bf16x8 pf = __builtin_bit_cast(bf16x8, w);
-                // O^T (128 d x 32 q) += V^T[:, keys] P^T[keys, :]
-#pragma unroll
-                for (int dt = 0; dt < 4; dt++) {
-                    const uint16_t *vr = vs + (dt * 32 + l32) * VP + half * 32 + kk * 16 + 4 * g;
-                    u32x2 lo = *(const u32x2 *)vr;
-                    u32x2 hi = *(const u32x2 *)(vr + 8);
-                    bf16x8 a = __builtin_bit_cast(bf16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
-                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pf, o[dt], 0, 0, 0);
-                }
-            }
-        }
-        __syncthreads();
-    }
-
-    // normalize and stage O [32 q x 128 d] per wave through LDS for row stores
-    const float l_tot = l_run + __shfl_xor(l_run, 32);
-    const float inv = 1.0f / l_tot;
-    if (outf) {
-        store_out_f32<68>((float *)lds + wave * 32 * 68, o, inv, lane, outf, bb, Sq, H * HD, hh * HD, q0);
-        return;
-    }
-    uint16_t *os = lds + wave * 32 * OP;
-    stage_out_bf16<OP>(os, o, inv, lane, q8 != 0);
-    __syncthreads();
-    const int64_t HDt = H * HD;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int r = i * 4 + (lane >> 4);
-        const int c = (lane & 15) * 8;
-        const int64_t qi = q0 + r;
-        if (qi < Sq)
-            *(u32x4 *)(out + (bb * Sq + qi) * HDt + hh * HD + c) = *(const u32x4 *)(os + r * OP + c);
-    }
-}
-
-}  // namespace anylen
-
-template <int NW, bool PRE, bool MASKED, int SMODE = 0, bool PAIR = false>
+template <int NW, bool PRE, bool MASKED, int SMODE = 0, bool PAIR = false, bool RV = false>
 void launch_fast(const uint16_t *q, Seg s0, Seg s1, int64_t h, int64_t sq, int64_t b, float sl2, uint16_t *out,
                  float *outf, const KeyMask &km, const int32_t *lim, const ScoreBound &sb, int q8,
                  hipStream_t stream) {
     const int64_t nq = (sq + 32 * NW - 1) / (32 * NW);
-    fast::attn_fast_kernel<NW, PRE, MASKED, SMODE, PAIR>
+    fast::attn_fast_kernel<NW, PRE, MASKED, SMODE, PAIR, RV>
         <<<dim3((unsigned)(nq * (PAIR ? h / 2 : h) * b)), dim3(64 * NW), 0, stream>>>(q, s0, s1, h, sq, nq, b, sl2,
                                                                                        out, outf, km, lim, sb, q8);
 }
@@ -1060,93 +880,89 @@ hipError_t finish_q8k(int out_qblk, bool rounded, const float *outf, int64_t b, 
     return launch_quant_rows(outf, h * 128, b * sq, h * 128, 256, out, h * 128, stream);
 }
 
+// [prefix ; own] with an empty prefix dropped; false: not a valid pair
+bool segments(KeySeg prefix, KeySeg own, Seg &s0, Seg &s1) {
+    if (prefix.len < 0 || own.len < 0 || prefix.len + own.len <= 0) return false;
+    if ((prefix.len > 0 && prefix.ld < prefix.len) || (own.len > 0 && own.ld < own.len)) return false;
+    s0 = prefix.len > 0 ? prefix : own;
+    s1 = prefix.len > 0 ? own : KeySeg{own.k, own.vt, 0, own.ld};
+    return true;
+}
+// V^T rows that start on 16 B (their base does): copied straight into LDS. The
+// cache's and the block's own V^T always have such rows; a caller's dense V^T
+// has them when its length is a multiple of 8.
+bool rows16(const Seg &s) { return s.len == 0 || s.ld % 8 == 0; }
+
 template <bool PRE>
-hipError_t launch(const uint16_t *q, const uint16_t *kp, const uint16_t *vtp, int64_t p, const uint16_t *ko,
-                  const uint16_t *vto, int64_t so, int64_t b, int64_t h, int64_t sq, float sl2, uint16_t *out,
-                  float *outf, const ScoreBound &sb, int out_qblk, hipStream_t stream) {
+hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq, float sl2,
+                  uint16_t *out, float *outf, const ScoreBound &sb, int out_qblk, hipStream_t stream) {
     if (sq <= 0 || b <= 0 || h <= 0) return hipSuccess;
-    if (p < 0 || so < 0 || p + so <= 0 || !out_qblk_ok(out_qblk, outf)) return hipErrorInvalidValue;
-    Seg s0{kp, vtp, p}, s1{ko, vto, so};
-    if (p <= 0) {
-        s0 = s1;
-        s1 = Seg{ko, vto, 0};
-    }
+    Seg s0, s1;
+    if (!segments(prefix, own, s0, s1) || !out_qblk_ok(out_qblk, outf)) return hipErrorInvalidValue;
     const int q8 = out_qblk == 32;
     float *f32out = out_qblk == 32 ? nullptr : outf;  // f32 output (0 with outf, or 256 not paired)
     bool rounded = false;
-    if ((p & 7) == 0 && (so & 7) == 0) {
-        const KeyMask km{nullptr, nullptr, p + so};
-        const int nw = fast_waves(b * h, sq);
-        if (out_qblk == 256 && nw == 8 && h % 2 == 0) {
-            launch_fast<8, PRE, false, 0, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, nullptr, sb, 0, stream);
-            rounded = true;
-        } else if (nw == 4) {
-            launch_fast<4, PRE, false>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
-        } else {
-            launch_fast<8, PRE, false>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
-        }
+    const KeyMask km{nullptr, nullptr, prefix.len + own.len};
+    const int nw = fast_waves(b * h, sq);
+    if (!rows16(s0) || !rows16(s1)) {
+        if (nw == 4)
+            launch_fast<4, false, false, 2, false, true>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
+        else
+            launch_fast<8, false, false, 2, false, true>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
+    } else if (out_qblk == 256 && nw == 8 && h % 2 == 0) {
+        launch_fast<8, PRE, false, 0, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, nullptr, sb, 0, stream);
+        rounded = true;
+    } else if (nw == 4) {
+        launch_fast<4, PRE, false>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
     } else {
-        const int64_t nq = (sq + anylen::QB - 1) / anylen::QB;
-        anylen::attn_any_kernel<false><<<dim3((unsigned)(nq * h * b)), dim3(256), 0, stream>>>(
-            q, s0, s1, h, sq, nq, b, sl2, out, f32out, KeyMask{nullptr, nullptr, p + so}, q8);
+        launch_fast<8, PRE, false>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
     }
     return finish_q8k(out_qblk, rounded, outf, b, h, sq, out, stream);
 }
 
 }  // namespace
 
-hipError_t launch_attention(const uint16_t *q, const uint16_t *kp, const uint16_t *vtp, int64_t p,
-                            const uint16_t *ko, const uint16_t *vto, int64_t so, int64_t b, int64_t h,
-                            int64_t sq, float scale, uint16_t *out, hipStream_t stream, float *outf) {
-    return launch<false>(q, kp, vtp, p, ko, vto, so, b, h, sq, scale * 1.4426950408889634f, out, outf,
+hipError_t launch_attention(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
+                            float scale, uint16_t *out, hipStream_t stream, float *outf) {
+    return launch<false>(q, prefix, own, b, h, sq, scale * 1.4426950408889634f, out, outf,
                          ScoreBound{nullptr, 0.f, 0.f}, 0, stream);
 }
 
-hipError_t launch_attention_masked(const uint16_t *q, const uint16_t *kp, const uint16_t *vtp, int64_t p,
-                                   const uint16_t *ko, const uint16_t *vto, int64_t so, int64_t b, int64_t h,
-                                   int64_t sq, float sl2, const int32_t *img, const uint8_t *kvalid,
-                                   int32_t *lim_scratch, uint16_t *out, hipStream_t stream, float *outf,
-                                   const float *k_prefix_norm, float q_norm, float k_own_norm, int out_qblk) {
+hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
+                                   float sl2, const int32_t *img, const uint8_t *kvalid, int32_t *lim_scratch,
+                                   uint16_t *out, hipStream_t stream, float *outf, const float *k_prefix_norm,
+                                   float q_norm, float k_own_norm, int out_qblk) {
     if (sq <= 0 || b <= 0 || h <= 0) return hipSuccess;
-    if (p < 0 || so < 0 || p + so <= 0 || !out_qblk_ok(out_qblk, outf)) return hipErrorInvalidValue;
+    Seg s0, s1;
+    if (!segments(prefix, own, s0, s1) || !out_qblk_ok(out_qblk, outf)) return hipErrorInvalidValue;
     const int out_q8 = out_qblk == 32;
     if (out_qblk == 32) outf = nullptr;
-    if (img && (p != 0 || so != sq)) return hipErrorInvalidValue;  // block-causal: one shared sequence
-    Seg s0{kp, vtp, p}, s1{ko, vto, so};
-    if (p <= 0) {
-        s0 = s1;
-        s1 = Seg{ko, vto, 0};
+    if (img && (prefix.len != 0 || own.len != sq)) return hipErrorInvalidValue;  // block-causal: one shared sequence
+    const KeyMask km{img, kvalid, prefix.len + own.len};
+    // the last visible key of each query (none known: every window is classified)
+    const int32_t *lim = nullptr;
+    if (img && lim_scratch && sq <= LIMIT_MAX_S) {
+        key_limit_kernel<<<dim3(1), dim3(1024), 0, stream>>>(img, (int)sq, lim_scratch);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        lim = lim_scratch;
     }
-    const KeyMask km{img, kvalid, p + so};
-    if ((p & 7) == 0 && (so & 7) == 0 && (!img || (lim_scratch && sq <= LIMIT_MAX_S))) {
-        if (img) {
-            key_limit_kernel<<<dim3(1), dim3(1024), 0, stream>>>(img, (int)sq, lim_scratch);
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-        }
-        // the bound is on scores in log2 units: q's norm times sl2
-        const ScoreBound sb{p > 0 ? k_prefix_norm : nullptr, q_norm * sl2, k_own_norm};
-        // sl2 == 1: q already carries the scale (the block's q/k/v epilogue)
-        if (sl2 == 1.0f)
-            launch_masked<true>(q, s0, s1, h, sq, b, sl2, out, outf, km, img ? lim_scratch : nullptr, sb, out_q8,
-                                stream);
-        else
-            launch_masked<false>(q, s0, s1, h, sq, b, sl2, out, outf, km, img ? lim_scratch : nullptr, sb, out_q8,
-                                 stream);
-        return finish_q8k(out_qblk, false, outf, b, h, sq, out, stream);
-    }
-    const int64_t nq = (sq + anylen::QB - 1) / anylen::QB;
-    anylen::attn_any_kernel<true><<<dim3((unsigned)(nq * h * b)), dim3(256), 0, stream>>>(
-        q, s0, s1, h, sq, nq, b, sl2, out, outf, km, out_q8);
+    // the bound is on scores in log2 units: q's norm times sl2
+    const ScoreBound sb{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm * sl2, k_own_norm};
+    if (!rows16(s0) || !rows16(s1))
+        launch_fast<8, false, true, 2, false, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream);
+    else if (sl2 == 1.0f)  // q already carries the scale (the block's q/k/v epilogue)
+        launch_masked<true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream);
+    else
+        launch_masked<false>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream);
     return finish_q8k(out_qblk, false, outf, b, h, sq, out, stream);
 }
 
-hipError_t launch_attention_log2(const uint16_t *q, const uint16_t *kp, const uint16_t *vtp, int64_t p,
-                                 const uint16_t *ko, const uint16_t *vto, int64_t so, int64_t b, int64_t h,
-                                 int64_t sq, uint16_t *out, hipStream_t stream, float *outf,
-                                 const float *k_prefix_norm, float q_norm, float k_own_norm, int out_qblk) {
-    return launch<true>(q, kp, vtp, p, ko, vto, so, b, h, sq, 1.0f, out, outf,
-                        ScoreBound{p > 0 ? k_prefix_norm : nullptr, q_norm, k_own_norm}, out_qblk, stream);
+hipError_t launch_attention_log2(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
+                                 uint16_t *out, hipStream_t stream, float *outf, const float *k_prefix_norm,
+                                 float q_norm, float k_own_norm, int out_qblk) {
+    return launch<true>(q, prefix, own, b, h, sq, 1.0f, out, outf,
+                        ScoreBound{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm, k_own_norm}, out_qblk, stream);
 }
 
 }  // namespace qimm

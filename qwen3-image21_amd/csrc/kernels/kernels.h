@@ -30,7 +30,7 @@ struct EpiParams {
     int64_t g_rows_per;
     // EPI_QKV: fused-column n + n_offset in [0, 3*hidden): q | k | v sections.
     // q, k: RmsNorm per 128-wide head, then RoPE with pe[s][128], to [B,H,S,D].
-    // v: transposed to vt [B,H,D,S]; also [B,H,S,D] into v_bhsd when non-null.
+    // v: transposed to vt [B,H,D,vt_ld]; also [B,H,S,D] into v_bhsd when non-null.
     uint16_t *q;
     uint16_t *k;
     uint16_t *vt;
@@ -38,6 +38,7 @@ struct EpiParams {
     const float *norm_q;
     const float *norm_k;
     const float *pe;
+    int64_t vt_ld;  // row elements of vt, a multiple of 8
     int64_t seq;
     int64_t heads;
     int64_t hidden;
@@ -157,37 +158,44 @@ hipError_t launch_quant_rows(const float *x, int64_t ldx, int64_t m, int64_t k, 
 // Q8_0, 256 for Q4_K / Q6_K (Q8_K), 0 for float weights (a plain matmul).
 inline int act_block(int fmt) { return fmt == WF_Q8_0 ? 32 : (fmt == WF_Q4_K || fmt == WF_Q6_K) ? 256 : 0; }
 
-// Joint attention over [prefix ; own] keys. q, k_* : [B,H,S,128] bf16;
-// vt_* : [B,H,128,S] bf16; out [B,Sq,H*128] bf16, or outf [B,Sq,H*128] f32
-// instead when outf is set (out is then not written). out_qblk 32 / 256: out
+// One segment of keys: k [B,H,len,128] bf16, vt [B,H,128,ld] bf16 with ld >= len
+// (row elements from len on may hold anything). vt_ld(len) is the row length of
+// the V^T this library lays out itself: rows then start on 16 B.
+struct KeySeg {
+    const uint16_t *k;
+    const uint16_t *vt;
+    int64_t len;
+    int64_t ld;
+};
+inline int64_t vt_ld(int64_t len) { return (len + 7) & ~(int64_t)7; }
+
+// Joint attention over [prefix ; own] keys. q : [B,H,S,128] bf16; out
+// [B,Sq,H*128] bf16, or outf [B,Sq,H*128] f32 instead when outf is set (out is
+// then not written). out_qblk 32 / 256: out
 // holds candle's activation rounding of the output instead, bf16(d q) per Q8_0
 // (32 values) / Q8_K (256 values) block (quant_act4's arithmetic), the to_out
 // input in the candle mode: Q8_0 in the kernels' epilogue; Q8_K by the paired
 // cached-step kernel where it runs (an even head count), else through outf
 // (then required, f32 scratch) and the rows quantizer.
-hipError_t launch_attention(const uint16_t *q, const uint16_t *kp, const uint16_t *vtp,
-                            int64_t p, const uint16_t *ko, const uint16_t *vto, int64_t so,
-                            int64_t b, int64_t h, int64_t sq, float scale, uint16_t *out,
-                            hipStream_t stream, float *outf = nullptr);
+hipError_t launch_attention(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
+                            float scale, uint16_t *out, hipStream_t stream, float *outf = nullptr);
 // Masked attention (build_block_causal_mask semantics): img [sq] image block
 // ids (-1 text) for a prefix-less call where queries and keys are one
-// sequence (so == sq), kvalid [b][p + so] key validity; either may be null.
-// sl2 = softmax scale * log2(e), or 1 when q already carries it. lim_scratch
-// (sq int32, may be null) holds each query's last visible key for the
-// block-causal form; without it that form takes the register-staged kernel.
-hipError_t launch_attention_masked(const uint16_t *q, const uint16_t *kp, const uint16_t *vtp, int64_t p,
-                                   const uint16_t *ko, const uint16_t *vto, int64_t so, int64_t b, int64_t h,
-                                   int64_t sq, float sl2, const int32_t *img, const uint8_t *kvalid,
-                                   int32_t *lim_scratch, uint16_t *out, hipStream_t stream,
-                                   float *outf = nullptr, const float *k_prefix_norm = nullptr,
-                                   float q_norm = 0.f, float k_own_norm = 0.f, int out_qblk = 0);
+// sequence (own.len == sq), kvalid [b][prefix + own] key validity; either may be
+// null. sl2 = softmax scale * log2(e), or 1 when q already carries it.
+// lim_scratch (sq int32, may be null) holds each query's last visible key for
+// the block-causal form; without it every key window is looked at.
+hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
+                                   float sl2, const int32_t *img, const uint8_t *kvalid, int32_t *lim_scratch,
+                                   uint16_t *out, hipStream_t stream, float *outf = nullptr,
+                                   const float *k_prefix_norm = nullptr, float q_norm = 0.f, float k_own_norm = 0.f,
+                                   int out_qblk = 0);
 // The same with q already multiplied by scale * log2(e) (the QKV epilogue's
 // q_scale), so scores are in log2 units.
-hipError_t launch_attention_log2(const uint16_t *q, const uint16_t *kp, const uint16_t *vtp,
-                                 int64_t p, const uint16_t *ko, const uint16_t *vto, int64_t so,
-                                 int64_t b, int64_t h, int64_t sq, uint16_t *out, hipStream_t stream,
-                                 float *outf = nullptr, const float *k_prefix_norm = nullptr,
-                                 float q_norm = 0.f, float k_own_norm = 0.f, int out_qblk = 0);
+hipError_t launch_attention_log2(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
+                                 uint16_t *out, hipStream_t stream, float *outf = nullptr,
+                                 const float *k_prefix_norm = nullptr, float q_norm = 0.f, float k_own_norm = 0.f,
+                                 int out_qblk = 0);
 // Score bound of the fast kernels (both launches above): with q_norm >= every
 // query's norm (as passed, before sl2), k_own_norm >= every own key's norm and,
 // when there is a prefix, *k_prefix_norm (device) >= every prefix key's norm,
@@ -205,8 +213,9 @@ hipError_t launch_row_norm_max(const uint16_t *k, int64_t rows, float *part, flo
 hipError_t launch_qk_prep(const float *x, int64_t b, int64_t s, int64_t h, const float *w,
                           const float *pe, int mode, uint16_t *out, hipStream_t stream);
 
-// [B,H,S,128] bf16 -> [B,H,128,S] bf16 (and back when inverse != 0).
-hipError_t launch_transpose_sd(const uint16_t *in, int64_t bh, int64_t s, uint16_t *out,
+// [B,H,S,128] bf16 -> [B,H,128,ld] bf16 (and back when inverse != 0); row
+// elements from s on are written 0.
+hipError_t launch_transpose_sd(const uint16_t *in, int64_t bh, int64_t s, int64_t ld, uint16_t *out,
                                int inverse, hipStream_t stream);
 
 // ---- the denoising step around the blocks (step.hip), all f32 ----

@@ -416,16 +416,17 @@ __global__ __launch_bounds__(256, 2) void qgemm_kernel(const uint16_t *__restric
 #pragma unroll
                 for (int i = 0; i < 8; i++) v[i] = cs[(r0 + i) * CP + d];
                 const int64_t b = m / S, s = m % S;
-                if ((S & 7) == 0 && (s & 7) == 0 && m + 7 < M) {
+                uint16_t *dst = ep.vt + ((b * H + head) * 128 + d) * ep.vt_ld + s;
+                if (s + 7 < S && m + 7 < M && ((uintptr_t)dst & 15) == 0) {
                     u32x4 pk{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]),
                              pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
-                    *(u32x4 *)(ep.vt + ((b * H + head) * 128 + d) * S + s) = pk;
+                    *(u32x4 *)dst = pk;
                 } else {
                     for (int i = 0; i < 8; i++) {
                         const int64_t mi = m + i;
                         if (mi >= M) break;
                         const int64_t bi = mi / S, si = mi % S;
-                        ep.vt[((bi * H + head) * 128 + d) * S + si] =
+                        ep.vt[((bi * H + head) * 128 + d) * ep.vt_ld + si] =
                             (uint16_t)(pack_bf16x2(v[i], 0.f) & 0xffffu);
                     }
                 }
@@ -634,7 +635,7 @@ EpiParams rows_from(const EpiParams &ep, int epi, const GemmWeight &w, int64_t h
         const int64_t S = ep.seq, H = ep.heads, b0 = head / S, s0 = head % S;
         if (ep.q) e.q = ep.q + (b0 * H * S + s0) * 128;
         if (ep.k) e.k = ep.k + (b0 * H * S + s0) * 128;
-        if (ep.vt) e.vt = ep.vt + b0 * H * 128 * S + s0;
+        if (ep.vt) e.vt = ep.vt + b0 * H * 128 * ep.vt_ld + s0;
         if (ep.v_bhsd) e.v_bhsd = ep.v_bhsd + (b0 * H * S + s0) * 128;
         if (ep.pe) e.pe = ep.pe + s0 * 128;
     }

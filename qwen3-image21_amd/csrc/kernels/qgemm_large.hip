@@ -617,13 +617,14 @@ __global__ __launch_bounds__(256, 1) void qgemm_large_kernel(const uint16_t *__r
                 if (m >= M) continue;
                 const u32x4 v = *(const u32x4 *)(tile + d * 128 + ((ch * 8) ^ ((d & 15) << 3)));
                 const int64_t b = m / S, s = m % S;
-                if ((S & 7) == 0 && m + 7 < M) {
-                    *(u32x4 *)(ep.vt + ((b * H + head) * 128 + d) * S + s) = v;
+                uint16_t *dst = ep.vt + ((b * H + head) * 128 + d) * ep.vt_ld + s;
+                if (s + 7 < S && m + 7 < M && ((uintptr_t)dst & 15) == 0) {
+                    *(u32x4 *)dst = v;
                 } else {
                     for (int e = 0; e < 8; e++) {
                         const int64_t me = m + e;
                         if (me >= M) break;
-                        ep.vt[((me / S * H + head) * 128 + d) * S + me % S] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+                        ep.vt[((me / S * H + head) * 128 + d) * ep.vt_ld + me % S] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
                     }
                 }
             }

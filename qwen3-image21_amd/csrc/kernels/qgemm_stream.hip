@@ -741,8 +741,8 @@ __device__ void unit_epilogue(const float *part, const Plan &p, int64_t unit, in
                     *(uint32_t *)(dst + ((b * H + head) * S + s) * 128 + 2 * lane) = pack_bf16x2(y0, y1);
                 } else {
                     const uint32_t pk = pack_bf16x2(x0, x1);
-                    ep.vt[((b * H + head) * 128 + 2 * lane) * S + s] = (uint16_t)(pk & 0xffffu);
-                    ep.vt[((b * H + head) * 128 + 2 * lane + 1) * S + s] = (uint16_t)(pk >> 16);
+                    ep.vt[((b * H + head) * 128 + 2 * lane) * ep.vt_ld + s] = (uint16_t)(pk & 0xffffu);
+                    ep.vt[((b * H + head) * 128 + 2 * lane + 1) * ep.vt_ld + s] = (uint16_t)(pk >> 16);
                     if (ep.v_bhsd) *(uint32_t *)(ep.v_bhsd + ((b * H + head) * S + s) * 128 + 2 * lane) = pk;
                 }
             }
@@ -1675,10 +1675,10 @@ __global__ __launch_bounds__(256) void stream_qkv_kernel(const float *__restrict
         const int d = tid >> 1, t0 = (VT_T / 2) * (tid & 1);
         const int nt = (int)min((int64_t)(VT_T / 2), S - s0 - t0);
         if (nt <= 0) return;
-        uint16_t *dst = ep.vt + ((b * H + head) * 128 + d) * S + s0 + t0;
+        uint16_t *dst = ep.vt + ((b * H + head) * 128 + d) * ep.vt_ld + s0 + t0;
         const uint16_t *src = tile + d * VT_P + t0;
-        if (nt == VT_T / 2 && (S & 7) == 0) {
-            // 16 B aligned: S and s0 + t0 are multiples of 8
+        if (nt == VT_T / 2) {
+            // 16 B aligned: vt_ld and s0 + t0 are multiples of 8
 #pragma unroll
             for (int j = 0; j < VT_T / 16; j++) {
                 u32x4 w;

@@ -790,7 +790,7 @@ __global__ __launch_bounds__(64 * NW, 1) void qgemm_wide_kernel(const uint16_t *
                         *(const u32x4 *)((uint16_t *)lds + hg * (256 * 128) + t * 128 + 8 * (c ^ (t & 15)));
                 }
             } else {
-                // v: transposed to vt [B,H,128,S] (consecutive lanes hold
+                // v: transposed to vt [B,H,128,vt_ld] (consecutive lanes hold
                 // consecutive tokens of a d row), and [B,H,S,128] when v_bhsd is set
                 const int dbase = 32 * sub + 4 * g;
 #pragma unroll
@@ -798,11 +798,11 @@ __global__ __launch_bounds__(64 * NW, 1) void qgemm_wide_kernel(const uint16_t *
                     if (m0 + 32 * i + l32 >= M) continue;
                     uint32_t b, s;
                     tok(32 * i + l32, b, s);
-                    uint16_t *vrow = ep.vt + ((int64_t)b * H + head) * 128 * S + s;
+                    uint16_t *vrow = ep.vt + ((int64_t)b * H + head) * 128 * ep.vt_ld + s;
 #pragma unroll
                     for (int r = 0; r < 16; r++) {
                         const int d = dbase + 8 * (r >> 2) + (r & 3);
-                        vrow[(int64_t)d * S] = (uint16_t)(pack_bf16x2(acc[i][r], 0.f) & 0xffffu);
+                        vrow[(int64_t)d * ep.vt_ld] = (uint16_t)(pack_bf16x2(acc[i][r], 0.f) & 0xffffu);
                     }
                     if (ep.v_bhsd) {
                         uint16_t *brow = ep.v_bhsd + (((int64_t)b * H + head) * S + s) * 128;

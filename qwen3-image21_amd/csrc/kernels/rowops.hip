@@ -389,8 +389,8 @@ __global__ void v_prep_kernel(const float *__restrict__ x, int64_t B, int64_t S,
     vt[i] = (uint16_t)(pack_bf16x2(x[((b * S + s) * H + h) * 128 + d], 0.f) & 0xffffu);
 }
 
-// ---- [BH][S][128] <-> [BH][128][S] bf16 via 64x64 LDS tiles ----
-__global__ __launch_bounds__(256) void transpose_sd_kernel(const uint16_t *__restrict__ in, int64_t S,
+// ---- [BH][S][128] <-> [BH][128][ld] bf16 via 64x64 LDS tiles ----
+__global__ __launch_bounds__(256) void transpose_sd_kernel(const uint16_t *__restrict__ in, int64_t S, int64_t ld,
                                                            uint16_t *__restrict__ out, int inverse) {
     __shared__ uint16_t tile[64][65];
     const int64_t bh = blockIdx.z;
@@ -403,14 +403,14 @@ __global__ __launch_bounds__(256) void transpose_sd_kernel(const uint16_t *__res
             tile[r][tx] = s < S ? in[(bh * S + s) * 128 + d] : (uint16_t)0;
         } else {
             const int64_t d = d0 + r, s = s0 + tx;
-            tile[tx][r] = s < S ? in[(bh * 128 + d) * S + s] : (uint16_t)0;
+            tile[tx][r] = s < S ? in[(bh * 128 + d) * ld + s] : (uint16_t)0;
         }
     }
     __syncthreads();
     for (int r = ty; r < 64; r += 4) {
         if (!inverse) {
             const int64_t d = d0 + r, s = s0 + tx;
-            if (s < S) out[(bh * 128 + d) * S + s] = tile[tx][r];
+            if (s < ld) out[(bh * 128 + d) * ld + s] = tile[tx][r];
         } else {
             const int64_t s = s0 + r, d = d0 + tx;
             if (s < S) out[(bh * S + s) * 128 + d] = tile[r][tx];
@@ -503,11 +503,11 @@ hipError_t launch_qk_prep(const float *x, int64_t b, int64_t s, int64_t h, const
     return hipGetLastError();
 }
 
-hipError_t launch_transpose_sd(const uint16_t *in, int64_t bh, int64_t s, uint16_t *out, int inverse,
+hipError_t launch_transpose_sd(const uint16_t *in, int64_t bh, int64_t s, int64_t ld, uint16_t *out, int inverse,
                                hipStream_t stream) {
     if (bh <= 0 || s <= 0) return hipSuccess;
     dim3 grid((unsigned)((s + 63) / 64), 2u, (unsigned)bh);
-    transpose_sd_kernel<<<grid, dim3(256), 0, stream>>>(in, s, out, inverse);
+    transpose_sd_kernel<<<grid, dim3(256), 0, stream>>>(in, s, ld, out, inverse);
     return hipGetLastError();
 }
 

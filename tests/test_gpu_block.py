@@ -127,6 +127,26 @@ def test_block_matches_oracle(torch_cuda, qctx, attn_type, down_type, b, s, p):
     check_modes(SMALL, w, x, mod, pe, kpre, vpre, runs, want_kv=True)
 
 
+@pytest.mark.parametrize("b,s,p,act", [(1, 77, 203, "candle"), (2, 147, 33, "candle"), (2, 523, 65, "bf16"),
+                                       (1, 1031, 131, "candle")])
+def test_block_ragged_tokens_ignore_row_padding(torch_cuda, qctx, b, s, p, act):
+    """Token counts and prefixes that are no multiple of 8 leave V^T row padding in
+    the workspace. A larger call on NaN inputs fills the workspace with NaN first:
+    the output is the one of a context of its own, bit for bit, and the oracle's."""
+    torch = torch_cuda
+    w, x, mod, pe, kpre, vpre = make_case(b + s + p, SMALL, b, s, p, synth.Q4_K, synth.Q6_K)
+    mode = qimm.ACT_CANDLE if act == "candle" else qimm.ACT_BF16
+    own = qimm.Context(0)
+    alone, _ = run_block(torch, own, SMALL, w, x, mod, pe, kpre, vpre, act=mode)
+    own.close()
+    wn, xn, modn, pen, _, _ = make_case(3, SMALL, 1, 2048, 0, synth.Q4_K, synth.Q6_K)
+    run_block(torch, qctx, SMALL, wn, np.full_like(xn, np.nan), modn, pen)
+    got, _ = run_block(torch, qctx, SMALL, w, x, mod, pe, kpre, vpre, act=mode)
+    assert np.array_equal(got, alone)
+    ref, _, _ = O.block_forward(SMALL, w, x, mod, pe, kpre, vpre, mode=O.CANDLE if act == "candle" else O.EXACT)
+    check(got, ref, x, exact=act == "bf16")
+
+
 def test_block_in_place_and_separate_mlp_inputs(torch_cuda, qctx):
     w, x, mod, pe, kpre, vpre = make_case(7, SMALL, 1, 64, 16, synth.Q8_0, synth.Q8_0, fused=False)
     runs = run_modes(torch_cuda, qctx, SMALL, w, x, mod, pe, kpre, vpre, alias=True)

@@ -338,6 +338,29 @@ def test_attention_eight_wave_form_ragged_segments(torch_cuda, qctx, sq, p, so):
     assert max_abs_rel(got, want) <= 2e-2, max_abs_rel(got, want)
 
 
+@pytest.mark.parametrize("h,b,sq,p,so", [
+    (2, 1, 65, 1, 128),       # one prefix key
+    (2, 1, 70, 57, 64),       # prefix of one window, 7 keys short of it
+    (2, 2, 130, 63, 72),      # last V^T chunk holds seven keys
+    (2, 1, 40, 65, 120),      # second prefix window with a single key
+    (1, 2, 90, 217, 8),       # several prefix windows, one key in the last chunk
+    (1, 1, 20, 0, 1),         # a single key: V^T rows of 2 B, through registers
+    (2, 1, 129, 0, 127),      # dense V^T of an odd length
+    (1, 2, 200, 131, 203),    # both lengths odd
+    (2, 1, 77, 24, 196),      # V^T rows on 8 B
+    (128, 2, 193, 9, 131),    # the 8-wave form with V^T through registers
+    (128, 2, 250, 131, 136),  # the 8-wave form with a ragged prefix
+])
+def test_attention_any_lengths(torch_cuda, qctx, h, b, sq, p, so):
+    """Segment ends inside a 64-key window and inside an 8-key V^T chunk: the
+    prefix rows are padded by the cache (copied into LDS, cleared past the end),
+    the own V^T is the caller's dense one (through registers unless so % 8 == 0)."""
+    got, q, ko, vo, kp, vp = _attention_case(torch_cuda, qctx, b, h, sq, p, so, seed=sq + p + so)
+    want = O.attention(q, ko, vo, kp, vp, mode=O.EXACT)
+    assert cos_sim(got, want) >= 0.9999, cos_sim(got, want)
+    assert max_abs_rel(got, want) <= 2e-2, max_abs_rel(got, want)
+
+
 @pytest.mark.parametrize("sq", [4096, 2304])
 def test_attention_config2_shape_sampled_rows(torch_cuda, qctx, sq):
     """B1 H32, sq image queries over 256 prefix + sq own keys; sampled query rows.

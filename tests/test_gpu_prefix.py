@@ -128,6 +128,22 @@ def test_attention_cached_step_key_valid(torch_cuda, qctx, b, h, p, so, pads):
     assert cos_sim(got, want) >= 0.9999 and max_abs_rel(got, want) <= 2e-2
 
 
+@pytest.mark.parametrize("runs", [[(-1, 77)], [(-1, 101), (0, 300), (-1, 102)], [(0, 65), (1, 130), (-1, 66)]])
+def test_attention_block_causal_odd_lengths(torch_cuda, qctx, runs):
+    """Token counts off the 8-key chunks: the caller's dense V^T goes through registers."""
+    ids = np.concatenate([np.full(n, i, dtype=np.int64) for i, n in runs])
+    kvalid = np.ones((2, ids.size), dtype=np.uint8)
+    kvalid[1, 11:17] = 0  # padded keys of the second prompt (every query still sees earlier ones)
+    got, want = _masked_case(torch_cuda, qctx, ids, kvalid, 3, seed=ids.size)
+    assert cos_sim(got, want) >= 0.9999 and max_abs_rel(got, want) <= 2e-2, (cos_sim(got, want),
+                                                                             max_abs_rel(got, want))
+
+
+@pytest.mark.parametrize("p,so", [(33, 131), (150, 64), (64, 77)])
+def test_attention_cached_step_key_valid_odd_lengths(torch_cuda, qctx, p, so):
+    test_attention_cached_step_key_valid(torch_cuda, qctx, 2, 2, p, so, (0, p // 3))
+
+
 def _masked_case(torch, qctx, ids, kvalid, h, rows=None, seed=0, qmul=1.0):
     """Prefix-less masked attention of ids.size tokens on the GPU and in the oracle (exact mode),
     on all rows or on the listed query rows."""
