@@ -443,33 +443,34 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
                         __builtin_amdgcn_global_load_lds((const void *)(vg + vrow[i] * (uint32_t)(2 * b.ld) + 2 * gc),
                                                          (lds_ptr_t)(base + TILE + (wave + NW * i) * 1024), 16, 0, 0);
                     }
+                    // an end inside a chunk: the lane's own V^T chunks are cleared from the
+                    // end on (a masked key's probability is 0, and the row padding may hold
+                    // anything: 0 x NaN must not arise). Waiting for them here, once per
+                    // segment, keeps the test out of the other blocks' path (1.2% there).
+                    if (b.hi & 7) {
+                        __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+#pragma unroll 1
+                        for (int i = 0; i < DI; i++) {
+                            u32x4 *p = (u32x4 *)(base + TILE + (wave + NW * i) * 1024 + 16 * lane);
+                            const int left = b.hi - (((lane & 7) ^ (((8 * (wave + NW * i) + (lane >> 3)) >> 1) & 7)) << 3);
+                            u32x4 v = *p;
+#pragma unroll
+                            for (int e = 0; e < 4; e++) v[e] &= left > 2 * e + 1 ? 0xffffffffu : left > 2 * e ? 0xffffu : 0u;
+                            *p = v;
+                        }
+                    }
                 }
             }
             if constexpr (RV && !MASKED) load_v(b);
         };
-        // After this wave's copies of block b have landed, before the barrier that
-        // publishes them: the lane's own V^T chunks of a block whose end lies
-        // inside a chunk are cleared from the end on (a masked key's probability is
-        // 0, and the row padding may hold anything: 0 x NaN must not arise).
-        // RV writes its chunks here; the masked form has no registers to hold them
-        // over a step (132 spilled) and loads them here too.
+        // RV: the next block's chunks go to LDS at the end of a step, before the
+        // barrier that publishes them; the masked form has no registers to hold
+        // them over a step (132 spilled) and loads them here too.
         auto seal = [&](const Blk &b, int stage) __attribute__((always_inline)) {
+            if constexpr (RV && MASKED) load_v(b);
             uint8_t *base = lds + stage * STAGE + TILE;
-            if constexpr (RV) {
-                if constexpr (MASKED) load_v(b);
 #pragma unroll
-                for (int i = 0; i < DI; i++) *(u32x4 *)(base + (wave + NW * i) * 1024 + 16 * lane) = vreg[i];
-            } else if (b.hi & 7) {
-#pragma unroll 1
-                for (int i = 0; i < DI; i++) {
-                    u32x4 *p = (u32x4 *)(base + (wave + NW * i) * 1024 + 16 * lane);
-                    const int left = b.hi - (((lane & 7) ^ (((8 * (wave + NW * i) + (lane >> 3)) >> 1) & 7)) << 3);
-                    u32x4 v = *p;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] &= left > 2 * e + 1 ? 0xffffffffu : left > 2 * e ? 0xffffu : 0u;
-                    *p = v;
-                }
-            }
+            for (int i = 0; i < DI; i++) *(u32x4 *)(base + (wave + NW * i) * 1024 + 16 * lane) = vreg[i];
         };
 
         // S^T row m of a 32-key half is key pi(m) = m with bits 2 and 3 swapped,
@@ -707,7 +708,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
                 half_step(stg, 1, b.hi, kmask, kid, kb0, partial, stat);
             }
             __builtin_amdgcn_s_waitcnt(WAIT_VM0);  // vmcnt(0): block j+1 landed
-            if (j + 1 < nblk) seal(blk_of(j + 1), cur ^ 1);
+            if constexpr (RV)
+                if (j + 1 < nblk) seal(blk_of(j + 1), cur ^ 1);
             __syncthreads();
         };
 
@@ -716,7 +718,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             dma(blk_of(0), 0);
         }
         __builtin_amdgcn_s_waitcnt(WAIT_VM0);
-        if (nblk > 0) seal(blk_of(0), 0);
+        if constexpr (RV)
+            if (nblk > 0) seal(blk_of(0), 0);
         __syncthreads();
         // the fixed-reference form when the score bound allows it (wave-uniform)
         bool stat_ok = false;
@@ -904,18 +907,19 @@ hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64
     bool rounded = false;
     const KeyMask km{nullptr, nullptr, prefix.len + own.len};
     const int nw = fast_waves(b * h, sq);
+    constexpr int SM = PRE ? 0 : 2;  // without the block's norms no score bound is known
     if (!rows16(s0) || !rows16(s1)) {
         if (nw == 4)
             launch_fast<4, false, false, 2, false, true>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
         else
             launch_fast<8, false, false, 2, false, true>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
-    } else if (out_qblk == 256 && nw == 8 && h % 2 == 0) {
-        launch_fast<8, PRE, false, 0, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, nullptr, sb, 0, stream);
+    } else if (PRE && out_qblk == 256 && nw == 8 && h % 2 == 0) {
+        launch_fast<8, true, false, 0, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, nullptr, sb, 0, stream);
         rounded = true;
     } else if (nw == 4) {
-        launch_fast<4, PRE, false>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
+        launch_fast<4, PRE, false, SM>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
     } else {
-        launch_fast<8, PRE, false>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
+        launch_fast<8, PRE, false, SM>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
     }
     return finish_q8k(out_qblk, rounded, outf, b, h, sq, out, stream);
 }
