@@ -85,7 +85,10 @@ int qimm_stream_synchronize(qimm_ctx *ctx, void *stream);
  * blocks running along cols, exactly as candle's quantized VarBuilder hands
  * it to QMatMul::from_arc (src/quantized_transformer.rs:31-33). bytes must be
  * rows * cols / block_size * block_bytes. The library owns the device copy
- * and may re-stride blocks for aligned loads; values are never changed. */
+ * and may re-stride blocks for aligned loads; values are never changed. Beside
+ * the blocks of a quantized tensor it keeps their values as bf16 rows (2 bytes
+ * a value) for the products of many tokens, as long as at least half of the
+ * device memory stays free; qimm_weight_device_bytes counts both. */
 int qimm_weight_upload(qimm_ctx *ctx, int ggml_type, int64_t rows, int64_t cols,
                        const void *host_bytes, size_t nbytes, qimm_weight **out);
 int qimm_weight_free(qimm_weight *w);

@@ -27,6 +27,7 @@ struct qimm_weight {
     int64_t rows = 0, cols = 0;
     void *dev = nullptr;        // codes / blocks
     void *dev_scales = nullptr; // Q8_0 f16 scales
+    void *dev_bf16 = nullptr;   // bf16 rows of a quantized weight (keep_bf16_rows)
     size_t dev_bytes = 0;
     qimm::GemmWeight gw{};
 };

@@ -72,12 +72,17 @@ struct GemmWeight {
     int64_t n, k;
     const uint8_t *q;       // codes / blocks
     const uint16_t *scales; // WF_Q8_0 only
+    // the weight's values as bf16 rows [N][K]: q itself for WF_BF16, for the
+    // quantized formats the copy that the upload lays out (null: none was made)
+    const uint16_t *bf16 = nullptr;
 };
 
 // y = A[M,K] (bf16, row stride lda) x W[N,K]^T with the epilogue selected by epi.
-// Dispatches to the 256x256 large-M kernel when qgemm_large_fits (at least 512
-// rows, and more 128x128 tiles than one wave of two workgroups per CU), else to
-// the 128x128 kernel.
+// Short M streams the weights (launch_qgemm_stream). Above it, weights with bf16
+// rows take launch_qgemm_bf16 or the 128x128 kernel, whichever is estimated
+// faster; without bf16 rows the 256x256 kernels take what qgemm_large_fits (at
+// least 512 rows, and more 128x128 tiles than one wave of two workgroups per
+// CU), the 128x128 kernel the rest.
 hipError_t launch_qgemm(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda,
                         int epi, const EpiParams &ep, hipStream_t stream);
 bool qgemm_large_fits(const GemmWeight &w, int64_t m);
@@ -106,6 +111,23 @@ bool qgemm_wide_fits(const GemmWeight &w);
 bool qgemm_wide_pairs_fit(const GemmWeight &w);
 hipError_t launch_qgemm_wide(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda, int epi,
                              const EpiParams &ep, hipStream_t stream);
+// The large-M kernel over bf16 weight rows (GemmWeight::bf16; N % 256 == 0,
+// K % 128 == 0), and how it takes a product: `head` tiles of 256 tokens and the
+// rest in tiles of 128, or (splits > 1) tiles of 128 split over K with partial
+// sums in EpiParams::part_ws; us = the estimated time.
+bool qgemm_bf16_fits(const GemmWeight &w);
+struct Bf16Plan {
+    int64_t head;
+    int splits;
+    double us;
+};
+Bf16Plan qgemm_bf16_plan(const GemmWeight &w, int64_t m, bool may_split);
+// estimated time of its SwiGLU form with the Q8_K rounding (N % 512 == 0)
+double qgemm_bf16_q8k_us(const GemmWeight &w, int64_t m);
+hipError_t launch_qgemm_bf16(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda, int epi,
+                             const EpiParams &ep, const Bf16Plan &plan, hipStream_t stream);
+// out [N][K] = the bf16 values of a quantized weight
+hipError_t launch_weight_rows_bf16(const GemmWeight &w, uint16_t *out, hipStream_t stream);
 // Sum of split-K partials part[splits][m][N] (f32) in split order, with the
 // epilogue epi applied (the second kernel of the split paths).
 hipError_t launch_split_epilogue(const float *part, int splits, int64_t m, int64_t N, int epi, const EpiParams &ep,

@@ -505,10 +505,14 @@ int device_cu_count() {
 // picks the measured best share count or one within 3% of it on each, e.g.
 // Q8_0 3072x9216 at 256 tokens: 4 shares, 36.7 us (2 shares: 59.7), and
 // 9216x3072: 3 shares, 37.5 us (unsplit: 40.3).
-int qgemm_mid_splits(const GemmWeight &w, int64_t m) {
-    if (m <= 0 || qgemm_large_fits(w, m) || qgemm_stream_fits(w, m)) return 1;
+namespace {
+struct MidCost {
+    int splits;
+    double us;
+};
+MidCost mid_cost(const GemmWeight &w, int64_t m) {
     const int64_t tiles = (w.n / BN) * ((m + BM - 1) / BM), cus = device_cus(), steps = w.k / BK;
-    if (cus <= 0) return 1;
+    if (cus <= 0) return {1, 0.0};
     auto cost = [&](int s) {
         const int64_t per_cu = (tiles * s + cus - 1) / cus;
         const double st = (double)(steps / s);
@@ -525,10 +529,49 @@ int qgemm_mid_splits(const GemmWeight &w, int64_t m) {
             best = s;
         }
     }
-    return best;
+    return {best, best_cost};
+}
+}  // namespace
+
+int qgemm_mid_splits(const GemmWeight &w, int64_t m) {
+    if (m <= 0 || qgemm_large_fits(w, m) || qgemm_stream_fits(w, m)) return 1;
+    return mid_cost(w, m).splits;
 }
 
 namespace {
+
+// Whether a product of m rows takes the kernel over bf16 rows, and how: above
+// the weight-streaming sizes, when it is estimated faster than the 128x128
+// kernel (whose cost estimate, fitted at 256 and 384 tokens, is 1.1 times short
+// above, for Q6_K 1.3 times: 4096 x 12288 at 300 / 512 / 1024 tokens 70 / 74 /
+// 130 us estimated, 83-88 / 97-103 / 180 measured). Below, few tokens are bound by the weight
+// bytes, and the 128x128 kernel reads the codes. splits 0: no.
+Bf16Plan bf16_plan(const GemmWeight &w, int64_t m, int64_t lda, bool may_split) {
+    if (!qgemm_bf16_fits(w) || lda > ((int64_t)1 << 22) || qgemm_stream_fits(w, m)) return {0, 0, 0.0};
+    const Bf16Plan p = qgemm_bf16_plan(w, m, may_split);
+    const MidCost mid = mid_cost(w, m);
+    const double mid_us = mid.us * (w.fmt == WF_Q6_K ? 1.3 : m > 384 ? 1.1 : 1.0);
+    return mid_us > 0.0 && mid_us <= p.us ? Bf16Plan{0, 0, mid_us} : p;
+}
+// scratch of a split plan
+size_t bf16_workspace(const GemmWeight &w, int64_t m, const Bf16Plan &p) {
+    return p.splits > 1 ? STREAM_COUNTER_BYTES + (size_t)p.splits * (size_t)m * (size_t)w.n * 4 : 0;
+}
+// f32 rows rounded in a pass of their own, in us
+double quant_pass_us(const GemmWeight &w, int64_t m) { return 5.0 + (double)m * (double)(w.n / 2) * 6.0 / 4.5e6; }
+// Rows of a bf16-rows product handed to a product of their own: those after the
+// last full round of 256-token tiles (4299 tokens x N = 4096: 256 tiles for 256
+// CUs, then 203 rows), where the two together are estimated faster. 0 = none.
+int64_t bf16_tail_rows(const GemmWeight &w, int64_t m, int64_t lda, bool q8k, double whole_us) {
+    const int64_t cus = device_cus(), nt = w.n / 256, h = cus > 0 ? (m / 256) * nt / cus * cus / nt : 0;
+    const int64_t tail = m - 256 * h;
+    if (h <= 0 || tail <= 0 || tail >= 512) return 0;
+    const Bf16Plan ph = bf16_plan(w, 256 * h, lda, false), pt = bf16_plan(w, tail, lda, true);
+    if (!ph.splits) return 0;
+    const double head_us = q8k ? std::min(qgemm_bf16_q8k_us(w, 256 * h), ph.us + quant_pass_us(w, 256 * h)) : ph.us;
+    const double tail_us = pt.splits || pt.us > 0.0 ? pt.us + (q8k ? quant_pass_us(w, tail) : 0.0) : 25.0;
+    return head_us + tail_us + 3.0 < whole_us ? tail : 0;
+}
 
 // Rows of a large-M product handed to the shorter-M paths so that the 256x256
 // kernel runs whole waves: when the 256x256 tiles leave a last, partial wave
@@ -562,7 +605,7 @@ enum class SmallPath { STREAM, SPLIT, WHOLE };
 SmallPath small_path(const GemmWeight &w, int64_t m, const EpiParams &ep) {
     if (qgemm_stream_fits(w, m) && ep.part_ws && ep.part_ws_bytes >= qgemm_stream_workspace(w, m))
         return SmallPath::STREAM;
-    if (qgemm_mid_splits(w, m) > 1 && ep.part_ws && ep.part_ws_bytes >= qgemm_workspace(w, m)) return SmallPath::SPLIT;
+    if (qgemm_mid_splits(w, m) > 1 && ep.part_ws && ep.part_ws_bytes >= mid_workspace(w, m)) return SmallPath::SPLIT;
     return SmallPath::WHOLE;
 }
 
@@ -588,6 +631,12 @@ hipError_t launch_small(const GemmWeight &w, const uint16_t *a, int64_t m, int64
 }  // namespace
 
 size_t qgemm_workspace(const GemmWeight &w, int64_t m) {
+    if (const Bf16Plan p = bf16_plan(w, m, w.k, true); p.splits) {
+        size_t need = bf16_workspace(w, m, p);
+        for (bool q8k : {false, true})
+            if (const int64_t tail = bf16_tail_rows(w, m, w.k, q8k, 1e30)) need = std::max(need, qgemm_workspace(w, tail));
+        return need;
+    }
     if (qgemm_large_fits(w, m)) {
         size_t need = 0;
         for (bool pairs : {false, true})
@@ -642,11 +691,53 @@ EpiParams rows_from(const EpiParams &ep, int epi, const GemmWeight &w, int64_t h
     return e;
 }
 
+// A product over bf16 rows: the tail after full rounds as a product of its own
+// where that is faster and its epilogue's rows can be shifted, else one launch;
+// the rounding of the SwiGLU hidden state in the epilogue where it can be (whole
+// Q8_K blocks need 512 weight rows per tile), else in a pass over f32 rows.
+hipError_t launch_bf16_rows(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda, int epi, const EpiParams &ep,
+                            Bf16Plan p, hipStream_t stream) {
+    // q/k/v reduces whole sequences only; any split needs its scratch
+    if (p.splits > 1 && (ep.part_ws_bytes < bf16_workspace(w, m, p) || (epi == EPI_QKV && m % ep.seq)))
+        p = qgemm_bf16_plan(w, m, false);
+    const bool swiglu = epi == EPI_SWIGLU, q8k = swiglu && ep.hmid_q8k, q8_0 = swiglu && ep.hmid_q8_0;
+    if (q8k && (!ep.hmid || !ep.hmid_f32 || ep.ldh % 256 || (w.n / 2) % 256)) return hipErrorInvalidValue;
+    if (q8_0 && (!ep.hmid || !ep.hmid_f32 || (w.n / 2) % 32)) return hipErrorInvalidValue;
+    const double q8k_us = q8k ? qgemm_bf16_q8k_us(w, m) : 0.0, sep_us = p.us + quant_pass_us(w, m);
+    const double us = q8k ? std::min(q8k_us, sep_us) : p.us;
+    if (const int64_t tail = ep.part_ws ? bf16_tail_rows(w, m, lda, q8k, us) : 0) {
+        const int64_t head = m - tail;
+        bool shift = ep.part_ws_bytes >= qgemm_workspace(w, tail);
+        if (epi == EPI_RESID) shift = shift && ep.g_rows_per > 0 && head / ep.g_rows_per == (m - 1) / ep.g_rows_per;
+        if (epi == EPI_QKV) {
+            const Bf16Plan pt = bf16_plan(w, tail, lda, false);
+            shift = shift && ep.seq > 0 && head / ep.seq == (m - 1) / ep.seq &&
+                    (pt.splits ? true : small_path(w, tail, ep) == SmallPath::WHOLE);
+        }
+        if (shift) {
+            const hipError_t e = launch_qgemm(w, a, head, lda, epi, ep, stream);
+            if (e != hipSuccess) return e;
+            return launch_qgemm(w, a + head * lda, tail, lda, epi, rows_from(ep, epi, w, head), stream);
+        }
+    }
+    if ((q8k && sep_us < q8k_us) || (q8_0 && p.splits > 1)) {
+        EpiParams e = ep;
+        e.hmid_q8k = e.hmid_q8_0 = 0;
+        const hipError_t err = launch_qgemm_bf16(w, a, m, lda, EPI_SWIGLU, e, p, stream);
+        if (err != hipSuccess) return err;
+        return launch_quant_rows(ep.hmid_f32, ep.ldh, m, w.n / 2, q8k ? 256 : 32, ep.hmid, ep.ldh, stream);
+    }
+    if (q8k) p.splits = 1;
+    return launch_qgemm_bf16(w, a, m, lda, epi, ep, p, stream);
+}
+
 }  // namespace
 
 hipError_t launch_qgemm(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda, int epi,
                         const EpiParams &ep, hipStream_t stream) {
     if (m <= 0) return hipSuccess;
+    if (const Bf16Plan p = bf16_plan(w, m, lda, ep.part_ws != nullptr); p.splits && (epi != EPI_QKV || ep.hidden % 256 == 0))
+        return launch_bf16_rows(w, a, m, lda, epi, ep, p, stream);
     // a last, nearly empty round of 256x256 tiles: those rows as a shorter-M
     // product of their own (whole rounds above, the 128x128 or short-M path
     // for the tail), each part with its own form of the epilogue

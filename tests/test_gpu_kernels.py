@@ -101,6 +101,51 @@ def test_qmatmul_matches_bf16_weight_products(torch_cuda, qctx, t, m, n, k):
         assert cos_sim(got, yc) >= 0.9999 and max_abs_rel(got, yc) <= 2e-2
 
 
+# the kernel over bf16 rows: two k steps (the least), an odd and a large number of steps past
+# its three and two stages, one token past a tile of 128 and of 256, both tile sizes in one
+# launch (3072 x 12288: ten tiles of 256, four of 128), shares of K with unequal steps, and a
+# tail after full rounds (4299 rows x N = 4096)
+@pytest.mark.parametrize("t,m,n,k", [(synth.Q8_0, 129, 256, 128), (synth.BF16, 200, 256, 128), (synth.BF16, 385, 512, 384),
+                                     (synth.Q4_K, 257, 512, 1280), (synth.Q6_K, 300, 512, 5120),
+                                     (synth.Q4_K, 100, 1024, 4096), (synth.Q8_0, 3072, 12288, 128),
+                                     (synth.Q6_K, 4299, 4096, 256), (synth.Q4_K, 1025, 4096, 1024)])
+def test_qmatmul_bf16_rows(torch_cuda, qctx, t, m, n, k):
+    """Products of the bf16 activations and the bf16-rounded weights, f32 sums in any order."""
+    got, a, w = _gemm_case(torch_cuda, qctx, t, m, n, k, seed=m + n + k + t)
+    Wb = O.bf16_round(O.dequantize(t, w, n * k).reshape(n, k)).astype(np.float64)
+    rows = np.unique(np.concatenate([np.arange(min(m, 140)), np.arange(m // 2, m // 2 + 20), np.arange(m - 45, m)]))
+    a = a[rows].astype(np.float64)
+    scale = np.abs(a) @ np.abs(Wb).T
+    assert np.isfinite(got).all()
+    assert np.all(np.abs(got[rows] - a @ Wb.T) <= 2e-4 * scale + 1e-6)
+
+
+def test_no_room_for_bf16_rows(torch_cuda, qctx):
+    """With less than half of the device memory free an upload keeps the codes alone,
+    and the decoding kernels give the products (and a second upload with room, the rows)."""
+    torch = torch_cuda
+    m, n, k = 2304, 4096, 1024  # more 128x128 tiles than two per CU
+    rng = np.random.default_rng(77)
+    a_dev, _ = bf16_dev(torch, rng.standard_normal((m, k)).astype(np.float32))
+    free, total = torch.cuda.mem_get_info()
+    for t in (synth.Q4_K, synth.Q8_0, synth.Q6_K):
+        _, w, _, _ = synth.weight(rng, t, n, k)
+        ys, sizes = [], []
+        for hold_bytes in (0, free - total // 2 + (1 << 30)):
+            hold = torch.empty(max(hold_bytes, 0), dtype=torch.uint8, device="cuda")
+            W = qctx.upload(t, n, k, w.tobytes())
+            sizes.append(W.device_bytes())
+            del hold
+            torch.cuda.empty_cache()
+            y = torch.empty((m, n), dtype=torch.float32, device="cuda")
+            qctx.qmatmul(W, a_dev.data_ptr(), m, k, y.data_ptr(), synth.F32, stream(torch))
+            ys.append(host(y))
+            W.free()
+        assert sizes[0] - sizes[1] == 2 * n * k
+        # the same bf16 products, f32 sums in another order
+        assert np.isfinite(ys[1]).all() and max_abs_rel(ys[1], ys[0]) <= 1e-5
+
+
 @pytest.mark.parametrize("m,n,k", [(16, 4096, 4096),
                                    (1, 8192, 4096),     # a single token
                                    (7, 12288, 4096),
