@@ -59,7 +59,7 @@ static inline float f16_to_f32(uint16_t h) {
 }
 
 // Lays the values of a quantized weight out as bf16 rows beside its codes, for
-// the products of many tokens: a matrix kernel over bf16 rows runs 1.33-1.45
+// the products of many tokens: a matrix kernel over bf16 rows runs 1.38-1.52
 // PFLOP/s, one that decodes beside its MFMAs 1.10-1.18, while a few tokens are
 // bound by the weight bytes and keep reading the codes. The copy takes 2 bytes
 // a value (a 32-layer model of hidden 4096: 14 GB of the card's 288), and is

@@ -7,7 +7,7 @@
 // the block's token-parallel projections (call sites 133-135, 151, 196, 202).
 //
 // What bounds it: the matrix pipe at the clock the operand data allows (all-zero
-// operands run 1.65-1.85 PFLOP/s, random ones 1.33-1.45). Decoding 32 weights
+// operands run 1.65-1.85 PFLOP/s, random ones 1.38-1.52). Decoding 32 weights
 // per lane and k step beside the MFMAs costs more than reading twice the bytes:
 // the decoding kernel of the same tile (qgemm_wide.hip) runs 1.10-1.18, and a
 // form of this kernel that decodes in its load phases 1.04-1.17.
@@ -27,8 +27,8 @@
 //    read it, so every direct load has at least a whole k step to land.
 //  - TT = 2: two phases (weight half x all tokens: 16 MFMAs each), three stages.
 // Measured against the decoding kernel (Q4_K, one process, us): at 4096 tokens
-// q/k/v 12288 x 4096 366 -> 307, gate_up 24576 x 4096 715 -> 612, 4096 x 12288
-// 349 -> 285, 4096 x 4096 126 -> 101; at 3072 tokens q/k/v 326 -> 250; at 2048
+// q/k/v 12288 x 4096 366 -> 294, gate_up 24576 x 4096 715 -> 599, 4096 x 12288
+// 349 -> 272, 4096 x 4096 126 -> 98; at 3072 tokens q/k/v 326 -> 250; at 2048
 // tokens against the 128x128 kernel 4096 x 4096 95 -> 62, 4096 x 12288 (Q6_K)
 // 313 -> 172; bf16 weights 12288 x 4096 at 2050 tokens against the four-wave
 // kernel of qgemm_large.hip 219 -> 191.
@@ -229,12 +229,16 @@ __global__ __launch_bounds__(64 * NWAVE, 1) void qgemm_bf16_kernel(const uint16_
             __builtin_amdgcn_s_waitcnt(WAIT_VM0 | (TI + WI));  // step 0 has landed
             barrier();
             if (wave >= 4) barrier();  // waves 4-7 run one barrier behind
+            // the first token half of a step is read in the last phase of the step
+            // before it: 8, 4, 8 and 4 fragment reads per phase instead of 12, 4, 8
+            // and none (4096 tokens: 12288 x 4096 307 -> 294 us, 4096 x 12288 285 -> 272)
+            rd_t(0, 0);
             auto step = [&](int kt, auto s_) __attribute__((always_inline)) {
                 constexpr int s = decltype(s_)::value;
-                phase(InFlight{}, [&] { rd_t(s, 0); rd_w(s, 0); dma_t(s ^ 1, 1, kt + 1); }, 0, 0);
+                phase(InFlight{}, [&] { rd_w(s, 0); dma_t(s ^ 1, 1, kt + 1); }, 0, 0);
                 phase(InFlight{}, [&] { rd_t(s, 1); dma_w(s ^ 1, 1, kt + 1); }, 0, 1);
                 phase(InFlight{}, [&] { rd_w(s, 1); dma_t(s, 0, kt + 2); }, 1, 0);
-                phase(InFlight{}, [&] { dma_w(s, 0, kt + 2); }, 1, 1);
+                phase(InFlight{}, [&] { rd_t(s ^ 1, 0); dma_w(s, 0, kt + 2); }, 1, 1);
             };
             for (int kt = 0; kt < KT; kt += 2) {  // KT is even
                 step(kt, std::integral_constant<int, 0>{});
@@ -526,39 +530,61 @@ __global__ __launch_bounds__(64 * NWAVE, 1) void qgemm_bf16_kernel(const uint16_
     }
 }
 
-// ---- the bf16 rows of a quantized weight (its device layout), 8 values per thread ----
+// ---- the bf16 rows of a quantized weight (its device layout), 32 values per thread ----
 __global__ __launch_bounds__(256) void weight_rows_bf16_kernel(GemmWeight w, uint16_t *__restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, k8 = w.k / 8;
-    if (i >= w.n * k8) return;
-    const int64_t n = i / k8;
-    const int k = (int)(i % k8) * 8;
-    float v[8];
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, k32 = w.k / 32;
+    if (i >= w.n * k32) return;
+    const int64_t n = i / k32;
+    const int k = (int)(i % k32) * 32;
+    // value = code * sc[half] + off, one rounding to f32; codes of the 32 values in 8 words
+    uint32_t c[8];
+    float sc[2], off = 0.f;
+    int bias = 0;  // subtracted from the code
     if (w.fmt == WF_Q8_0) {
-        const float d = f16_to_f32(w.scales[n * (w.k / 32) + k / 32]);
-        const int8_t *q = (const int8_t *)(w.q + n * w.k + k);
+        sc[0] = sc[1] = f16_to_f32(w.scales[n * k32 + k / 32]);
+        const u32x4 *q = (const u32x4 *)(w.q + n * w.k + k);
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = (float)q[e] * d;
+        for (int e = 0; e < 8; e++) c[e] = q[e >> 2][e & 3] ^ 0x80808080u;  // code + 128, unsigned
+        bias = 128;
     } else if (w.fmt == WF_Q4_K) {
         const uint8_t *b = q4k_block(w.q, n, k / 256, w.k / 256), *p = b + 4;
         const int j = (k & 255) / 32, jl = j & 3;
-        const int sc = j < 4 ? p[jl] & 63 : (p[8 + jl] & 15) | (p[jl] >> 6 << 4);
+        const int s = j < 4 ? p[jl] & 63 : (p[8 + jl] & 15) | (p[jl] >> 6 << 4);
         const int mn = j < 4 ? p[4 + jl] & 63 : (p[8 + jl] >> 4) | (p[4 + jl] >> 6 << 4);
-        const float ds = f16_to_f32(*(const uint16_t *)b) * (float)sc, dm = f16_to_f32(*(const uint16_t *)(b + 2)) * (float)mn;
-        const uint8_t *q = b + 16 + 32 * (j >> 1) + (k & 31);
+        sc[0] = sc[1] = f16_to_f32(*(const uint16_t *)b) * (float)s;
+        off = -(f16_to_f32(*(const uint16_t *)(b + 2)) * (float)mn);
+        const u32x4 *q = (const u32x4 *)(b + 16 + 32 * (j >> 1));
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = __builtin_fmaf(ds, (float)((j & 1) ? q[e] >> 4 : q[e] & 15), -dm);
+        for (int e = 0; e < 8; e++) c[e] = (q[e >> 2][e & 3] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
     } else {  // WF_Q6_K
         const uint8_t *b = q6k_block(w.q, n, k / 256, w.k / 256);
-        const int hh = (k & 255) / 128, r = (k & 127) / 32, l = k & 31;
-        const float ds = f16_to_f32(*(const uint16_t *)(b + 208)) * (float)(int8_t)b[192 + 8 * hh + (32 * r + l) / 16];
+        const int hh = (k & 255) / 128, r = (k & 127) / 32;
+        const float d = f16_to_f32(*(const uint16_t *)(b + 208));
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int ql = b[64 * hh + l + e + 32 * (r & 1)], qh = b[128 + 32 * hh + l + e];
-            v[e] = ds * (float)(((r < 2 ? ql & 15 : ql >> 4) | ((qh >> (2 * r)) & 3) << 4) - 32);
-        }
+        for (int h = 0; h < 2; h++) sc[h] = d * (float)(int8_t)b[192 + 8 * hh + 2 * r + h];
+        const u32x4 *ql = (const u32x4 *)(b + 64 * hh + 32 * (r & 1)), *qh = (const u32x4 *)(b + 128 + 32 * hh);
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            c[e] = ((ql[e >> 2][e & 3] >> (r < 2 ? 0 : 4)) & 0x0F0F0F0Fu) |
+                   (((qh[e >> 2][e & 3] >> (2 * r)) & 0x03030303u) << 4);
+        bias = 32;
     }
-    *(u32x4 *)(out + n * w.k + k) = u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
-                                          pack_bf16x2(v[6], v[7])};
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        uint32_t o[4];
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+            float v[2];
+#pragma unroll
+            for (int l = 0; l < 2; l++) {
+                const int at = 2 * h + l;  // byte of the word pair
+                const int code = (int)((c[e + (at >> 2)] >> (8 * (at & 3))) & 0xffu) - bias;
+                v[l] = __builtin_fmaf((float)code, sc[e >> 2], off);
+            }
+            o[h] = pack_bf16x2(v[0], v[1]);
+        }
+        *(u32x4 *)(out + n * w.k + k + 4 * e) = u32x4{o[0], o[1], o[2], o[3]};
+    }
 }
 
 template <int EPI>
@@ -634,7 +660,7 @@ double qgemm_bf16_q8k_us(const GemmWeight &w, int64_t m) {
 
 hipError_t launch_weight_rows_bf16(const GemmWeight &w, uint16_t *out, hipStream_t stream) {
     if (w.fmt == WF_BF16 || w.k % 32) return hipErrorInvalidValue;
-    const int64_t n = w.n * (w.k / 8);
+    const int64_t n = w.n * (w.k / 32);
     weight_rows_bf16_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream>>>(w, out);
     return hipGetLastError();
 }
