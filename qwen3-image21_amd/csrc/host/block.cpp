@@ -184,7 +184,7 @@ namespace {
 // rounding (candle mode only), and the split-K scratch of the short- and mid-M
 // GEMM paths, sized for the largest projection.
 struct WsLayout {
-    size_t modp, xn, q, k, vt, att, h, lim, f32, total, part;
+    size_t modp, xn, q, k, vt, att, h, lim, keys, f32, total, part;
 };
 
 // The activation block of candle's vec-dot type for weight w under the
@@ -217,6 +217,8 @@ WsLayout ws_layout(const qimm_block *blk, int64_t batch, int64_t seq, int64_t mo
     L.att = off; off += align_up((size_t)(M * hid) * 2);
     L.h = off; off += align_up((size_t)(M * F) * 2);
     L.lim = off; off += align_up((size_t)seq * 4);  // per-query key limits of the block-causal mask
+    L.keys = off;  // sums of the attention's split query tiles
+    off += align_up(qimm::attention_scratch_bytes(batch * blk->cfg.heads, seq));
     L.f32 = off;
     if (act_qblk(blk, blk->out) || act_qblk(blk, blk->down))
         off += align_up((size_t)(M * std::max(hid, F)) * 4);
@@ -337,14 +339,15 @@ int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t ba
     const int att_q = round_sep ? 0 : qb_out;
     float *att_f32 = qb_out ? stage_f32 : nullptr;
     const qimm::KeySeg own{kb, vt, seq, ep.vt_ld};
+    float *keys_f32 = qimm::attention_scratch_bytes(batch * H, seq) ? (float *)(ws + L.keys) : nullptr;
     // score bound: q and own k from the RmsNorm weights, prefix k from the cache
     const float *kpn = kv ? kv->knorm + layer : nullptr;
     if (img || kvalid)
         QIMM_HIP(ctx, qimm::launch_attention_masked(qb, prefix, own, batch, H, seq, 1.0f, img, kvalid, (int32_t *)(ws + L.lim), att, s, att_f32, kpn,
-                                                    blk->q_norm_bound, blk->k_norm_bound, att_q));
+                                                    blk->q_norm_bound, blk->k_norm_bound, att_q, keys_f32));
     else
         QIMM_HIP(ctx, qimm::launch_attention_log2(qb, prefix, own, batch, H, seq, att, s, att_f32, kpn,
-                                                  blk->q_norm_bound, blk->k_norm_bound, att_q));
+                                                  blk->q_norm_bound, blk->k_norm_bound, att_q, keys_f32));
     if (kv) {
         const int rc = kv_release(kv, layer, s);
         if (rc) return rc;

@@ -30,6 +30,11 @@
 // chunks to the segment and clears the V^T columns past its end. V^T rows of 16 B
 // aligned stride (KeySeg::ld) are copied straight into LDS; rows of any other
 // stride go through registers (RV).
+// Against a register-staged kernel of 4 waves with per-element bounds, which took
+// every length that was no multiple of 8 before (kernel times): 6889 queries over
+// 131 + 6889 keys, 32 heads 3.04 -> 0.95 ms, 4299 tokens under the block-causal
+// mask 2.27 -> 0.66 ms, without the key split below.
+#include <algorithm>
 #include <type_traits>
 
 #include "device_common.h"
@@ -63,6 +68,16 @@ struct ScoreBound {
     float q_norm, k_own;
 };
 constexpr float STATIC_MAX = 64.0f;
+
+// The last, partial round of query tiles over the CUs, split over the keys: tiles
+// `full` .. in dispatch order are `parts` workgroups each. Part `slot` (counted
+// from `full`) leaves its unnormalized output o[slot][256][128] and, per query,
+// its reference point and row sum ml[slot][256][2].
+struct KeySplit {
+    int64_t full;
+    int parts;
+    float *o, *ml;
+};
 
 // v_permlane32_swap exchanges the upper 32 lanes of its first operand with
 // the lower 32 lanes of its second; with both operands holding x, each lane
@@ -263,13 +278,16 @@ constexpr float RESCALE_TH = 8.0f;    // log2 units
 // RV: V^T rows whose stride is not a multiple of 16 B (a caller's dense V^T of
 // an odd length) cannot be copied 16 B at a time into LDS: their chunks are
 // loaded unaligned into registers one block ahead and written to the same slots.
-template <int NW, bool PRE, bool MASKED, int SMODE, bool PAIR, bool RV>
+// SPLIT: the workgroups from KeySplit::full on are parts of tiles: each takes a
+// share of its tile's key blocks and leaves its sums (KeySplit) for attn_merge_kernel.
+template <int NW, bool PRE, bool MASKED, int SMODE, bool PAIR, bool RV, bool SPLIT>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16_t *__restrict__ q, Seg s0, Seg s1,
                                                                     int64_t H, int64_t Sq, int64_t nq, int64_t B,
                                                                     float sl2, uint16_t *__restrict__ out,
                                                                     float *__restrict__ outf, KeyMask km,
                                                                     const int32_t *__restrict__ lim,
-                                                                    ScoreBound sb, int q8) {
+                                                                    ScoreBound sb, int q8, KeySplit sp) {
+    static_assert(!SPLIT || (NW == 8 && PRE && !PAIR && !RV), "the split form is the block's 8-wave one");
     static_assert(NW == 4 || NW == 8, "4 or 8 waves");
     static_assert(!PAIR || !MASKED, "the paired form is the cached step's");
     constexpr int QB = 32 * NW;  // queries per workgroup
@@ -292,6 +310,15 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
     const int64_t HP = PAIR ? H / 2 : H;
     const int64_t total = nq * HP * B;
     int64_t L = blockIdx.x;
+    int part = 0, parts = 1;
+    int64_t slot = 0;  // of the part's sums
+    if constexpr (SPLIT)
+        if (L >= sp.full) {
+            slot = L - sp.full;
+            L = sp.full + slot / sp.parts;
+            part = (int)(slot % sp.parts);
+            parts = sp.parts;
+        }
     int64_t qt, bhp;
     if (MASKED && lim) {
         qt = nq - 1 - L / (HP * B);
@@ -357,6 +384,11 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
                 for (int i = 1; i < NW; i++) kmax = max(kmax, wlim[i]);
                 nblk = min(nblk, (kmax + KB - 1) / KB);
             }
+        }
+        int j0 = 0;  // the first key block; the last is nblk - 1
+        if constexpr (SPLIT) {
+            j0 = nblk * part / parts;
+            nblk = nblk * (part + 1) / parts;
         }
         const char *kb0 = (const char *)(s0.k + bh * (int64_t)len0 * HD);
         const char *kb1 = (const char *)(s1.k + bh * (int64_t)len1 * HD);
@@ -713,13 +745,13 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             __syncthreads();
         };
 
-        if (nblk > 0) {
-            if constexpr (MASKED) mask_load(blk_of(0));
-            dma(blk_of(0), 0);
+        if (nblk > j0) {
+            if constexpr (MASKED) mask_load(blk_of(j0));
+            dma(blk_of(j0), 0);
         }
         __builtin_amdgcn_s_waitcnt(WAIT_VM0);
         if constexpr (RV)
-            if (nblk > 0) seal(blk_of(0), 0);
+            if (nblk > j0) seal(blk_of(j0), 0);
         __syncthreads();
         // the fixed-reference form when the score bound allows it (wave-uniform)
         bool stat_ok = false;
@@ -728,7 +760,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             stat_ok = sb.q_norm * kn <= STATIC_MAX;
         }
         auto run = [&](auto stat) __attribute__((always_inline)) {
-            int j = 0;
+            int j = j0;
             for (; j + 1 < nblk; j += 2) {
                 step(j, 0, stat);
                 step(j + 1, 1, stat);
@@ -748,6 +780,17 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
 
         // normalize and stage O [32 q x 128 d] per wave through LDS for row stores
         const float l_tot = xsum32(l_run);
+        if constexpr (SPLIT)
+            if (parts > 1) {
+                if (g == 0) {
+                    float *ml = sp.ml + (slot * QB + wave * 32 + l32) * 2;
+                    ml[0] = m_run;
+                    ml[1] = l_tot;
+                }
+                store_out_f32<OPF>((float *)lds + wave * 32 * OPF, o, 1.0f, lane, sp.o + slot * QB * HD, 0, QB, HD, 0,
+                                   wave * 32);
+                return;
+            }
         const float inv = 1.0f / l_tot;
         const int64_t HDt = H * HD;
         uint16_t *os = (uint16_t *)lds + wave * 32 * OP;
@@ -820,16 +863,68 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
     if constexpr (PAIR) head(std::integral_constant<int, 1>{});
 }
 
+// Sums the parts of split tile blockIdx.x / 32 (in part order; relative to the
+// largest reference point), normalizes and stores as attn_fast_kernel does: one
+// query per 32 lanes, 4 d per lane, eight queries per workgroup.
+__global__ __launch_bounds__(256) void attn_merge_kernel(KeySplit sp, int64_t nq, int64_t H, int64_t B, int64_t Sq,
+                                                         int by_limit, uint16_t *__restrict__ out,
+                                                         float *__restrict__ outf, int q8) {
+    const int64_t r = blockIdx.x >> 5, total = nq * H * B;
+    const int ql = (int)(blockIdx.x & 31) * 8 + (threadIdx.x >> 5), d = (threadIdx.x & 31) * 4;
+    int64_t L = sp.full + r, qt, bh;  // the tile, as attn_fast_kernel maps it
+    if (by_limit) {
+        qt = nq - 1 - L / (H * B);
+        bh = L % (H * B);
+    } else {
+        if ((total & 7) == 0) L = (L & 7) * (total >> 3) + (L >> 3);
+        qt = L % nq;
+        bh = L / nq;
+    }
+    const int64_t qi = qt * 256 + ql;
+    if (qi >= Sq) return;
+    const float *ml = sp.ml + (r * sp.parts * 256 + ql) * 2, *o = sp.o + (r * sp.parts * 256 + ql) * HD + d;
+    float m = -INFINITY;
+    for (int p = 0; p < sp.parts; p++)  // a part without a visible key has no reference point
+        if (ml[p * 512 + 1] > 0.f) m = fmaxf(m, ml[p * 512]);
+    f32x4 acc{0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+    for (int p = 0; p < sp.parts; p++) {
+        const float lp = ml[p * 512 + 1], a = lp > 0.f ? __builtin_amdgcn_exp2f(ml[p * 512] - m) : lp;
+        l += a * lp;
+        const f32x4 v = *(const f32x4 *)(o + (int64_t)p * 256 * HD);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[e] += a * v[e];
+    }
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc[e] *= inv;
+    const int64_t at = ((bh / H) * Sq + qi) * (H * HD) + (bh % H) * HD + d;
+    if (outf)
+        *(f32x4 *)(outf + at) = acc;
+    else if (q8)
+        *(u32x2 *)(out + at) = quant_act4<32>(acc);
+    else
+        *(u32x2 *)(out + at) = u32x2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
+}
+
 }  // namespace fast
 
-template <int NW, bool PRE, bool MASKED, int SMODE = 0, bool PAIR = false, bool RV = false>
+template <int NW, bool PRE, bool MASKED, int SMODE = 0, bool PAIR = false, bool RV = false, bool SPLIT = false>
 void launch_fast(const uint16_t *q, Seg s0, Seg s1, int64_t h, int64_t sq, int64_t b, float sl2, uint16_t *out,
                  float *outf, const KeyMask &km, const int32_t *lim, const ScoreBound &sb, int q8,
-                 hipStream_t stream) {
+                 hipStream_t stream, KeySplit sp = KeySplit{0, 1, nullptr, nullptr}) {
+    if constexpr (!SPLIT && NW == 8 && PRE && !PAIR && !RV)
+        if (sp.parts > 1)
+            return launch_fast<NW, PRE, MASKED, SMODE, PAIR, RV, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, q8,
+                                                                       stream, sp);
     const int64_t nq = (sq + 32 * NW - 1) / (32 * NW);
-    fast::attn_fast_kernel<NW, PRE, MASKED, SMODE, PAIR, RV>
-        <<<dim3((unsigned)(nq * (PAIR ? h / 2 : h) * b)), dim3(64 * NW), 0, stream>>>(q, s0, s1, h, sq, nq, b, sl2,
-                                                                                       out, outf, km, lim, sb, q8);
+    const int64_t tiles = nq * (PAIR ? h / 2 : h) * b, rest = SPLIT ? tiles - sp.full : 0;
+    fast::attn_fast_kernel<NW, PRE, MASKED, SMODE, PAIR, RV, SPLIT>
+        <<<dim3((unsigned)(tiles + rest * (sp.parts - 1))), dim3(64 * NW), 0, stream>>>(q, s0, s1, h, sq, nq, b, sl2, out,
+                                                                                        outf, km, lim, sb, q8, sp);
+    if constexpr (SPLIT)
+        fast::attn_merge_kernel<<<dim3((unsigned)(rest * 32)), dim3(256), 0, stream>>>(sp, nq, h, b, sq, MASKED && lim ? 1 : 0,
+                                                                                      out, outf, q8);
 }
 
 // The masked kernel with the softmax form decided on the host where the score
@@ -837,15 +932,15 @@ void launch_fast(const uint16_t *q, Seg s0, Seg s1, int64_t h, int64_t sq, int64
 template <bool PRE>
 void launch_masked(const uint16_t *q, Seg s0, Seg s1, int64_t h, int64_t sq, int64_t b, float sl2, uint16_t *out,
                    float *outf, const KeyMask &km, const int32_t *lim, const ScoreBound &sb, int q8,
-                   hipStream_t stream) {
+                   hipStream_t stream, const KeySplit &sp) {
     if (sb.q_norm <= 0.f)
-        launch_fast<8, PRE, true, 2>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, q8, stream);
+        launch_fast<8, PRE, true, 2>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, q8, stream, sp);
     else if (sb.k_prefix)
-        launch_fast<8, PRE, true, 0>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, q8, stream);
+        launch_fast<8, PRE, true, 0>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, q8, stream, sp);
     else if (sb.q_norm * sb.k_own <= STATIC_MAX)
-        launch_fast<8, PRE, true, 1>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, q8, stream);
+        launch_fast<8, PRE, true, 1>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, q8, stream, sp);
     else
-        launch_fast<8, PRE, true, 2>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, q8, stream);
+        launch_fast<8, PRE, true, 2>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, q8, stream, sp);
 }
 
 // Waves per workgroup of the unmasked fast kernel, from the rounds each form
@@ -863,6 +958,41 @@ int fast_waves(int64_t bh, int64_t sq) {
     const int64_t r4 = n4 % (2 * cus);
     const int64_t c4 = 105 * (n4 / (2 * cus)) + (r4 == 0 ? 0 : r4 <= cus ? 84 : 105);
     return c4 < c8 ? 4 : 8;
+}
+
+// Parts per tile of the last, partial round of 8-wave tiles (the others run
+// whole), 1 = not split, by an estimate in us: a tile takes 2.15 us per key block
+// (2.7 masked) and about 8 beside them, a part its share and the 8; the parts'
+// sums are written and read once (131 KB each at 4 TB/s) by one launch more.
+// Never more than two parts per CU: 68 MB of sums. `now` is the estimate without it.
+// Measured at 32 heads, kernel and merge: 4299 masked tokens (544 tiles for 256
+// CUs, the last 32 in 8 parts) 661 -> 385 us, 6889 queries over 7020 keys (864
+// tiles, the last 96 in 2) 953 -> 793, 3072 over 3289 (384, the last 128 in 2;
+// 4-wave tiles before) 236 -> 200.
+constexpr int MAX_PARTS = 8;
+int split_parts(int64_t bh, int64_t sq, int64_t keys, bool masked, double now, double more) {
+    const int64_t cus = device_cu_count(), tiles = (sq + 255) / 256 * bh;
+    if (cus <= 0 || tiles % cus == 0) return 1;
+    const int64_t rest = tiles % cus;
+    const double loop = (masked ? 2.7 : 2.15) * (double)((keys + 63) / 64);
+    int best = 1;
+    double best_us = 0.97 * now;
+    for (int s = 2; s <= MAX_PARTS && rest * s <= 2 * cus; s++) {
+        const double us = (double)(tiles / cus) * (loop + 8.0) + (double)((rest * s + cus - 1) / cus) * (loop / s + 8.0) + 6.0 +
+                          (double)(rest * s) * 0.131 * 2.0 / 4.0 + more;
+        if (us < best_us) {
+            best_us = us;
+            best = s;
+        }
+    }
+    return best;
+}
+double tile_rounds_us(int64_t bh, int64_t sq, int64_t keys, bool masked, double rounds) {
+    return rounds * ((masked ? 2.7 : 2.15) * (double)((keys + 63) / 64) + 8.0);
+}
+KeySplit key_split(int64_t bh, int64_t sq, int parts, float *scratch) {
+    const int64_t cus = device_cu_count(), tiles = (sq + 255) / 256 * bh, rest = tiles % cus;
+    return KeySplit{tiles - rest, parts, scratch, scratch + rest * parts * 256 * 128};
 }
 
 // sl2 = softmax scale * log2(e) applied to raw scores, or 1 when q already
@@ -898,7 +1028,8 @@ bool rows16(const Seg &s) { return s.len == 0 || s.ld % 8 == 0; }
 
 template <bool PRE>
 hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq, float sl2,
-                  uint16_t *out, float *outf, const ScoreBound &sb, int out_qblk, hipStream_t stream) {
+                  uint16_t *out, float *outf, const ScoreBound &sb, int out_qblk, hipStream_t stream,
+                  float *scratch = nullptr) {
     if (sq <= 0 || b <= 0 || h <= 0) return hipSuccess;
     Seg s0, s1;
     if (!segments(prefix, own, s0, s1) || !out_qblk_ok(out_qblk, outf)) return hipErrorInvalidValue;
@@ -908,6 +1039,23 @@ hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64
     const KeyMask km{nullptr, nullptr, prefix.len + own.len};
     const int nw = fast_waves(b * h, sq);
     constexpr int SM = PRE ? 0 : 2;  // without the block's norms no score bound is known
+    if constexpr (PRE)
+        if (scratch && rows16(s0) && rows16(s1)) {
+            const int64_t cus = std::max(device_cu_count(), 1), keys = prefix.len + own.len, n8 = (sq + 255) / 256 * b * h;
+            const bool pair = out_qblk == 256 && nw == 8 && h % 2 == 0;
+            const int64_t n4 = (sq + 127) / 128 * b * h, r4 = n4 % (2 * cus);
+            const double rounds = pair ? 2.0 * (double)((n8 / 2 + cus - 1) / cus)
+                                  : nw == 8 ? (double)((n8 + cus - 1) / cus)
+                                            : 1.05 * (double)(n4 / (2 * cus)) + (r4 == 0 ? 0.0 : r4 <= cus ? 0.84 : 1.05);
+            // the paired kernel rounds in its epilogue, the split one in a pass over f32 rows
+            const double more = pair ? 5.0 + (double)(b * sq * h) * 128.0 * 6.0 / 4.5e6 : 0.0;
+            if (const int parts = split_parts(b * h, sq, keys, false, tile_rounds_us(b * h, sq, keys, false, rounds), more);
+                parts > 1) {
+                launch_fast<8, true, false>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream,
+                                            key_split(b * h, sq, parts, scratch));
+                return finish_q8k(out_qblk, false, outf, b, h, sq, out, stream);
+            }
+        }
     if (!rows16(s0) || !rows16(s1)) {
         if (nw == 4)
             launch_fast<4, false, false, 2, false, true>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
@@ -926,6 +1074,13 @@ hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64
 
 }  // namespace
 
+size_t attention_scratch_bytes(int64_t bh, int64_t sq) {
+    const int64_t cus = device_cu_count(), tiles = (sq + 255) / 256 * bh;
+    if (cus <= 0 || tiles % cus == 0) return 0;
+    const int64_t rest = tiles % cus, parts = std::min<int64_t>(MAX_PARTS, 2 * cus / rest);
+    return parts > 1 ? (size_t)(rest * parts) * 256 * (128 + 2) * 4 : 0;
+}
+
 hipError_t launch_attention(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
                             float scale, uint16_t *out, hipStream_t stream, float *outf) {
     return launch<false>(q, prefix, own, b, h, sq, scale * 1.4426950408889634f, out, outf,
@@ -935,7 +1090,7 @@ hipError_t launch_attention(const uint16_t *q, KeySeg prefix, KeySeg own, int64_
 hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
                                    float sl2, const int32_t *img, const uint8_t *kvalid, int32_t *lim_scratch,
                                    uint16_t *out, hipStream_t stream, float *outf, const float *k_prefix_norm,
-                                   float q_norm, float k_own_norm, int out_qblk) {
+                                   float q_norm, float k_own_norm, int out_qblk, float *scratch) {
     if (sq <= 0 || b <= 0 || h <= 0) return hipSuccess;
     Seg s0, s1;
     if (!segments(prefix, own, s0, s1) || !out_qblk_ok(out_qblk, outf)) return hipErrorInvalidValue;
@@ -955,18 +1110,26 @@ hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own,
     const ScoreBound sb{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm * sl2, k_own_norm};
     if (!rows16(s0) || !rows16(s1))
         launch_fast<8, false, true, 2, false, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream);
-    else if (sl2 == 1.0f)  // q already carries the scale (the block's q/k/v epilogue)
-        launch_masked<true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream);
-    else
-        launch_masked<false>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream);
+    else if (sl2 == 1.0f) {  // q already carries the scale (the block's q/k/v epilogue)
+        KeySplit sp{0, 1, nullptr, nullptr};
+        if (scratch) {
+            const int64_t cus = std::max(device_cu_count(), 1), n8 = (sq + 255) / 256 * b * h;
+            const double now = tile_rounds_us(b * h, sq, km.kv_len, true, (double)((n8 + cus - 1) / cus));
+            if (const int parts = split_parts(b * h, sq, km.kv_len, true, now, 0.0); parts > 1)
+                sp = key_split(b * h, sq, parts, scratch);
+        }
+        launch_masked<true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream, sp);
+    } else
+        launch_masked<false>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream,
+                             KeySplit{0, 1, nullptr, nullptr});
     return finish_q8k(out_qblk, false, outf, b, h, sq, out, stream);
 }
 
 hipError_t launch_attention_log2(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
                                  uint16_t *out, hipStream_t stream, float *outf, const float *k_prefix_norm,
-                                 float q_norm, float k_own_norm, int out_qblk) {
+                                 float q_norm, float k_own_norm, int out_qblk, float *scratch) {
     return launch<true>(q, prefix, own, b, h, sq, 1.0f, out, outf,
-                        ScoreBound{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm, k_own_norm}, out_qblk, stream);
+                        ScoreBound{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm, k_own_norm}, out_qblk, stream, scratch);
 }
 
 }  // namespace qimm

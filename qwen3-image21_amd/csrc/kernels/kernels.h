@@ -211,13 +211,16 @@ hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own,
                                    float sl2, const int32_t *img, const uint8_t *kvalid, int32_t *lim_scratch,
                                    uint16_t *out, hipStream_t stream, float *outf = nullptr,
                                    const float *k_prefix_norm = nullptr, float q_norm = 0.f, float k_own_norm = 0.f,
-                                   int out_qblk = 0);
+                                   int out_qblk = 0, float *scratch = nullptr);
 // The same with q already multiplied by scale * log2(e) (the QKV epilogue's
 // q_scale), so scores are in log2 units.
 hipError_t launch_attention_log2(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
                                  uint16_t *out, hipStream_t stream, float *outf = nullptr,
                                  const float *k_prefix_norm = nullptr, float q_norm = 0.f, float k_own_norm = 0.f,
-                                 int out_qblk = 0);
+                                 int out_qblk = 0, float *scratch = nullptr);
+// scratch (attention_scratch_bytes, may be null) lets both launches split the
+// last, partial round of query tiles over the keys.
+size_t attention_scratch_bytes(int64_t bh, int64_t sq);
 // Score bound of the fast kernels (both launches above): with q_norm >= every
 // query's norm (as passed, before sl2), k_own_norm >= every own key's norm and,
 // when there is a prefix, *k_prefix_norm (device) >= every prefix key's norm,

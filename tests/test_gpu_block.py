@@ -177,6 +177,46 @@ def test_block_large_norm_weights_running_max_path(torch_cuda, qctx):
         check_modes(SMALL, w, x, mod, pe, kpre, vpre, runs, want_kv=True)
 
 
+@pytest.mark.parametrize("s,p,norm", [(700, 65, 1.0), (700, 65, 3.0), (257, 260, 3.0), (1100, 0, 1.0)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_block_attention_split_over_keys(torch_cuda, qctx, s, p, norm, padded):
+    """Few query tiles: the attention splits their keys over workgroups and merges the
+    parts' sums, against the fixed reference (norm weights 1) and relative to each
+    part's own maximum (3: beyond its bound), and, padded, with whole 64-key windows
+    of a part masked; both activation modes against the oracle."""
+    w, x, mod, pe, kpre, vpre = make_case(17 + s + p, SMALL, 1, s, p, synth.Q8_0, synth.Q8_0)
+    rng = np.random.default_rng(s + p)
+    for n in ("norm_q", "norm_k"):
+        w[n] = (norm * (1 + 0.1 * rng.standard_normal(128))).astype(np.float32)
+    if not padded:
+        check_modes(SMALL, w, x, mod, pe, kpre, vpre, run_modes(torch_cuda, qctx, SMALL, w, x, mod, pe, kpre, vpre, want_kv=True),
+                    want_kv=True)
+        return
+    torch = torch_cuda
+    valid = np.ones((1, p + s), dtype=np.uint8)
+    valid[0, 5:min(200, p + s // 2)] = 0
+    outs = []
+    for act in (qimm.ACT_CANDLE, qimm.ACT_BF16):
+        keep = []
+        blk = qctx.block_create(qimm.BlockConfig(256, 2, 128, 768), block_tensors(w, keep))
+        blk.set_act_mode(act)
+        xd, md, pd, vd = dev(torch, x), dev(torch, mod), dev(torch, pe), dev(torch, valid)
+        out, kv = torch.empty_like(xd), None
+        if p:
+            kv = qctx.kv_create(1, 1, 2, p)
+            kd, vvd = dev(torch, kpre.view(np.int16)), dev(torch, vpre.view(np.int16))
+            kv.store(0, kd.data_ptr(), vvd.data_ptr(), stream(torch))
+        blk.forward_masked(xd.data_ptr(), out.data_ptr(), 1, s, md.data_ptr(), 1, pd.data_ptr(), None, vd.data_ptr(), kv, 0,
+                           stream=stream(torch))
+        outs.append(host(out))
+        blk.free()
+        if kv:
+            kv.free()
+    mask = np.broadcast_to(valid[:, None, :], (1, s, p + s))
+    refs = [O.block_forward(SMALL, w, x, mod, pe, kpre, vpre, mask=mask, mode=m)[0] for m in (O.CANDLE, O.EXACT)]
+    check_block(*(a.reshape(-1, 256) for a in (outs[0], outs[1], refs[0], refs[1], x)))
+
+
 def test_block_deterministic(torch_cuda, qctx):
     w, x, mod, pe, kpre, vpre = make_case(9, SMALL, 1, 96, 32, synth.Q4_K, synth.Q6_K)
     a, _ = run_block(torch_cuda, qctx, SMALL, w, x, mod, pe, kpre, vpre)
