@@ -233,10 +233,12 @@ WsLayout ws_layout(const qimm_block *blk, int64_t batch, int64_t seq, int64_t mo
 // TransformerBlock::forward (src/quantized_transformer.rs:258-285) with
 // modulation rows [B, mod_rows, 4 hidden] (mod_rows 1 broadcasts over the
 // tokens, mod_rows == seq gives one row per token) and an optional attention
-// mask; kv supplies the prefix K/V of the cached step.
+// mask; kv supplies the prefix K/V of the cached step. k_out [B,H,S,128] / v_out
+// receive the own keys and values; vt_out [B,H,128,vt_ld(S)] takes the place of
+// the workspace's transposed values.
 int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t batch, int64_t seq, const float *mod,
                        int64_t mod_rows, const float *pe, const qimm_attn_mask *mask, const qimm_kv *kv,
-                       int64_t layer, uint16_t *k_out, uint16_t *v_out, void *stream) {
+                       int64_t layer, uint16_t *k_out, uint16_t *v_out, void *stream, uint16_t *vt_out = nullptr) {
     if (!blk || !x || !x_out || !mod || !pe) return QIMM_ERR_ARG;
     qimm_ctx *ctx = blk->ctx;
     const int64_t hid = blk->cfg.hidden, H = blk->cfg.heads, F = blk->cfg.mlp;
@@ -267,7 +269,7 @@ int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t ba
     float *modp = (float *)(ws + L.modp);
     uint16_t *xn = (uint16_t *)(ws + L.xn), *qb = (uint16_t *)(ws + L.q);
     uint16_t *kb = k_out ? k_out : (uint16_t *)(ws + L.k);
-    uint16_t *vt = (uint16_t *)(ws + L.vt), *att = (uint16_t *)(ws + L.att), *hm = (uint16_t *)(ws + L.h);
+    uint16_t *vt = vt_out ? vt_out : (uint16_t *)(ws + L.vt), *att = (uint16_t *)(ws + L.att), *hm = (uint16_t *)(ws + L.h);
     const size_t part_need = L.part;
     if (part_need) {
         rc = ensure_part_workspace(ctx, part_need);
@@ -405,6 +407,15 @@ int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t ba
 }
 
 }  // namespace
+
+namespace qimm_host {
+
+int block_prefix_forward(qimm_block *blk, float *x, int64_t batch, int64_t seq, const float *mod, const float *pe,
+                         const qimm_attn_mask *mask, uint16_t *k, uint16_t *vt, void *stream) {
+    return block_forward_impl(blk, x, x, batch, seq, mod, 1, pe, mask, nullptr, 0, k, nullptr, stream, vt);
+}
+
+}  // namespace qimm_host
 
 extern "C" {
 

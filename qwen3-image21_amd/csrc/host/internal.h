@@ -99,6 +99,11 @@ int block_values(int type);
 int kv_layer(const qimm_kv *kv, int64_t layer, hipStream_t s, qimm::KeySeg *seg);
 int kv_release(const qimm_kv *kv, int64_t layer, hipStream_t s);
 
+// One block of the prefix fill, in place on x: its keys and transposed values go
+// straight to a cache layer's k and vt (internal layout).
+int block_prefix_forward(qimm_block *blk, float *x, int64_t batch, int64_t seq, const float *mod, const float *pe,
+                         const qimm_attn_mask *mask, uint16_t *k, uint16_t *vt, void *stream);
+
 }  // namespace qimm_host
 
 #define QIMM_HIP(ctx, call)                                         \

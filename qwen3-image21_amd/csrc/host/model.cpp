@@ -237,14 +237,18 @@ int qimm_model_prefix_fill(qimm_model *m, const float *txt, int64_t text_len, co
     hipStream_t s = (hipStream_t)stream;
     QIMM_HIP(ctx, hipSetDevice(ctx->device));
     const int64_t H = kv->heads, trows = batch * text_len, crows = batch * cond_len;
+    // a device cache of the model's heads takes each block's keys and transposed
+    // values as the block writes them; other caches are stored from [B,H,P,128] copies
+    const bool direct = !kv->host && H * 128 == hid;
     const size_t need = (size_t)(trows * (tw + 2 * hid) + crows * hid + batch * P * hid) * 4 +
-                        (size_t)(2 * batch * H * P * 128) * 2 + (size_t)batch * (kTimeDim + 6 * hid) * 4 + 16 * 256;
+                        (direct ? 0 : (size_t)(2 * batch * H * P * 128) * 2) + (size_t)batch * (kTimeDim + 6 * hid) * 4 + 16 * 256;
     int rc = ensure_ws(m, need);
     if (rc) return rc;
     Carver c{(char *)m->ws};
     float *tn = c.take<float>(trows * tw), *tmid = c.take<float>(trows * hid), *tx = c.take<float>(trows * hid);
     float *cx = c.take<float>(crows * hid), *x = c.take<float>(batch * P * hid);
-    uint16_t *kl = c.take<uint16_t>(batch * H * P * 128), *vl = c.take<uint16_t>(batch * H * P * 128);
+    uint16_t *kl = direct ? nullptr : c.take<uint16_t>(batch * H * P * 128);
+    uint16_t *vl = direct ? nullptr : c.take<uint16_t>(batch * H * P * 128);
     float *tsin = c.take<float>(batch * kTimeDim), *tmp = c.take<float>(batch * hid), *temb = c.take<float>(batch * hid);
     float *modv = c.take<float>(batch * 4 * hid);
     // txt_in: text_norm -> in_layer -> GELU(tanh) -> out_layer (:56-81)
@@ -277,9 +281,24 @@ int qimm_model_prefix_fill(qimm_model *m, const float *txt, int64_t text_len, co
     QIMM_HIP(ctx, qimm::launch_linear_f32(temb, hid, m->mod, batch, 4 * hid, hid, qimm::ACT_NONE, modv, 4 * hid, s));
     // every block under the block-causal mask, keeping its k, v (:383-391)
     qimm_attn_mask mask{image_ids, key_valid};
+    const qimm_attn_mask *mk = image_ids || key_valid ? &mask : nullptr;
+    if (direct) {
+        // the layers' score bounds: none while they are rewritten, then each block's
+        // bound on its normed keys (what its own step tests beside the cache's)
+        std::vector<float> bound((size_t)m->cfg.layers, INFINITY);
+        QIMM_HIP(ctx, qimm::launch_set_floats(kv->knorm, bound.data(), m->cfg.layers, s));
+        for (int64_t i = 0; i < m->cfg.layers; i++) {
+            qimm_block *blk = m->blocks[(size_t)i];
+            rc = block_prefix_forward(blk, x, batch, P, modv, pe, mk, kv->k + i * kv->layer_elems(),
+                                      kv->vt + i * kv->vt_elems(), stream);
+            if (rc) return rc;
+            if (blk->k_norm_bound < INFINITY) bound[(size_t)i] = blk->k_norm_bound;
+        }
+        QIMM_HIP(ctx, qimm::launch_set_floats(kv->knorm, bound.data(), m->cfg.layers, s));
+        return QIMM_OK;
+    }
     for (int64_t i = 0; i < m->cfg.layers; i++) {
-        rc = qimm_block_forward_masked(m->blocks[(size_t)i], x, x, batch, P, modv, 1, pe, image_ids || key_valid ? &mask : nullptr,
-                                       nullptr, 0, kl, vl, stream);
+        rc = qimm_block_forward_masked(m->blocks[(size_t)i], x, x, batch, P, modv, 1, pe, mk, nullptr, 0, kl, vl, stream);
         if (rc) return rc;
         if ((rc = qimm_kv_store_layer(kv, i, kl, vl, stream))) return rc;
     }

@@ -250,6 +250,8 @@ hipError_t launch_linear_f32(const float *x, int64_t ldx, const float *w, int64_
                              int act_out, float *y, int64_t ldy, hipStream_t stream);
 // out[rows][width] = 1 in each row's first half, 0 in its second (the t = 0 timestep embedding)
 hipError_t launch_zero_sinusoid(float *out, int64_t rows, int64_t width, hipStream_t stream);
+// dst[i] = values[i] (host values, passed by value: capturable, no host memory read later)
+hipError_t launch_set_floats(float *dst, const float *values, int64_t n, hipStream_t stream);
 // y = x / sqrt(mean(x^2) + eps) * w, per row of d values
 hipError_t launch_rows_rmsnorm(const float *x, const float *w, int64_t rows, int64_t d, float eps, float *y,
                                hipStream_t stream);

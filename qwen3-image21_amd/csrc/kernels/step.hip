@@ -15,6 +15,8 @@
 //   more rows (img_in, proj_out, txt_in): f32 matrix instructions over tiles
 //     whose k range the workgroup's waves share (linear_mfma_kernel);
 //   widths or addresses that do not allow 16 B loads: linear_any_kernel.
+#include <algorithm>
+
 #include "device_common.h"
 #include "kernels.h"
 
@@ -326,6 +328,13 @@ __global__ void zero_sinusoid_kernel(float *__restrict__ out, int64_t n, int wid
     if (i < n) out[i] = (int)(i % width) < width / 2 ? 1.0f : 0.0f;
 }
 
+struct Floats {
+    float v[256];
+};
+__global__ void set_floats_kernel(float *__restrict__ dst, Floats f, int n) {
+    if ((int)threadIdx.x < n) dst[threadIdx.x] = f.v[threadIdx.x];
+}
+
 unsigned grid1(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
@@ -358,6 +367,16 @@ hipError_t launch_linear_f32(const float *x, int64_t ldx, const float *w, int64_
     }
     const dim3 grid(blocks(n, LT), blocks(m, LT));
     linear_any_kernel<<<grid, dim3(256), 0, stream>>>(x, ldx, w, m, n, k, act_out, y, ldy);
+    return hipGetLastError();
+}
+
+hipError_t launch_set_floats(float *dst, const float *values, int64_t n, hipStream_t stream) {
+    for (int64_t at = 0; at < n; at += 256) {
+        Floats f{};
+        const int len = (int)std::min<int64_t>(256, n - at);
+        std::copy(values + at, values + at + len, f.v);
+        set_floats_kernel<<<dim3(1), dim3(256), 0, stream>>>(dst + at, f, len);
+    }
     return hipGetLastError();
 }
 

@@ -195,6 +195,38 @@ def test_prefix_fill_matches_oracle(torch_cuda, qctx):
     mdl.free()
 
 
+@pytest.mark.parametrize("text,b", [(21, 2), (77, 1), (603, 1)])
+def test_prefix_fill_into_the_cache_equals_the_stored_copy(torch_cuda, qctx, text, b):
+    """A device cache takes a fill's keys and values as the blocks write them, a host
+    cache from [B,H,P,128] copies: the same bits on both, at token counts that leave
+    row padding, and the same cached step over them."""
+    torch = torch_cuda
+    layers, rng = 2, np.random.default_rng(text)
+    g, blocks = model_weights(51, layers)
+    mdl = Built(qctx, g, blocks)
+    txt_d = dev(torch, rng.standard_normal((b, text, JD)).astype(np.float32))
+    pe = O.rope_table([(1, 4, 8)], [0] * text + [1] * 32)
+    pe_d, step_pe = dev(torch, pe[:text]), dev(torch, np.ascontiguousarray(pe[text:]))
+    ids_d = dev(torch, np.full(text, -1, np.int32))
+    lat, tsd = dev(torch, rng.standard_normal((b, 32, CH)).astype(np.float32)), t_sin_dev(torch, qctx, [0.4] * b)
+    got = []
+    for make in (qctx.kv_create, qctx.kv_create_host):
+        kv = make(layers, b, SMALL["heads"], text)
+        mdl.model.prefix_fill(txt_d.data_ptr(), text, None, 0, b, qimm.joint_layout_pieces(text), ids_d.data_ptr(), None,
+                              pe_d.data_ptr(), kv, stream(torch))
+        out = []
+        for i in range(layers):
+            k, v = (torch.empty((b, SMALL["heads"], text, 128), dtype=torch.int16, device="cuda") for _ in range(2))
+            kv.load(i, k.data_ptr(), v.data_ptr(), stream(torch))
+            out += [host(k), host(v)]
+        pred = torch.empty_like(lat)
+        mdl.model.forward(lat.data_ptr(), b, 32, tsd.data_ptr(), step_pe.data_ptr(), kv, pred.data_ptr(), stream=stream(torch))
+        got.append(out + [host(pred)])
+        kv.free()
+    assert all(np.array_equal(x, y) for x, y in zip(*got)) and np.isfinite(got[0][-1]).all()
+    mdl.free()
+
+
 def test_sampling_loop_with_cfg(torch_cuda, qctx):
     """Three steps of the T2I loop (src/pipeline.rs:168-193): prefix fill for the
     prompt and the negative prompt, then per step the cached forward twice, the
