@@ -619,8 +619,9 @@ bool qgemm_bf16_fits(const GemmWeight &w) {
 // 128-token tiles, 250 mixed 10 + 4); or, where the 128-token tiles leave CUs
 // without one, those tiles split over K (shares of at least 8 steps, at most one
 // workgroup per CU, so the partial sums stay within 32 MiB), summed in share
-// order by the reduction that applies the epilogue (about 8 us, and the sums
-// written and read once at 6.5 TB/s).
+// order by the reduction that applies the epilogue (3 us, and the sums written
+// and read once at 8 TB/s, mostly out of the MALL: 4096 x 12288 at 300 tokens, 5
+// shares: 41.7 us and 5.3).
 Bf16Plan qgemm_bf16_plan(const GemmWeight &w, int64_t m, bool may_split) {
     const int64_t cus = std::max(device_cu_count(), 1), nt = w.n / 256, steps = w.k / BK, full = (m + 255) / 256;
     // the time at which the last of n1 tiles of 256 tokens, then n2 of 128, ends
@@ -645,8 +646,8 @@ Bf16Plan qgemm_bf16_plan(const GemmWeight &w, int64_t m, bool may_split) {
     best.us = std::max(best.us, rows_us);
     const int64_t tiles = (m + 127) / 128 * nt;
     for (int s = 2; may_split && s <= 16 && tiles * s <= cus && steps / s >= 8 && m * w.n < ((int64_t)1 << 31); s++) {
-        const double t = std::max(rows_us, round_us((steps + s - 1) / s, true, tiles * s, cus)) + 8.4 +
-                         8.0 * s * (double)m * (double)w.n / 6.5e6;
+        const double t = std::max(rows_us, round_us((steps + s - 1) / s, true, tiles * s, cus)) + 3.0 +
+                         8.0 * s * (double)m * (double)w.n / 8e6;
         if (t < best.us) best = Bf16Plan{0, s, t};
     }
     return best;
