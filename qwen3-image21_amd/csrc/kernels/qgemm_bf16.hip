@@ -291,26 +291,43 @@ __global__ __launch_bounds__(64 * NWAVE, 1) void qgemm_bf16_kernel(const uint16_
                 }
             }
         } else if constexpr (EPI == EPI_RESID) {
-            // x_out may alias x_in: each element is read and written by the same
-            // lane, a token's loads before its stores
+            // 16 token rows at a time through the wave's part of LDS, so that the x rows
+            // are read and written 512 B at a time, the next 16 rows' x in flight during
+            // the current ones' (4096 x 4096 at 4096 tokens 117 -> 110 us against 16 B
+            // pieces of 16 rows per access; the plain bf16 epilogue takes 103). x_out may
+            // alias x_in: each element is read and written by the same lane.
+            constexpr int P = 132;  // floats per staged row
+            float *stg = (float *)lds + wave * (16 * P);
+            const int64_t mr = m0 + wt * 16 * TT + (lane >> 5), nr = n0 + 128 * wn + 4 * (lane & 31);
+            const bool one = m0 / ep.g_rows_per == (min(m0 + BM, M) - 1) / ep.g_rows_per;  // one gate row
+            f32x4 xv[2][8], gv{};
+            if (one) gv = *(const f32x4 *)(ep.gvec + m0 / ep.g_rows_per * ep.g_stride + nr);
+            auto load_x = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+                for (int q = 0; q < 8; q++) xv[j & 1][q] = *(const f32x4 *)(ep.x_in + min(mr + 16 * j + 2 * q, M - 1) * N + nr);
+            };
+            __syncthreads();  // every wave is done with the operand stages
+            load_x(0);
 #pragma unroll
             for (int j = 0; j < TT; j++) {
-                const int64_t m = mw + 16 * j;
-                if (m >= M) continue;
-                const float *grow = ep.gvec + (int64_t)((int)m / (int)ep.g_rows_per) * ep.g_stride + nw;
-                f32x4 xv[8], gv[8];
+                if (j + 1 < TT) load_x(j + 1);
 #pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    xv[i] = *(const f32x4 *)(ep.x_in + m * N + nw + 16 * i);
-                    gv[i] = *(const f32x4 *)(grow + 16 * i);
-                }
+                for (int i = 0; i < 8; i++) *(f32x4 *)(stg + l16 * P + 16 * i + 4 * lg) = acc[i][j];
+                __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
+                __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                for (int i = 0; i < 8; i++) {
+                for (int q = 0; q < 8; q++) {
+                    const int64_t m = mr + 16 * j + 2 * q;
+                    const f32x4 a = *(const f32x4 *)(stg + (2 * q + (lane >> 5)) * P + 4 * (lane & 31));
+                    if (m >= M) continue;
+                    const f32x4 gr = one ? gv : *(const f32x4 *)(ep.gvec + m / ep.g_rows_per * ep.g_stride + nr);
                     f32x4 o;
 #pragma unroll
-                    for (int e = 0; e < 4; e++) o[e] = xv[i][e] + gv[i][e] * acc[i][j][e];
-                    *(f32x4 *)(ep.x_out + m * N + nw + 16 * i) = o;
+                    for (int e = 0; e < 4; e++) o[e] = xv[j & 1][q][e] + gr[e] * a[e];
+                    *(f32x4 *)(ep.x_out + m * N + nr) = o;
                 }
+                __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);  // the rows are read
+                __builtin_amdgcn_wave_barrier();
             }
         } else if constexpr (EPI == EPI_SWIGLU || EPI == EPI_SWIGLU_Q8K) {
             // rows interleaved per 64 (gate | up): tiles i < 4 are gate rows, i + 4 the
