@@ -198,8 +198,9 @@ int act_qblk(const qimm_block *blk, const qimm_weight *w) {
 // their producers would round them in their epilogues (the gate_up kernels
 // for Q8_K blocks at large M and for Q8_0 blocks at large M or in the
 // undivided 128x128 kernel, the attention kernels for Q8_0 and, paired over
-// two heads, for Q8_K): the reference form the fused ones are checked against
-// bit for bit.
+// two heads, for Q8_K): the reference form the fused ones are checked against,
+// bit for bit where both divide the work alike (a pass of its own can make
+// another split over keys or K the faster one).
 bool separate_rounding() {
     const char *e = getenv("QIMM_SEPARATE_ROUNDING");
     return e && e[0] == '1';
@@ -428,7 +429,12 @@ int qimm_block_reserve(qimm_block *blk, int64_t batch, int64_t seq, int64_t mod_
     QIMM_HIP(ctx, hipSetDevice(ctx->device));
     int rc = ensure_workspace(ctx, L.total);
     if (rc) return rc;
-    return L.part ? ensure_part_workspace(ctx, L.part) : QIMM_OK;
+    // any smaller forward too: fewer tokens may split over K where these do not
+    size_t part = L.part;
+    const qimm_weight *ws_list[] = {blk->qkv, blk->q, blk->k, blk->v, blk->out, blk->gate_up, blk->down};
+    for (const qimm_weight *wt : ws_list)
+        if (wt) part = std::max(part, qimm::qgemm_workspace_up_to(wt->gw, batch * seq));
+    return part ? ensure_part_workspace(ctx, part) : QIMM_OK;
 }
 
 int qimm_block_set_act_mode(qimm_block *blk, int mode) {

@@ -1075,10 +1075,11 @@ hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64
 }  // namespace
 
 size_t attention_scratch_bytes(int64_t bh, int64_t sq) {
+    // what any split of up to this many tiles can take (MAX_PARTS per tile, two
+    // parts per CU): it grows with the tiles, so that scratch reserved for a size
+    // serves every smaller one
     const int64_t cus = device_cu_count(), tiles = (sq + 255) / 256 * bh;
-    if (cus <= 0 || tiles % cus == 0) return 0;
-    const int64_t rest = tiles % cus, parts = std::min<int64_t>(MAX_PARTS, 2 * cus / rest);
-    return parts > 1 ? (size_t)(rest * parts) * 256 * (128 + 2) * 4 : 0;
+    return (size_t)std::min<int64_t>(MAX_PARTS * tiles, 2 * std::max<int64_t>(cus, 0)) * 256 * (128 + 2) * 4;
 }
 
 hipError_t launch_attention(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,

@@ -52,8 +52,9 @@ struct EpiParams {
     // EPI_SWIGLU with hmid_q8k set: hmid receives the hidden state rounded as
     // candle's Q8_K (quant_act4<256> over each 256 columns of a row, ldh and the
     // hidden width multiples of 256), and hmid_f32 is f32 scratch of the same
-    // shape for it (the large-M paired kernel, else the f32 state and then the
-    // rows quantizer)
+    // shape for it (in the epilogue of the 512-row tiles of the kernel over bf16
+    // rows or of the large-M paired kernel, else the f32 state and then the rows
+    // quantizer)
     int hmid_q8k = 0;
     // EPI_SWIGLU with hmid_q8_0 set: hmid receives the hidden state rounded as
     // candle's Q8_0 activations (bf16(d q), one d per 32 columns of a row), by
@@ -139,6 +140,8 @@ int qgemm_mid_splits(const GemmWeight &w, int64_t m);
 // (0 = none): the short-M path's, or the split 128x128 path's partial sums,
 // each after STREAM_COUNTER_BYTES of counters. Without it the unsplit kernels run.
 size_t qgemm_workspace(const GemmWeight &w, int64_t m);
+// The most that any product of up to m rows may use.
+size_t qgemm_workspace_up_to(const GemmWeight &w, int64_t m);
 
 // Static scratch of the allocation-free product (noalloc.hip): one file-scope
 // device array per device. The split 128x128 partials stay within 32 MiB for

@@ -630,6 +630,14 @@ hipError_t launch_small(const GemmWeight &w, const uint16_t *a, int64_t m, int64
 
 }  // namespace
 
+size_t qgemm_workspace_up_to(const GemmWeight &w, int64_t m) {
+    // weight streaming at its sizes; beyond them split grids stay within two
+    // 128x128 tiles, or one 128x256 tile, of f32 sums per CU
+    size_t need = m > 0 ? STREAM_COUNTER_BYTES + (size_t)device_cus() * 2 * 128 * 128 * 4 : 0;
+    for (int64_t s = 1; s <= m && qgemm_stream_fits(w, s); s++) need = std::max(need, qgemm_stream_workspace(w, s));
+    return need;
+}
+
 size_t qgemm_workspace(const GemmWeight &w, int64_t m) {
     if (const Bf16Plan p = bf16_plan(w, m, w.k, true); p.splits) {
         size_t need = bf16_workspace(w, m, p);

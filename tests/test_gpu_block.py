@@ -335,6 +335,34 @@ def test_block_reserve_then_forward(torch_cuda, qctx):
     assert np.array_equal(a, b)
 
 
+def test_block_reserve_covers_smaller_forwards(torch_cuda):
+    """After a reserve, forwards of fewer tokens need no more scratch either, though
+    they may split over K or over keys where the reserved size does not: they can be
+    captured (an allocation or a synchronize would fail the capture)."""
+    torch = torch_cuda
+    ctx, keep = qimm.Context(0), []
+    w, x, mod, pe, _, _ = make_case(21, SMALL, 1, 300, 0, synth.Q4_K, synth.Q6_K)
+    blk = ctx.block_create(qimm.BlockConfig(256, 2, 128, 768), block_tensors(w, keep))
+    blk.reserve(1, 4096)
+    md = dev(torch, mod)
+    for s in (300, 130, 77, 20):
+        xd, pd = dev(torch, x[:, :s]), dev(torch, pe[:s])
+        out = torch.empty_like(xd)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            blk.forward(xd.data_ptr(), out.data_ptr(), 1, s, md.data_ptr(), pd.data_ptr(), None, 0, stream=stream(torch))
+        eager = torch.empty_like(xd)
+        blk.forward(xd.data_ptr(), eager.data_ptr(), 1, s, md.data_ptr(), pd.data_ptr(), None, 0, stream=stream(torch))
+        for _ in range(3):
+            out.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager)
+    blk.free()
+    ctx.close()
+
+
 @pytest.mark.parametrize("case", ["config1_128x128", "wide_ragged", "two_k_shares"])
 def test_hidden_q8_0_rounding_in_gate_up_epilogue_bit_identical(torch_cuda, qctx, monkeypatch, case):
     """Q8_0 down weights in candle mode: the Q8_0 rounding of the SwiGLU hidden

@@ -127,12 +127,13 @@ def test_no_room_for_bf16_rows(torch_cuda, qctx):
     m, n, k = 2304, 4096, 1024  # more 128x128 tiles than two per CU
     rng = np.random.default_rng(77)
     a_dev, _ = bf16_dev(torch, rng.standard_normal((m, k)).astype(np.float32))
-    free, total = torch.cuda.mem_get_info()
     for t in (synth.Q4_K, synth.Q8_0, synth.Q6_K):
         _, w, _, _ = synth.weight(rng, t, n, k)
         ys, sizes = [], []
-        for hold_bytes in (0, free - total // 2 + (1 << 30)):
-            hold = torch.empty(max(hold_bytes, 0), dtype=torch.uint8, device="cuda")
+        for room in (True, False):
+            torch.cuda.empty_cache()  # so that the memory held is taken from what is free now
+            free, total = torch.cuda.mem_get_info()
+            hold = torch.empty(0 if room else max(free - total // 2 + (1 << 30), 0), dtype=torch.uint8, device="cuda")
             W = qctx.upload(t, n, k, w.tobytes())
             sizes.append(W.device_bytes())
             del hold
