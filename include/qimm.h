@@ -159,7 +159,7 @@ int qimm_rope_table(const int64_t *shapes, int64_t nshapes, const uint8_t *image
  * after Q/K norm and RoPE, stored bf16 (KV_CACHE_DTYPE, src/transformer.rs:24)
  * in device memory owned by the library, persistent across steps. Head dim
  * must be 128. Internally k is [B,H,P,128] and v is stored transposed
- * [B,H,128,P] for the attention kernel. */
+ * [B,H,128,P rounded up to 8] for the attention kernel. */
 int qimm_kv_create(qimm_ctx *ctx, int64_t layers, int64_t batch, int64_t heads,
                    int64_t prefix_len, int64_t head_dim, qimm_kv **out);
 int qimm_kv_destroy(qimm_kv *kv);

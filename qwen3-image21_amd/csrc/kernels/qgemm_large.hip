@@ -1,7 +1,8 @@
 // Large-M dequant-GEMM for gfx950 (M >= 512 token rows): C = A (bf16) x W^T
 // (GGUF blocks), same epilogues as the 128x128 kernel. Quantized weights with
-// K % 256 == 0 take the eight-wave kernel of qgemm_wide.hip instead; this one
-// serves bf16-stored weights and the remaining quantized shapes.
+// K % 256 == 0 take the eight-wave kernel of qgemm_wide.hip instead, weights
+// with bf16 rows (bf16-stored ones among them) that of qgemm_bf16.hip; this one
+// serves the shapes those two do not take.
 //
 // Replaces candle's QMatMul::forward (src/quantized_transformer.rs:19-33) on
 // the block's token-parallel projections (call sites 133-135, 151, 196, 202).

@@ -1,6 +1,7 @@
 // Large-M dequant-GEMM for gfx950 with quantized weights (Q4_K, Q6_K, Q8_0;
-// M >= 512 token rows, K % 256 == 0): C = A (bf16) x W^T, the epilogues of
-// the other GEMM kernels.
+// M >= 512 token rows, K % 256 == 0) without bf16 rows beside their codes
+// (qgemm_bf16.hip takes the others): C = A (bf16) x W^T, the epilogues of the
+// other GEMM kernels.
 //
 // Replaces candle's QMatMul::forward (src/quantized_transformer.rs:19-33) on
 // the block's token-parallel projections (call sites 133-135, 151, 196, 202).
