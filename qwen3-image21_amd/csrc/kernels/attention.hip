@@ -17,11 +17,11 @@
 // half are read in a bit-swapped order so that each lane's P^T registers hold 8
 // consecutive keys and every V^T fragment is one 16 B LDS read; the running
 // maximum is folded into the S accumulator start (C = -m) and only moves when it
-// grew by more than 2^8 (rescale_th: at odd lengths, whenever it grew), so the
-// common path is p = exp2(s) (q pre-scaled by
+// grew by more than 2^8, so the common path is p = exp2(s) (q pre-scaled by
 // scale*log2 e) and the rescale of O is a rare wave-uniform branch; row sums use
 // v_dot2_f32_bf16 over the packed bf16 probabilities, the same values the PV
-// product uses.
+// product uses. The exact form (SMODE 3) follows every growth of the maximum and
+// sums the f32 probabilities instead; exact_softmax() says which calls take it.
 // With MASKED it also applies the key mask of build_block_causal_mask (image
 // ids) and key validity, per 64-key window and wave: a window whose keys all lie
 // before the wave's first query, or all share the queries' image block, runs
@@ -67,11 +67,8 @@ struct KeyMask {
 struct ScoreBound {
     const float *k_prefix;
     float q_norm, k_own;
-    // the running-maximum form moves its reference point when the maximum grew by
-    // more than this (log2 units)
-    float rescale_th;
 };
-constexpr float RESCALE_TH = 8.0f;
+constexpr float RESCALE_TH = 8.0f;  // log2 units
 constexpr float STATIC_MAX = 64.0f;
 
 // The last, partial round of query tiles over the CUs, split over the keys: tiles
@@ -277,8 +274,9 @@ constexpr int lds_bytes(int nw) { return 2 * STAGE > nw * 32 * OP * 2 ? 2 * STAG
 // Two waves per SIMD either way: one 8-wave or two 4-wave workgroups per CU.
 // SMODE: 0 = the softmax reference is chosen in the kernel from the score
 // bound (the prefix keys' norm is a device value); 1 = fixed reference, 2 =
-// running maximum, both decided on the host. A kernel with one form has only
-// that loop's registers to allocate.
+// running maximum, both decided on the host; 3 = exact (!PRE: sl2 is 1 where q
+// carries the scale). A kernel with one form has only that loop's registers to
+// allocate.
 // RV: V^T rows whose stride is not a multiple of 16 B (a caller's dense V^T of
 // an odd length) cannot be copied 16 B at a time into LDS: their chunks are
 // loaded unaligned into registers one block ahead and written to the same slots.
@@ -291,9 +289,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
                                                                     float *__restrict__ outf, KeyMask km,
                                                                     const int32_t *__restrict__ lim,
                                                                     ScoreBound sb, int q8, KeySplit sp) {
-    static_assert(!SPLIT || (NW == 8 && PRE && !PAIR && !RV), "the split form is the block's 8-wave one");
+    constexpr bool EXACT = SMODE == 3;
+    static_assert(!SPLIT || (NW == 8 && (PRE || EXACT) && !PAIR && !RV), "the split form is the block's 8-wave one");
+    static_assert(!EXACT || !PRE, "the exact form scales its scores itself");
+    static_assert(!RV || EXACT, "lengths of such rows take the exact form");
     static_assert(NW == 4 || NW == 8, "4 or 8 waves");
-    static_assert(!PAIR || !MASKED, "the paired form is the cached step's");
+    static_assert(!PAIR || (!MASKED && !EXACT), "the paired form is the cached step's");
     constexpr int QB = 32 * NW;  // queries per workgroup
     constexpr int DI = 16 / NW;  // DMA instructions per wave per 16 KB tile
     // operand stages / output staging; in the paired form then each query's
@@ -530,31 +531,19 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
         // scores are kept relative to m_run (score units): the S accumulation
         // starts at -m_run
-        float m_run = 0.f, l_run = 0.f;
+        float m_run = EXACT ? -INFINITY : 0.f, l_run = 0.f;
         f32x16 negm;
 #pragma unroll
         for (int r = 0; r < 16; r++) negm[r] = 0.f;
         bool first_half = true;
         bool fresh = true;  // MASKED: this lane's query has seen no visible key yet
 
+        // -inf for the scores of half h of a window that its query does not see.
         // kmask: visible keys of the window (bit kv), kid: lane kv holds the image
         // id of window key kv, kb0: index of the window's first key, partial: test
         // each score (MASKED only)
-        auto half_step = [&](const uint8_t *stg, int h, int hi, uint64_t kmask, int kid, int kb0,
-                             bool partial, auto stat) __attribute__((always_inline)) {
-            constexpr bool STATIC = decltype(stat)::value;
-            f32x16 st;
-            if constexpr (STATIC) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) st[r] = 0.f;
-            } else {
-                st = negm;
-            }
-#pragma unroll
-            for (int kk = 0; kk < 8; kk++) {
-                const bf16x8 a = *(const bf16x8 *)(stg + h * 32 * 256 + kaddr[kk]);
-                st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[kk], st, 0, 0, 0);
-            }
+        auto hide = [&](f32x16 st, int h, int hi, uint64_t kmask, int kid, int kb0,
+                        bool partial) __attribute__((always_inline)) {
             if (hi < h * 32 + 32) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
@@ -589,6 +578,25 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
                     }
                 }
             }
+            return st;
+        };
+
+        auto half_step = [&](const uint8_t *stg, int h, int hi, uint64_t kmask, int kid, int kb0,
+                             bool partial, auto stat) __attribute__((always_inline)) {
+            constexpr bool STATIC = decltype(stat)::value;
+            f32x16 st;
+            if constexpr (STATIC) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) st[r] = 0.f;
+            } else {
+                st = negm;
+            }
+#pragma unroll
+            for (int kk = 0; kk < 8; kk++) {
+                const bf16x8 a = *(const bf16x8 *)(stg + h * 32 * 256 + kaddr[kk]);
+                st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[kk], st, 0, 0, 0);
+            }
+            st = hide(st, h, hi, kmask, kid, kb0, partial);
             if constexpr (!STATIC) {
             float m0 = st[0], m1 = st[1];
 #pragma unroll
@@ -603,9 +611,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
                 // a lane's first visible key sets its reference point; a row with
                 // none yet keeps 0 (its probabilities are exp2(-inf) = 0)
                 const bool has = mx > -INFINITY;
-                rescale = __builtin_amdgcn_ballot_w64(fresh ? has : mx > sb.rescale_th) != 0;
+                rescale = __builtin_amdgcn_ballot_w64(fresh ? has : mx > RESCALE_TH) != 0;
             } else {
-                rescale = first_half || __builtin_amdgcn_ballot_w64(mx > sb.rescale_th);
+                rescale = first_half || __builtin_amdgcn_ballot_w64(mx > RESCALE_TH);
             }
             if (rescale) {
                 // move the reference point up by d (log2 units); the first half of
@@ -696,6 +704,57 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             }
         };
 
+        // The exact form: the maximum over the window's 64 keys, the reference point
+        // always at the running maximum (the largest probability is 1, with no
+        // rounding), f32 row sums. A row with no visible key yet has the reference
+        // point 0 (its probabilities are exp2(-inf) = 0).
+        float m_ref = 0.f;
+        auto pv_exact = [&](const uint8_t *stg, int h, const f32x16 &st) __attribute__((always_inline)) {
+            uint32_t pk[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float a = __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * i], sl2, -m_ref));
+                const float b = __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * i + 1], sl2, -m_ref));
+                pk[i] = pack_bf16x2(a, b);
+                l_run += a;
+                l_run += b;
+            }
+#pragma unroll
+            for (int kk = 0; kk < 2; kk++) {
+                const bf16x8 pf = __builtin_bit_cast(bf16x8, u32x4{pk[4 * kk], pk[4 * kk + 1], pk[4 * kk + 2], pk[4 * kk + 3]});
+#pragma unroll
+                for (int dt = 0; dt < 4; dt++) {
+                    const bf16x8 a = *(const bf16x8 *)(stg + dt * 32 * 128 + vaddr[h][kk]);
+                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pf, o[dt], 0, 0, 0);
+                }
+            }
+        };
+        auto exact_step = [&](const uint8_t *stg, int hi, uint64_t kmask, int kid, int kb0,
+                              bool partial) __attribute__((always_inline)) {
+            f32x16 s0 = qk_static(stg, 0), s1 = qk_static(stg, 1);
+            s0 = hide(s0, 0, hi, kmask, kid, kb0, partial);
+            s1 = hide(s1, 1, hi, kmask, kid, kb0, partial);
+            float m0 = s0[0], m1 = s1[0];
+#pragma unroll
+            for (int r = 1; r < 16; r++) {
+                m0 = fmaxf(m0, s0[r]);
+                m1 = fmaxf(m1, s1[r]);
+            }
+            const float m_new = fmaxf(m_run, xmax32(fmaxf(m0, m1)) * sl2);
+            if (__builtin_amdgcn_ballot_w64(m_new > m_run)) {
+                m_ref = m_new == -INFINITY ? 0.f : m_new;
+                const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
+                m_run = m_new;
+                l_run *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
+            }
+            pv_exact(stg, 0, s0);
+            pv_exact(stg, 1, s1);
+        };
+
         // MASKED: lane kv loads the image id of window key kv (0 without ids), or
         // KEY_OFF for a padded key, one block ahead; waited for with the tiles.
         constexpr int KEY_OFF = -0x7fffffff - 1;
@@ -735,7 +794,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
             }
             if (j + 1 < nblk) dma(blk_of(j + 1), cur ^ 1);
             const uint8_t *stg = lds + cur * STAGE;
-            if constexpr (decltype(stat)::value && !MASKED) {
+            if constexpr (EXACT) {
+                if (!skip) exact_step(stg, b.hi, kmask, kid, kb0, partial);
+            } else if constexpr (decltype(stat)::value && !MASKED) {
                 const f32x16 s0 = qk_static(stg, 0), s1 = qk_static(stg, 1);
                 pv_static(stg, 0, s0, b.hi);
                 pv_static(stg, 1, s1, b.hi);
@@ -759,7 +820,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
         __syncthreads();
         // the fixed-reference form when the score bound allows it (wave-uniform)
         bool stat_ok = false;
-        if (sb.q_norm > 0.f) {
+        if (!EXACT && sb.q_norm > 0.f) {
             const float kn = sb.k_prefix ? fmaxf(sb.k_own, *sb.k_prefix) : sb.k_own;
             stat_ok = sb.q_norm * kn <= STATIC_MAX;
         }
@@ -773,7 +834,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fast_kernel(const uint16
         };
         if constexpr (SMODE == 1) {
             run(std::true_type{});
-        } else if constexpr (SMODE == 2) {
+        } else if constexpr (SMODE == 2 || EXACT) {
             run(std::false_type{});
         } else {
             if (stat_ok)
@@ -917,7 +978,7 @@ template <int NW, bool PRE, bool MASKED, int SMODE = 0, bool PAIR = false, bool 
 void launch_fast(const uint16_t *q, Seg s0, Seg s1, int64_t h, int64_t sq, int64_t b, float sl2, uint16_t *out,
                  float *outf, const KeyMask &km, const int32_t *lim, const ScoreBound &sb, int q8,
                  hipStream_t stream, KeySplit sp = KeySplit{0, 1, nullptr, nullptr}) {
-    if constexpr (!SPLIT && NW == 8 && PRE && !PAIR && !RV)
+    if constexpr (!SPLIT && NW == 8 && (PRE || SMODE == 3) && !PAIR && !RV)
         if (sp.parts > 1)
             return launch_fast<NW, PRE, MASKED, SMODE, PAIR, RV, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, q8,
                                                                        stream, sp);
@@ -1030,6 +1091,21 @@ bool segments(KeySeg prefix, KeySeg own, Seg &s0, Seg &s1) {
 // has them when its length is a multiple of 8.
 bool rows16(const Seg &s) { return s.len == 0 || s.ld % 8 == 0; }
 
+// Which calls take the exact form: those with a segment length that is no multiple
+// of 8, and the block-causal mask without key limits. There is no other reason in
+// the lengths than that these calls have always had its precision (a register-staged
+// kernel of their own served them) and keep it, while the multiples of 8 have always
+// had the lagging and fixed references. Relative error against 64 bits: exact /
+// fixed, queries like their keys, 77 keys 1.71e-3 / 2.13e-3, 765 keys 1.91e-3 /
+// 2.15e-3; exact / lagging, random queries, 2577 keys 2.26e-3 / 2.33e-3. Time:
+// as the lagging form's; attention of a block, fixed -> exact: 3072 queries over 217 +
+// 3072 keys 201 -> 221 us, 6889 over 131 + 6889 757 -> 845, block-causal 4299 353 -> 409,
+// 4096 over 217 + 4096 309 -> 340 with the Q8_K rounding as a pass (the paired kernel
+// has no exact form).
+bool exact_softmax(const KeySeg &prefix, const KeySeg &own, bool unlimited) {
+    return ((prefix.len | own.len) & 7) != 0 || unlimited;
+}
+
 template <bool PRE>
 hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq, float sl2,
                   uint16_t *out, float *outf, const ScoreBound &sb, int out_qblk, hipStream_t stream,
@@ -1042,11 +1118,12 @@ hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64
     bool rounded = false;
     const KeyMask km{nullptr, nullptr, prefix.len + own.len};
     const int nw = fast_waves(b * h, sq);
+    const bool exact = exact_softmax(prefix, own, false);
+    const bool pair = PRE && !exact && out_qblk == 256 && nw == 8 && h % 2 == 0;
     constexpr int SM = PRE ? 0 : 2;  // without the block's norms no score bound is known
     if constexpr (PRE)
         if (scratch && rows16(s0) && rows16(s1)) {
             const int64_t cus = std::max(device_cu_count(), 1), keys = prefix.len + own.len, n8 = (sq + 255) / 256 * b * h;
-            const bool pair = out_qblk == 256 && nw == 8 && h % 2 == 0;
             const int64_t n4 = (sq + 127) / 128 * b * h, r4 = n4 % (2 * cus);
             const double rounds = pair ? 2.0 * (double)((n8 / 2 + cus - 1) / cus)
                                   : nw == 8 ? (double)((n8 + cus - 1) / cus)
@@ -1055,17 +1132,24 @@ hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64
             const double more = pair ? 5.0 + (double)(b * sq * h) * 128.0 * 6.0 / 4.5e6 : 0.0;
             if (const int parts = split_parts(b * h, sq, keys, false, tile_rounds_us(b * h, sq, keys, false, rounds), more);
                 parts > 1) {
-                launch_fast<8, true, false>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream,
-                                            key_split(b * h, sq, parts, scratch));
+                const KeySplit sp = key_split(b * h, sq, parts, scratch);
+                if (exact)
+                    launch_fast<8, false, false, 3>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream, sp);
+                else
+                    launch_fast<8, true, false>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream, sp);
                 return finish_q8k(out_qblk, false, outf, b, h, sq, out, stream);
             }
         }
     if (!rows16(s0) || !rows16(s1)) {
         if (nw == 4)
-            launch_fast<4, false, false, 2, false, true>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
+            launch_fast<4, false, false, 3, false, true>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
         else
-            launch_fast<8, false, false, 2, false, true>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
-    } else if (PRE && out_qblk == 256 && nw == 8 && h % 2 == 0) {
+            launch_fast<8, false, false, 3, false, true>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
+    } else if (exact && nw == 4) {
+        launch_fast<4, false, false, 3>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
+    } else if (exact) {
+        launch_fast<8, false, false, 3>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
+    } else if (pair) {
         launch_fast<8, true, false, 0, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, nullptr, sb, 0, stream);
         rounded = true;
     } else if (nw == 4) {
@@ -1086,22 +1170,10 @@ size_t attention_scratch_bytes(int64_t bh, int64_t sq) {
     return (size_t)std::min<int64_t>(MAX_PARTS * tiles, 2 * std::max<int64_t>(cus, 0)) * 256 * (128 + 2) * 4;
 }
 
-// How far the running maximum may grow before the reference point follows. At
-// lengths that are multiples of 8 it lags by up to 2^8; at others it follows every
-// growth, as the kernel that served them before did: the largest probability is
-// then exactly 1, with no rounding to bf16. 24 heads, relative error against 64
-// bits and time, lagging -> following: 2244 queries after a prefix of 333, 2.33e-3
-// and 103 us -> 2.26e-3 and 128 us; 1020 after 77, 2.33e-3 and 41 us -> 2.22e-3 and
-// 46 us; 420 after 2001, 2.34e-3 and 71 us -> 2.26e-3 and 82 us. The kernel before:
-// the same errors as following, at 293, 93 and 234 us.
-static float rescale_th(const KeySeg &prefix, const KeySeg &own) {
-    return ((prefix.len | own.len) & 7) == 0 ? RESCALE_TH : 0.f;
-}
-
 hipError_t launch_attention(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
                             float scale, uint16_t *out, hipStream_t stream, float *outf) {
     return launch<false>(q, prefix, own, b, h, sq, scale * 1.4426950408889634f, out, outf,
-                         ScoreBound{nullptr, 0.f, 0.f, rescale_th(prefix, own)}, 0, stream);
+                         ScoreBound{nullptr, 0.f, 0.f}, 0, stream);
 }
 
 hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
@@ -1124,10 +1196,11 @@ hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own,
         lim = lim_scratch;
     }
     // the bound is on scores in log2 units: q's norm times sl2
-    const ScoreBound sb{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm * sl2, k_own_norm, rescale_th(prefix, own)};
+    const ScoreBound sb{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm * sl2, k_own_norm};
+    const bool exact = exact_softmax(prefix, own, img && !lim);
     if (!rows16(s0) || !rows16(s1))
-        launch_fast<8, false, true, 2, false, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream);
-    else if (sl2 == 1.0f) {  // q already carries the scale (the block's q/k/v epilogue)
+        launch_fast<8, false, true, 3, false, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream);
+    else if (exact || sl2 == 1.0f) {  // 1: q already carries the scale (the block's q/k/v epilogue)
         KeySplit sp{0, 1, nullptr, nullptr};
         if (scratch) {
             const int64_t cus = std::max(device_cu_count(), 1), n8 = (sq + 255) / 256 * b * h;
@@ -1135,7 +1208,10 @@ hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own,
             if (const int parts = split_parts(b * h, sq, km.kv_len, true, now, 0.0); parts > 1)
                 sp = key_split(b * h, sq, parts, scratch);
         }
-        launch_masked<true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream, sp);
+        if (exact)
+            launch_fast<8, false, true, 3>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream, sp);
+        else
+            launch_masked<true>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream, sp);
     } else
         launch_masked<false>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream,
                              KeySplit{0, 1, nullptr, nullptr});
@@ -1146,7 +1222,7 @@ hipError_t launch_attention_log2(const uint16_t *q, KeySeg prefix, KeySeg own, i
                                  uint16_t *out, hipStream_t stream, float *outf, const float *k_prefix_norm,
                                  float q_norm, float k_own_norm, int out_qblk, float *scratch) {
     return launch<true>(q, prefix, own, b, h, sq, 1.0f, out, outf,
-                        ScoreBound{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm, k_own_norm, rescale_th(prefix, own)}, out_qblk, stream, scratch);
+                        ScoreBound{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm, k_own_norm}, out_qblk, stream, scratch);
 }
 
 }  // namespace qimm

@@ -217,6 +217,90 @@ def test_block_attention_split_over_keys(torch_cuda, qctx, s, p, norm, padded):
     check_block(*(a.reshape(-1, 256) for a in (outs[0], outs[1], refs[0], refs[1], x)))
 
 
+def exact_softmax_error(q, k, v, see):
+    """Relative error against 64 bits that bf16 probabilities relative to the running maximum
+    (windows of 64 keys), f32 sums of the unrounded ones and a bf16 output have, and the 64-bit
+    values; q, k, v [n, 128] f64 (scores in log2 units), see [queries, keys] bool."""
+    def bf(a):
+        return O.bf16_round(a.astype(np.float32)).astype(np.float64)
+
+    s = np.where(see, q @ k.T, -np.inf)
+    w = np.exp2(s - s.max(1, keepdims=True))
+    want = w @ v / w.sum(1, keepdims=True)
+    m, l, o = np.full(len(q), -np.inf), np.zeros(len(q)), np.zeros((len(q), 128))
+    for j in range(0, len(k), 64):
+        new = np.maximum(m, s[:, j:j + 64].max(1))
+        ref = np.where(np.isinf(new), 0.0, new)
+        a, pr = np.exp2(m - ref), np.exp2(s[:, j:j + 64] - ref[:, None])
+        m, l, o = new, l * a + pr.sum(1), o * a[:, None] + bf(pr) @ v[j:j + 64]
+    return bf(o / l[:, None]) - want, want
+
+
+@pytest.mark.parametrize("s,p,mask", [(77, 0, None), (77, 0, "ids"), (131, 61, None), (131, 61, "valid"), (64, 77, None),
+                                      (700, 65, None), (701, 64, "valid"), (1031, 0, "ids")])
+def test_block_attention_precision_at_odd_lengths(torch_cuda, qctx, s, p, mask):
+    """Lengths that are no multiple of 8: the block's attention rounds its probabilities
+    relative to the running maximum and sums them unrounded, whatever its norms bound.
+    to_out is the identity, gate1 opens fully and gate2 is shut, so that x_out - x is the
+    attention's bf16 output; to_q is to_k and norm_q undoes
+    the softmax scale, so that q is k. Its error
+    against 64 bits is the emulated one (the fixed reference's is 1.09-1.2 times that
+    here). 64 and more query tiles over few CUs split over the keys (700 tokens and more)."""
+    torch = torch_cuda
+    w, x, mod, pe, kpre, vpre = make_case(s + p, SMALL, 1, s, p, synth.BF16, synth.BF16)
+    rng = np.random.default_rng(s)
+    eye = O.f32_to_bf16(np.eye(256, dtype=np.float32))
+    w["to_out"] = (synth.BF16, eye.view(np.uint8).reshape(-1), 256, 256)
+    w["to_q"] = w["to_k"]
+    w["norm_k"] = (0.2 * (1 + 0.1 * rng.standard_normal(128))).astype(np.float32)
+    w["norm_q"] = (w["norm_k"] / np.float32(128 ** -0.5 * np.log2(np.e))).astype(np.float32)
+    mod[..., 256:512], mod[..., 768:] = 30.0, 0.0
+    if p:
+        kpre = O.f32_to_bf16(0.2 * rng.standard_normal((1, 2, p, 128)))
+    n = p + s
+    ids = np.r_[np.full(s // 3, -1), np.zeros(s // 3), np.full(s - 2 * (s // 3), -1)].astype(np.int32) if mask == "ids" else None
+    valid = np.ones((1, n), dtype=np.uint8)
+    if mask == "valid":
+        valid[0, 3:p - 2] = 0
+    see = np.broadcast_to(valid[0] != 0, (s, n))
+    if ids is not None:
+        i, j = np.arange(s)[:, None], np.arange(s)[None, :]
+        see = (i >= j) | ((ids[:, None] >= 0) & (ids[:, None] == ids[None, :]))
+    keep = []
+    blk = qctx.block_create(qimm.BlockConfig(256, 2, 128, 768), block_tensors(w, keep))
+    blk.set_act_mode(qimm.ACT_BF16)
+    xd, md, pd = dev(torch, x), dev(torch, mod), dev(torch, pe)
+    idd, vd = (None if ids is None else dev(torch, ids)), dev(torch, valid)
+    kd, vdv = (dev(torch, a.view(np.int16)) if p else None for a in (kpre, vpre))
+    kv = qctx.kv_create(1, 1, 2, p) if p else None
+    if p:
+        kv.store(0, kd.data_ptr(), vdv.data_ptr(), stream(torch))
+    out = torch.empty_like(xd)
+    k = torch.empty((2, s, 128), dtype=torch.bfloat16, device="cuda")
+    v = torch.empty_like(k)
+    args = (xd.data_ptr(), out.data_ptr(), 1, s, md.data_ptr())
+    tail = (k.data_ptr(), v.data_ptr(), stream(torch))
+    if mask:
+        blk.forward_masked(*args, 1, pd.data_ptr(), None if ids is None else idd.data_ptr(),
+                           vd.data_ptr() if mask == "valid" else None, kv, 0, *tail)
+    else:
+        blk.forward(*args, pd.data_ptr(), kv, 0, *tail)
+    got = (host(out).astype(np.float64) - x)[0]
+    k, v = host(k.float()).astype(np.float64), host(v.float()).astype(np.float64)
+    blk.free()
+    if kv is not None:
+        kv.free()
+    err, emu, size = 0.0, 0.0, 0.0
+    for h in range(2):
+        pk, pv = ((O.bf16_to_f32(a)[0, h].astype(np.float64) for a in (kpre, vpre)) if p else (np.zeros((0, 128)),) * 2)
+        e, want = exact_softmax_error(k[h], np.concatenate([pk, k[h]]), np.concatenate([pv, v[h]]), see)
+        err += np.sum((got[:, 128 * h:128 * (h + 1)] - want) ** 2)
+        emu += np.sum(e ** 2)
+        size += np.sum(want ** 2)
+    print(f"error against 64 bits {np.sqrt(err / size):.3e}, emulated {np.sqrt(emu / size):.3e}", flush=True)
+    assert err <= 1.04 ** 2 * emu
+
+
 def test_block_deterministic(torch_cuda, qctx):
     w, x, mod, pe, kpre, vpre = make_case(9, SMALL, 1, 96, 32, synth.Q4_K, synth.Q6_K)
     a, _ = run_block(torch_cuda, qctx, SMALL, w, x, mod, pe, kpre, vpre)
