@@ -135,6 +135,28 @@ int qimm_qmatmul_noalloc(qimm_ctx *ctx, const qimm_weight *w, const void *x_bf16
  * compute-unit count (the split plans). No counterpart in the reference. */
 int64_t qimm_qmatmul_scratch_bytes(const qimm_weight *w, int64_t m);
 
+/* How qimm_qmatmul takes the product of m rows with a rows x cols weight of the
+ * type, with or without bf16 rows beside its codes (bf16_rows 1 or 0; float
+ * types always have them), on a device of cus compute units: no device is
+ * needed to ask. The block's products take the same kernels, with their own
+ * epilogues. No counterpart in the reference. */
+typedef enum {
+    QIMM_GEMM_STREAM = 1,   /* weight streaming, few rows */
+    QIMM_GEMM_128 = 2,      /* 128 x 128 tiles, decoding */
+    QIMM_GEMM_LARGE = 3,    /* 256 x 256 tiles, four waves, decoding */
+    QIMM_GEMM_WIDE = 4,     /* 256 x 256 tiles, eight waves, decoding */
+    QIMM_GEMM_BF16_ROWS = 5 /* tiles of 256 and 128 tokens over bf16 rows */
+} qimm_gemm_kernel;
+typedef struct {
+    int32_t kernel;         /* of the rows before the tail */
+    int32_t splits;         /* shares of K that a second launch adds (1: none) */
+    int64_t large_tiles;    /* QIMM_GEMM_BF16_ROWS: token tiles of 256 */
+    int64_t tail;           /* last rows that are a product of their own (0: none) */
+    int64_t scratch;        /* bytes of split-K scratch */
+} qimm_gemm_route;
+int qimm_qmatmul_route(int ggml_type, int64_t rows, int64_t cols, int bf16_rows, int64_t m,
+                       int cus, qimm_gemm_route *out);
+
 /* ---------------- host-side layout and RoPE ---------------- */
 
 /* JointLayout::new (src/joint_layout.rs:52-103). text_image_mask may be NULL

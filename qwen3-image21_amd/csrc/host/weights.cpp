@@ -293,6 +293,34 @@ int qimm_qmatmul_noalloc(qimm_ctx *ctx, const qimm_weight *w, const void *x_bf16
     return QIMM_OK;
 }
 
+int qimm_qmatmul_route(int ggml_type, int64_t rows, int64_t cols, int bf16_rows, int64_t m, int cus,
+                       qimm_gemm_route *out) {
+    static_assert(qimm::GEMM_STREAM == QIMM_GEMM_STREAM && qimm::GEMM_128 == QIMM_GEMM_128 &&
+                      qimm::GEMM_LARGE == QIMM_GEMM_LARGE && qimm::GEMM_WIDE == QIMM_GEMM_WIDE &&
+                      qimm::GEMM_BF16_ROWS == QIMM_GEMM_BF16_ROWS,
+                  "kernel numbers of qimm.h");
+    if (!out || m <= 0 || cus <= 0) return QIMM_ERR_ARG;
+    if (!block_values(ggml_type)) return QIMM_ERR_TYPE;
+    if (rows <= 0 || rows % 128 || cols <= 0 || cols % 64 || row_bytes(ggml_type, cols) < 0) return QIMM_ERR_SHAPE;
+    const qimm::AssumeCus assume(cus);
+    static uint16_t some;  // an address for the plans, which only test for one
+    qimm::GemmWeight w{};
+    w.fmt = ggml_type == QIMM_TYPE_Q8_0 ? qimm::WF_Q8_0
+            : ggml_type == QIMM_TYPE_Q4_K ? qimm::WF_Q4_K
+            : ggml_type == QIMM_TYPE_Q6_K ? qimm::WF_Q6_K : qimm::WF_BF16;
+    w.n = rows;
+    w.k = cols;
+    if (w.fmt == qimm::WF_BF16 || bf16_rows) w.bf16 = &some;
+    qimm::EpiParams ep{};
+    ep.ldo = rows;
+    ep.part_ws_bytes = qimm::qgemm_workspace(w, m);
+    if (ep.part_ws_bytes) ep.part_ws = (float *)&some;
+    const int64_t tail = qimm::qgemm_route(w, m, cols, qimm::EPI_F32, ep).tail;
+    const qimm::GemmRoute r = qimm::qgemm_route(w, m - tail, cols, qimm::EPI_F32, ep);
+    *out = {r.kernel, r.splits, r.head, tail, (int64_t)ep.part_ws_bytes};
+    return QIMM_OK;
+}
+
 int64_t qimm_qmatmul_scratch_bytes(const qimm_weight *w, int64_t m) {
     if (!w || m < 0) return -1;
     if (hipSetDevice(w->ctx->device) != hipSuccess) return -1;

@@ -86,9 +86,29 @@ struct GemmWeight {
 // CU), the 128x128 kernel the rest.
 hipError_t launch_qgemm(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda,
                         int epi, const EpiParams &ep, hipStream_t stream);
+// How launch_qgemm takes a product: the kernel (qimm_gemm_kernel's values), its shares
+// of K, the token tiles of 256 of the kernel over bf16 rows, the last rows that run as
+// a product of their own first (0: none), and whether the kernel rounds the SwiGLU
+// hidden state itself.
+enum : int { GEMM_STREAM = 1, GEMM_128 = 2, GEMM_LARGE = 3, GEMM_WIDE = 4, GEMM_BF16_ROWS = 5 };
+struct GemmRoute {
+    int kernel;
+    int splits;
+    int64_t head;
+    int64_t tail;
+    bool rounds;
+};
+GemmRoute qgemm_route(const GemmWeight &w, int64_t m, int64_t lda, int epi, const EpiParams &ep);
 bool qgemm_large_fits(const GemmWeight &w, int64_t m);
 // Compute units of the current device (0 if the runtime cannot say), read once.
 int device_cu_count();
+// While it lives, this thread plans for a device of `cus` compute units (a route is
+// asked for without a device).
+struct AssumeCus {
+    explicit AssumeCus(int cus);
+    ~AssumeCus();
+    int before;
+};
 
 // Short-M weight-streaming path (M <= 64): split-K partial sums, added in a
 // fixed order by the epilogue (in the same launch for Q4_K / Q6_K at M <= 16).

@@ -480,7 +480,14 @@ hipError_t launch_any(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t
 
 }  // namespace
 
+namespace {
+thread_local int assumed_cus = 0;
+}
+AssumeCus::AssumeCus(int cus) : before(assumed_cus) { assumed_cus = cus; }
+AssumeCus::~AssumeCus() { assumed_cus = before; }
+
 int device_cu_count() {
+    if (assumed_cus > 0) return assumed_cus;
     // initialised once, by the first caller (a function-local static: thread-safe)
     static const int cus = [] {
         int dev = 0, v = 0;
@@ -609,23 +616,17 @@ SmallPath small_path(const GemmWeight &w, int64_t m, const EpiParams &ep) {
     return SmallPath::WHOLE;
 }
 
-hipError_t launch_small(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda, int epi, const EpiParams &ep,
-                        hipStream_t stream) {
-    const SmallPath path = small_path(w, m, ep);
-    if (path == SmallPath::STREAM) return launch_qgemm_stream(w, a, m, lda, epi, ep, ep.part_ws, stream);
-    if (path == SmallPath::SPLIT) {
-        const int splits = qgemm_mid_splits(w, m);
-        // partial sums [splits][m][n] after the counter area, then the fixed-order
-        // reduction that applies the epilogue
-        float *part = (float *)((char *)ep.part_ws + STREAM_COUNTER_BYTES);
-        EpiParams pe{};
-        pe.out = part;
-        pe.ldo = w.n;
-        const hipError_t e = launch_any(w, a, m, lda, EPI_F32, pe, stream, splits);
-        if (e != hipSuccess) return e;
-        return launch_split_epilogue(part, splits, m, w.n, epi, ep, stream);
-    }
-    return launch_any(w, a, m, lda, epi, ep, stream, 1);
+// the 128x128 kernel, split: partial sums [splits][m][n] after the counter area,
+// then the fixed-order reduction that applies the epilogue
+hipError_t launch_split(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda, int epi, const EpiParams &ep,
+                        int splits, hipStream_t stream) {
+    float *part = (float *)((char *)ep.part_ws + STREAM_COUNTER_BYTES);
+    EpiParams pe{};
+    pe.out = part;
+    pe.ldo = w.n;
+    const hipError_t e = launch_any(w, a, m, lda, EPI_F32, pe, stream, splits);
+    if (e != hipSuccess) return e;
+    return launch_split_epilogue(part, splits, m, w.n, epi, ep, stream);
 }
 
 }  // namespace
@@ -699,20 +700,20 @@ EpiParams rows_from(const EpiParams &ep, int epi, const GemmWeight &w, int64_t h
     return e;
 }
 
-// A product over bf16 rows: the tail after full rounds as a product of its own
-// where that is faster and its epilogue's rows can be shifted, else one launch;
-// the rounding of the SwiGLU hidden state in the epilogue where it can be (whole
-// Q8_K blocks need 512 weight rows per tile), else in a pass over f32 rows.
-hipError_t launch_bf16_rows(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda, int epi, const EpiParams &ep,
-                            Bf16Plan p, hipStream_t stream) {
+// A product over bf16 rows (plan p of bf16_plan): the tail after full rounds as a
+// product of its own where that is faster and its epilogue's rows can be shifted,
+// else one launch; the rounding of the SwiGLU hidden state in the epilogue where
+// it can be (whole Q8_K blocks need 512 weight rows per tile), else in a pass over
+// f32 rows.
+GemmRoute bf16_route(const GemmWeight &w, int64_t m, int64_t lda, int epi, const EpiParams &ep, Bf16Plan p) {
     // q/k/v reduces whole sequences only; any split needs its scratch
     if (p.splits > 1 && (ep.part_ws_bytes < bf16_workspace(w, m, p) || (epi == EPI_QKV && m % ep.seq)))
         p = qgemm_bf16_plan(w, m, false);
     const bool swiglu = epi == EPI_SWIGLU, q8k = swiglu && ep.hmid_q8k, q8_0 = swiglu && ep.hmid_q8_0;
-    if (q8k && (!ep.hmid || !ep.hmid_f32 || ep.ldh % 256 || (w.n / 2) % 256)) return hipErrorInvalidValue;
-    if (q8_0 && (!ep.hmid || !ep.hmid_f32 || (w.n / 2) % 32)) return hipErrorInvalidValue;
     const double q8k_us = q8k ? qgemm_bf16_q8k_us(w, m) : 0.0, sep_us = p.us + quant_pass_us(w, m);
     const double us = q8k ? std::min(q8k_us, sep_us) : p.us;
+    GemmRoute r{GEMM_BF16_ROWS, p.splits, p.head, 0, q8k ? sep_us >= q8k_us : q8_0 && p.splits == 1};
+    if (q8k && r.rounds) r.splits = 1;
     if (const int64_t tail = ep.part_ws ? bf16_tail_rows(w, m, lda, q8k, us) : 0) {
         const int64_t head = m - tail;
         bool shift = ep.part_ws_bytes >= qgemm_workspace(w, tail);
@@ -722,66 +723,63 @@ hipError_t launch_bf16_rows(const GemmWeight &w, const uint16_t *a, int64_t m, i
             shift = shift && ep.seq > 0 && head / ep.seq == (m - 1) / ep.seq &&
                     (pt.splits ? true : small_path(w, tail, ep) == SmallPath::WHOLE);
         }
-        if (shift) {
-            const hipError_t e = launch_qgemm(w, a, head, lda, epi, ep, stream);
-            if (e != hipSuccess) return e;
-            return launch_qgemm(w, a + head * lda, tail, lda, epi, rows_from(ep, epi, w, head), stream);
-        }
+        if (shift) r.tail = tail;
     }
-    if ((q8k && sep_us < q8k_us) || (q8_0 && p.splits > 1)) {
-        EpiParams e = ep;
-        e.hmid_q8k = e.hmid_q8_0 = 0;
-        const hipError_t err = launch_qgemm_bf16(w, a, m, lda, EPI_SWIGLU, e, p, stream);
-        if (err != hipSuccess) return err;
-        return launch_quant_rows(ep.hmid_f32, ep.ldh, m, w.n / 2, q8k ? 256 : 32, ep.hmid, ep.ldh, stream);
-    }
-    if (q8k) p.splits = 1;
-    return launch_qgemm_bf16(w, a, m, lda, epi, ep, p, stream);
+    return r;
 }
 
 }  // namespace
 
-hipError_t launch_qgemm(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda, int epi,
-                        const EpiParams &ep, hipStream_t stream) {
-    if (m <= 0) return hipSuccess;
+GemmRoute qgemm_route(const GemmWeight &w, int64_t m, int64_t lda, int epi, const EpiParams &ep) {
     if (const Bf16Plan p = bf16_plan(w, m, lda, ep.part_ws != nullptr); p.splits && (epi != EPI_QKV || ep.hidden % 256 == 0))
-        return launch_bf16_rows(w, a, m, lda, epi, ep, p, stream);
+        return bf16_route(w, m, lda, epi, ep, p);
     // a last, nearly empty round of 256x256 tiles: those rows as a shorter-M
     // product of their own (whole rounds above, the 128x128 or short-M path
     // for the tail), each part with its own form of the epilogue
-    if (const int64_t tail = tail_rows(w, m, epi, ep)) {
-        const int64_t head = m - tail;
+    const int64_t tail = tail_rows(w, m, epi, ep);
+    if (qgemm_large_fits(w, m)) {
+        // the Q8_K rounding of the hidden state inside the paired kernel, the Q8_0 one
+        // in the eight-wave kernel's epilogue
+        const bool wide = qgemm_wide_fits(w) && (epi != EPI_QKV || ep.hidden % 256 == 0);
+        return {wide ? GEMM_WIDE : GEMM_LARGE, 1, 0, tail, ep.hmid_q8k ? qgemm_wide_pairs_fit(w) : wide};
+    }
+    switch (small_path(w, m, ep)) {
+    case SmallPath::STREAM: return {GEMM_STREAM, 1, 0, tail, false};
+    case SmallPath::SPLIT: return {GEMM_128, qgemm_mid_splits(w, m), 0, tail, false};
+    default: return {GEMM_128, 1, 0, tail, !ep.hmid_q8k};  // Q8_0 blocks in the undivided kernel's epilogue
+    }
+}
+
+hipError_t launch_qgemm(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda, int epi,
+                        const EpiParams &ep, hipStream_t stream) {
+    if (m <= 0) return hipSuccess;
+    const int rounding = epi != EPI_SWIGLU ? 0 : ep.hmid_q8k ? 256 : ep.hmid_q8_0 ? 32 : 0;
+    if (rounding && (!ep.hmid || !ep.hmid_f32 || (w.n / 2) % rounding || (rounding == 256 && ep.ldh % 256)))
+        return hipErrorInvalidValue;
+    const GemmRoute r = qgemm_route(w, m, lda, epi, ep);
+    if (r.tail) {
+        const int64_t head = m - r.tail;
         const hipError_t e = launch_qgemm(w, a, head, lda, epi, ep, stream);
         if (e != hipSuccess) return e;
-        return launch_qgemm(w, a + head * lda, tail, lda, epi, rows_from(ep, epi, w, head), stream);
+        return launch_qgemm(w, a + head * lda, r.tail, lda, epi, rows_from(ep, epi, w, head), stream);
     }
-    if (epi == EPI_SWIGLU && ep.hmid_q8k) {
-        // the Q8_K rounding of the hidden state: inside the paired large-M
-        // kernel where it runs, else the f32 state and then the rows quantizer
-        if (!ep.hmid || !ep.hmid_f32 || ep.ldh % 256 || (w.n / 2) % 256) return hipErrorInvalidValue;
-        if (qgemm_large_fits(w, m) && qgemm_wide_pairs_fit(w)) return launch_qgemm_large(w, a, m, lda, epi, ep, stream);
-        EpiParams e = ep;
-        e.hmid_q8k = 0;
-        const hipError_t err = launch_qgemm(w, a, m, lda, EPI_SWIGLU, e, stream);
-        if (err != hipSuccess) return err;
-        return launch_quant_rows(ep.hmid_f32, ep.ldh, m, w.n / 2, 256, ep.hmid, ep.ldh, stream);
-    }
-    if (epi == EPI_SWIGLU && ep.hmid_q8_0) {
-        // the Q8_0 rounding of the hidden state: in the epilogue of the large-M
-        // kernel or the undivided 128x128 kernel where one of them runs, else
-        // the f32 state and then the rows quantizer
-        if (!ep.hmid || !ep.hmid_f32 || (w.n / 2) % 32) return hipErrorInvalidValue;
-        if (qgemm_large_fits(w, m) ? qgemm_wide_fits(w) : small_path(w, m, ep) == SmallPath::WHOLE)
-            return qgemm_large_fits(w, m) ? launch_qgemm_large(w, a, m, lda, epi, ep, stream)
-                                          : launch_small(w, a, m, lda, epi, ep, stream);
-        EpiParams e = ep;
-        e.hmid_q8_0 = 0;
-        const hipError_t err = launch_qgemm(w, a, m, lda, EPI_SWIGLU, e, stream);
-        if (err != hipSuccess) return err;
-        return launch_quant_rows(ep.hmid_f32, ep.ldh, m, w.n / 2, 32, ep.hmid, ep.ldh, stream);
-    }
-    if (qgemm_large_fits(w, m)) return launch_qgemm_large(w, a, m, lda, epi, ep, stream);
-    return launch_small(w, a, m, lda, epi, ep, stream);
+    auto run = [&](const EpiParams &e) {
+        switch (r.kernel) {
+        case GEMM_STREAM: return launch_qgemm_stream(w, a, m, lda, epi, e, e.part_ws, stream);
+        case GEMM_128:
+            return r.splits > 1 ? launch_split(w, a, m, lda, epi, e, r.splits, stream)
+                                : launch_any(w, a, m, lda, epi, e, stream, 1);
+        case GEMM_BF16_ROWS: return launch_qgemm_bf16(w, a, m, lda, epi, e, Bf16Plan{r.head, r.splits, 0.0}, stream);
+        default: return launch_qgemm_large(w, a, m, lda, epi, e, stream);
+        }
+    };
+    if (!rounding || r.rounds) return run(ep);
+    // the f32 hidden state, then the rows quantizer
+    EpiParams e = ep;
+    e.hmid_q8k = e.hmid_q8_0 = 0;
+    const hipError_t err = run(e);
+    if (err != hipSuccess) return err;
+    return launch_quant_rows(ep.hmid_f32, ep.ldh, m, w.n / 2, rounding, ep.hmid, ep.ldh, stream);
 }
 
 }  // namespace qimm

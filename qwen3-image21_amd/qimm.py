@@ -48,6 +48,7 @@ SIGNATURES = [
     ("qimm_qmatmul", _i32, [_vp, _vp, _vp, _i64, _i64, _vp, _i32, _vp]),
     ("qimm_qmatmul_noalloc", _i32, [_vp, _vp, _vp, _i64, _i64, _vp, _i32, _vp]),
     ("qimm_qmatmul_scratch_bytes", _i64, [_vp, _i64]),
+    ("qimm_qmatmul_route", _i32, [_i32, _i64, _i64, _i32, _i64, _i32, _vp]),
     ("qimm_joint_layout", _i32, [_i64, _vp, _vp, _i64, _i64, _i64, _vp, _i64,
                                  C.POINTER(_i64), C.POINTER(_i64), C.POINTER(_i64)]),
     ("qimm_rope_table", _i32, [_vp, _i64, _vp, _i64, _vp, C.c_double, _vp]),
@@ -138,6 +139,16 @@ class GgufTensorInfo(C.Structure):
                 ("data", _vp), ("nbytes", C.c_size_t), ("offset", C.c_uint64)]
 
 
+class GemmRoute(C.Structure):
+    """qimm_gemm_route."""
+    _fields_ = [("kernel", C.c_int32), ("splits", C.c_int32), ("large_tiles", _i64), ("tail", _i64),
+                ("scratch", _i64)]
+
+
+# qimm_gemm_kernel
+GEMM_STREAM, GEMM_128, GEMM_LARGE, GEMM_WIDE, GEMM_BF16_ROWS = 1, 2, 3, 4, 5
+
+
 class QimmError(RuntimeError):
     def __init__(self, msg, status=None):
         super().__init__(msg)
@@ -169,6 +180,15 @@ def load(path: str = LIB_PATH) -> C.CDLL:
 
 def status_name(rc: int) -> str:
     return STATUS.get(rc, f"status {rc}")
+
+
+def qmatmul_route(ggml_type: int, rows: int, cols: int, m: int, cus: int, bf16_rows: bool = True) -> GemmRoute:
+    """How Context.qmatmul takes m rows on a device of cus compute units (no device needed)."""
+    r = GemmRoute()
+    rc = load().qimm_qmatmul_route(ggml_type, rows, cols, int(bf16_rows), m, cus, C.byref(r))
+    if rc:
+        raise QimmError(f"qimm_qmatmul_route: {status_name(rc)}", rc)
+    return r
 
 
 class Context:

@@ -8,6 +8,7 @@ import subprocess
 import pytest
 
 import qimm
+from test_gpu_kernels import BF16_ROWS_CASES, bf16_rows_route
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "qimm.h")
@@ -63,3 +64,25 @@ def test_ctx_create_without_gpu_fails_cleanly():
     h = C.c_void_p()
     rc = qimm.load().qimm_ctx_create(0, C.byref(h))
     assert rc != 0 and not h.value
+
+
+@pytest.mark.parametrize("t,m,n,k,route", BF16_ROWS_CASES)
+def test_bf16_rows_cases_take_the_paths_they_name(t, m, n, k, route):
+    """The GPU cases of the kernel over bf16 rows run that kernel, in the shares of K, tiles
+    and tail that each is there for, on 256 compute units."""
+    assert bf16_rows_route(t, m, n, k, 256) == (True, route)
+
+
+def test_qmatmul_route_codes():
+    lib = qimm.load()
+    r = qimm.GemmRoute()
+    assert lib.qimm_qmatmul_route(qimm.Q4_K, 256, 256, 1, 100, 256, None) == 1
+    assert lib.qimm_qmatmul_route(qimm.Q4_K, 256, 256, 1, 0, 256, C.byref(r)) == 1
+    assert lib.qimm_qmatmul_route(qimm.Q4_K, 96, 256, 1, 100, 256, C.byref(r)) == 2
+    assert lib.qimm_qmatmul_route(7, 256, 256, 1, 100, 256, C.byref(r)) == 3
+    # few rows stream the codes; without bf16 rows many rows decode in 256 x 256 tiles
+    assert qimm.qmatmul_route(qimm.Q4_K, 4096, 4096, 16, 256).kernel == qimm.GEMM_STREAM
+    assert qimm.qmatmul_route(qimm.Q4_K, 4096, 4096, 4352, 256).kernel == qimm.GEMM_BF16_ROWS
+    assert qimm.qmatmul_route(qimm.Q4_K, 4096, 4096, 4352, 256, bf16_rows=False).kernel == qimm.GEMM_WIDE
+    # float weights are bf16 rows themselves
+    assert qimm.qmatmul_route(qimm.BF16, 4096, 4096, 4352, 256, bf16_rows=False).kernel == qimm.GEMM_BF16_ROWS

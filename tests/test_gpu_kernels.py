@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+import qimm
 import synth
 from gpu_util import bf16_dev, cos_sim, dev, host, max_abs_rel, stream
 from test_oracle_codecs import q4k_block, q6k_block, q8_block, Q8_CODES
@@ -101,16 +102,32 @@ def test_qmatmul_matches_bf16_weight_products(torch_cuda, qctx, t, m, n, k):
         assert cos_sim(got, yc) >= 0.9999 and max_abs_rel(got, yc) <= 2e-2
 
 
-# the kernel over bf16 rows: two k steps (the least), an odd and a large number of steps past
-# its three and two stages, one token past a tile of 128 and of 256, both tile sizes in one
-# launch (3072 x 12288: ten tiles of 256, four of 128), shares of K with unequal steps, and a
-# tail after full rounds (4299 rows x N = 4096)
-@pytest.mark.parametrize("t,m,n,k", [(synth.Q8_0, 129, 256, 128), (synth.BF16, 200, 256, 128), (synth.BF16, 385, 512, 384),
-                                     (synth.Q4_K, 257, 512, 1280), (synth.Q6_K, 300, 512, 5120),
-                                     (synth.Q4_K, 100, 1024, 4096), (synth.Q8_0, 3072, 12288, 128),
-                                     (synth.Q6_K, 4299, 4096, 256), (synth.Q4_K, 1025, 4096, 1024)])
-def test_qmatmul_bf16_rows(torch_cuda, qctx, t, m, n, k):
+# the kernel over bf16 rows: type, m, n, k and how 256 compute units take it (shares of K,
+# token tiles of 256, tail rows; tests/test_capi_cpu.py holds the plan to it)
+BF16_ROWS_CASES = [
+    (synth.Q8_0, 129, 256, 128, (1, 0, 0)),      # two k steps, the least; one token past a tile of 128
+    (synth.BF16, 200, 256, 128, (1, 0, 0)),
+    (synth.BF16, 385, 512, 384, (1, 0, 0)),      # tiles of 128: six steps over three stages
+    (synth.Q4_K, 257, 512, 1280, (2, 0, 0)),
+    (synth.Q6_K, 300, 512, 5120, (10, 0, 0)),
+    (synth.Q6_K, 300, 4096, 12288, (5, 0, 0)),   # shares of 38 and 39 steps
+    (synth.Q4_K, 1025, 4096, 1024, (1, 0, 0)),   # nine tiles of 128, one token in the last
+    (synth.Q4_K, 2049, 4096, 1024, (1, 9, 0)),   # tiles of 256 alone, one token in the last
+    (synth.Q6_K, 4299, 4096, 256, (1, 2, 0)),    # both tile sizes in one launch
+    (synth.Q6_K, 4299, 4096, 4096, (1, 16, 203)),  # one full round, then a tail of its own
+]
+
+
+def bf16_rows_route(t, m, n, k, cus):
+    r = qimm.qmatmul_route(t, n, k, m, cus)
+    return (r.kernel == qimm.GEMM_BF16_ROWS, (r.splits, r.large_tiles, r.tail))
+
+
+@pytest.mark.parametrize("t,m,n,k,route", BF16_ROWS_CASES)
+def test_qmatmul_bf16_rows(torch_cuda, qctx, t, m, n, k, route):
     """Products of the bf16 activations and the bf16-rounded weights, f32 sums in any order."""
+    cus = torch_cuda.cuda.get_device_properties(0).multi_processor_count
+    assert bf16_rows_route(t, m, n, k, cus) == (True, route)
     got, a, w = _gemm_case(torch_cuda, qctx, t, m, n, k, seed=m + n + k + t)
     Wb = O.bf16_round(O.dequantize(t, w, n * k).reshape(n, k)).astype(np.float64)
     rows = np.unique(np.concatenate([np.arange(min(m, 140)), np.arange(m // 2, m // 2 + 20), np.arange(m - 45, m)]))
@@ -302,7 +319,6 @@ def test_qmatmul_large_m_tail_rows(torch_cuda, qctx, m, n, k, t, out):
 
 
 def test_qmatmul_rejects_bad_shapes(torch_cuda, qctx):
-    import qimm
     rng = np.random.default_rng(8)
     _, w, _, _ = synth.weight(rng, synth.Q8_0, 96, 64)   # N not a multiple of 128
     W = qctx.upload(synth.Q8_0, 96, 64, w.tobytes())
