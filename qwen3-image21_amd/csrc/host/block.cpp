@@ -198,9 +198,8 @@ int act_qblk(const qimm_block *blk, const qimm_weight *w) {
 // their producers would round them in their epilogues (the gate_up kernels
 // for Q8_K blocks at large M and for Q8_0 blocks at large M or in the
 // undivided 128x128 kernel, the attention kernels for Q8_0 and, paired over
-// two heads, for Q8_K): the reference form the fused ones are checked against,
-// bit for bit where both divide the work alike (a pass of its own can make
-// another split over keys or K the faster one).
+// two heads, for Q8_K): the reference form the fused ones are checked against bit
+// for bit, with the work divided as they divide it.
 bool separate_rounding() {
     const char *e = getenv("QIMM_SEPARATE_ROUNDING");
     return e && e[0] == '1';
@@ -339,7 +338,6 @@ int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t ba
     const int qb_out = act_qblk(blk, blk->out);
     float *stage_f32 = (float *)(ws + L.f32);
     const bool round_sep = separate_rounding();
-    const int att_q = round_sep ? 0 : qb_out;
     float *att_f32 = qb_out ? stage_f32 : nullptr;
     const qimm::KeySeg own{kb, vt, seq, ep.vt_ld};
     float *keys_f32 = qimm::attention_scratch_bytes(batch * H, seq) ? (float *)(ws + L.keys) : nullptr;
@@ -347,10 +345,10 @@ int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t ba
     const float *kpn = kv ? kv->knorm + layer : nullptr;
     if (img || kvalid)
         QIMM_HIP(ctx, qimm::launch_attention_masked(qb, prefix, own, batch, H, seq, 1.0f, img, kvalid, (int32_t *)(ws + L.lim), att, s, att_f32, kpn,
-                                                    blk->q_norm_bound, blk->k_norm_bound, att_q, keys_f32));
+                                                    blk->q_norm_bound, blk->k_norm_bound, qb_out, keys_f32, round_sep));
     else
         QIMM_HIP(ctx, qimm::launch_attention_log2(qb, prefix, own, batch, H, seq, att, s, att_f32, kpn,
-                                                  blk->q_norm_bound, blk->k_norm_bound, att_q, keys_f32));
+                                                  blk->q_norm_bound, blk->k_norm_bound, qb_out, keys_f32, round_sep));
     if (kv) {
         const int rc = kv_release(kv, layer, s);
         if (rc) return rc;
@@ -384,9 +382,10 @@ int block_forward_impl(qimm_block *blk, const float *x, float *x_out, int64_t ba
     if (qb_down) eg.hmid_f32 = stage_f32;
     // the gate_up launch rounds them itself: Q8_K blocks (K-quant down
     // weights), Q8_0 blocks (Q8_0 down weights)
-    const bool round_in_gemm = (qb_down == 32 || (qb_down == 256 && F % 256 == 0)) && !separate_rounding();
-    eg.hmid_q8k = round_in_gemm && qb_down == 256;
-    eg.hmid_q8_0 = round_in_gemm && qb_down == 32;
+    eg.hmid_q8k = qb_down == 256 && F % 256 == 0;
+    eg.hmid_q8_0 = qb_down == 32;
+    eg.hmid_round_later = round_sep;
+    const bool round_in_gemm = (eg.hmid_q8k || eg.hmid_q8_0) && !round_sep;
     QIMM_HIP(ctx, qimm::launch_qgemm(blk->gate_up->gw, xn, M, hid, qimm::EPI_SWIGLU, eg, s));
     STAGE_MARK(7);
     if (qb_down && !round_in_gemm) QIMM_HIP(ctx, qimm::launch_quant_rows(stage_f32, F, M, F, qb_down, hm, F, s));

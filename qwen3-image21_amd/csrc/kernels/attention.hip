@@ -1109,13 +1109,13 @@ bool exact_softmax(const KeySeg &prefix, const KeySeg &own, bool unlimited) {
 template <bool PRE>
 hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq, float sl2,
                   uint16_t *out, float *outf, const ScoreBound &sb, int out_qblk, hipStream_t stream,
-                  float *scratch = nullptr) {
+                  float *scratch = nullptr, bool round_later = false) {
     if (sq <= 0 || b <= 0 || h <= 0) return hipSuccess;
     Seg s0, s1;
     if (!segments(prefix, own, s0, s1) || !out_qblk_ok(out_qblk, outf)) return hipErrorInvalidValue;
-    const int q8 = out_qblk == 32;
-    float *f32out = out_qblk == 32 ? nullptr : outf;  // f32 output (0 with outf, or 256 not paired)
-    bool rounded = false;
+    const int q8 = out_qblk == 32 && !round_later;
+    float *f32out = q8 ? nullptr : outf;  // f32 output (0 with outf, 256 not paired, or round_later)
+    bool rounded = round_later;
     const KeyMask km{nullptr, nullptr, prefix.len + own.len};
     const int nw = fast_waves(b * h, sq);
     const bool exact = exact_softmax(prefix, own, false);
@@ -1137,7 +1137,7 @@ hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64
                     launch_fast<8, false, false, 3>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream, sp);
                 else
                     launch_fast<8, true, false>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream, sp);
-                return finish_q8k(out_qblk, false, outf, b, h, sq, out, stream);
+                return finish_q8k(out_qblk, rounded, outf, b, h, sq, out, stream);
             }
         }
     if (!rows16(s0) || !rows16(s1)) {
@@ -1149,7 +1149,7 @@ hipError_t launch(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64
         launch_fast<4, false, false, 3>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
     } else if (exact) {
         launch_fast<8, false, false, 3>(q, s0, s1, h, sq, b, sl2, out, f32out, km, nullptr, sb, q8, stream);
-    } else if (pair) {
+    } else if (pair && !round_later) {
         launch_fast<8, true, false, 0, true>(q, s0, s1, h, sq, b, sl2, out, outf, km, nullptr, sb, 0, stream);
         rounded = true;
     } else if (nw == 4) {
@@ -1179,12 +1179,12 @@ hipError_t launch_attention(const uint16_t *q, KeySeg prefix, KeySeg own, int64_
 hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
                                    float sl2, const int32_t *img, const uint8_t *kvalid, int32_t *lim_scratch,
                                    uint16_t *out, hipStream_t stream, float *outf, const float *k_prefix_norm,
-                                   float q_norm, float k_own_norm, int out_qblk, float *scratch) {
+                                   float q_norm, float k_own_norm, int out_qblk, float *scratch, bool round_later) {
     if (sq <= 0 || b <= 0 || h <= 0) return hipSuccess;
     Seg s0, s1;
     if (!segments(prefix, own, s0, s1) || !out_qblk_ok(out_qblk, outf)) return hipErrorInvalidValue;
-    const int out_q8 = out_qblk == 32;
-    if (out_qblk == 32) outf = nullptr;
+    const int out_q8 = out_qblk == 32 && !round_later;
+    if (out_q8) outf = nullptr;
     if (img && (prefix.len != 0 || own.len != sq)) return hipErrorInvalidValue;  // block-causal: one shared sequence
     const KeyMask km{img, kvalid, prefix.len + own.len};
     // the last visible key of each query (none known: every window is classified)
@@ -1215,14 +1215,14 @@ hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own,
     } else
         launch_masked<false>(q, s0, s1, h, sq, b, sl2, out, outf, km, lim, sb, out_q8, stream,
                              KeySplit{0, 1, nullptr, nullptr});
-    return finish_q8k(out_qblk, false, outf, b, h, sq, out, stream);
+    return finish_q8k(out_qblk, round_later, outf, b, h, sq, out, stream);
 }
 
 hipError_t launch_attention_log2(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
                                  uint16_t *out, hipStream_t stream, float *outf, const float *k_prefix_norm,
-                                 float q_norm, float k_own_norm, int out_qblk, float *scratch) {
+                                 float q_norm, float k_own_norm, int out_qblk, float *scratch, bool round_later) {
     return launch<true>(q, prefix, own, b, h, sq, 1.0f, out, outf,
-                        ScoreBound{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm, k_own_norm}, out_qblk, stream, scratch);
+                        ScoreBound{prefix.len > 0 ? k_prefix_norm : nullptr, q_norm, k_own_norm}, out_qblk, stream, scratch, round_later);
 }
 
 }  // namespace qimm

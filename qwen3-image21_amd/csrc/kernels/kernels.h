@@ -62,6 +62,9 @@ struct EpiParams {
     // every other path writes the f32 state to hmid_f32 (which must be set)
     // and rounds it in its own pass. Needs (N / 2) % 32 == 0.
     int hmid_q8_0 = 0;
+    // with either: the work divided as for that rounding, but the state left in
+    // hmid_f32 as it is (the caller rounds it in a pass: the reference form)
+    int hmid_round_later = 0;
     // f32 scratch of part_ws_bytes for the short-M split-K path (optional;
     // without it short M takes the 128x128 kernel)
     float *part_ws = nullptr;
@@ -221,7 +224,9 @@ inline int64_t vt_ld(int64_t len) { return (len + 7) & ~(int64_t)7; }
 // (32 values) / Q8_K (256 values) block (quant_act4's arithmetic), the to_out
 // input in the candle mode: Q8_0 in the kernels' epilogue; Q8_K by the paired
 // cached-step kernel where it runs (an even head count), else through outf
-// (then required, f32 scratch) and the rows quantizer.
+// (then required, f32 scratch) and the rows quantizer. round_later: the work divided
+// as for that rounding, but the f32 output left in outf (the caller rounds it in a
+// pass: the reference form).
 hipError_t launch_attention(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
                             float scale, uint16_t *out, hipStream_t stream, float *outf = nullptr);
 // Masked attention (build_block_causal_mask semantics): img [sq] image block
@@ -234,13 +239,13 @@ hipError_t launch_attention_masked(const uint16_t *q, KeySeg prefix, KeySeg own,
                                    float sl2, const int32_t *img, const uint8_t *kvalid, int32_t *lim_scratch,
                                    uint16_t *out, hipStream_t stream, float *outf = nullptr,
                                    const float *k_prefix_norm = nullptr, float q_norm = 0.f, float k_own_norm = 0.f,
-                                   int out_qblk = 0, float *scratch = nullptr);
+                                   int out_qblk = 0, float *scratch = nullptr, bool round_later = false);
 // The same with q already multiplied by scale * log2(e) (the QKV epilogue's
 // q_scale), so scores are in log2 units.
 hipError_t launch_attention_log2(const uint16_t *q, KeySeg prefix, KeySeg own, int64_t b, int64_t h, int64_t sq,
                                  uint16_t *out, hipStream_t stream, float *outf = nullptr,
                                  const float *k_prefix_norm = nullptr, float q_norm = 0.f, float k_own_norm = 0.f,
-                                 int out_qblk = 0, float *scratch = nullptr);
+                                 int out_qblk = 0, float *scratch = nullptr, bool round_later = false);
 // scratch (attention_scratch_bytes, may be null) lets both launches split the
 // last, partial round of query tiles over the keys.
 size_t attention_scratch_bytes(int64_t bh, int64_t sq);

@@ -773,12 +773,12 @@ hipError_t launch_qgemm(const GemmWeight &w, const uint16_t *a, int64_t m, int64
         default: return launch_qgemm_large(w, a, m, lda, epi, e, stream);
         }
     };
-    if (!rounding || r.rounds) return run(ep);
+    if (!rounding || (r.rounds && !ep.hmid_round_later)) return run(ep);
     // the f32 hidden state, then the rows quantizer
     EpiParams e = ep;
     e.hmid_q8k = e.hmid_q8_0 = 0;
     const hipError_t err = run(e);
-    if (err != hipSuccess) return err;
+    if (err != hipSuccess || ep.hmid_round_later) return err;
     return launch_quant_rows(ep.hmid_f32, ep.ldh, m, w.n / 2, rounding, ep.hmid, ep.ldh, stream);
 }
 

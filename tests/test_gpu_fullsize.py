@@ -144,7 +144,7 @@ def _tied_gate_up(w, mlp):
     w["gate_up"] = (t, d.reshape(-1), rows, cols)
 
 
-@pytest.mark.parametrize("case", ["1024x1024", "ragged_ties"])
+@pytest.mark.parametrize("case", ["1024x1024", "ragged_ties", "eight_row_tail"])
 def test_hidden_rounding_in_gate_up_epilogue_bit_identical(torch_cuda, qctx, monkeypatch, case):
     """The candle-mode Q8_K rounding of the SwiGLU hidden state, done by the
     large-M gate_up kernel's epilogue (one workgroup per pair of 256-row tiles,
@@ -153,11 +153,14 @@ def test_hidden_rounding_in_gate_up_epilogue_bit_identical(torch_cuda, qctx, mon
     outputs. Cases: the 1024^2 Q4_K_M block (4096 tokens, MLP 12288: 16 token
     tiles x 48 tile pairs), and hidden 1024 / MLP 4096 at 1100 tokens (a last
     token tile of 76 rows) with every block's largest magnitude tied four times
-    across both tiles and both wave groups, opposite signs included."""
+    across both tiles and both wave groups, opposite signs included; and the same
+    MLP at 2056 tokens, where the rounding form hands its last 8 rows to the
+    streaming kernel (exact Q4_K weights) and the plain form would not: the
+    reference divides the rows as the form it stands for."""
     if case == "1024x1024":
         cfg, b, s, p = CFG4, 1, 4096, 256
     else:
-        cfg, b, s, p = dict(hidden=1024, heads=8, head_dim=128, mlp=4096), 1, 1100, 64
+        cfg, b, s, p = dict(hidden=1024, heads=8, head_dim=128, mlp=4096), 1, 1100 if case == "ragged_ties" else 2056, 64
     print(f"case: {case}, hidden {cfg['hidden']}, MLP {cfg['mlp']}, {s} tokens", flush=True)
     w, x, mod, pe, kpre, vpre = make_case(21, cfg, b, s, p, synth.Q4_K, synth.Q6_K)
     if case == "ragged_ties":
@@ -187,7 +190,7 @@ def _tied_heads(w, kpre, vpre, heads):
     vpre[:, 1::2] = vpre[:, 0::2] ^ np.uint16(0x8000)
 
 
-@pytest.mark.parametrize("case", ["heads_tied"])
+@pytest.mark.parametrize("case", ["heads_tied", "split_over_keys", "odd_prefix"])
 def test_attention_q8k_pair_rounding_bit_identical(torch_cuda, qctx, monkeypatch, case):
     """The candle-mode Q8_K rounding of the attention output (to_out's input,
     256 values = two heads of a query), done by the paired cached-step attention
@@ -196,10 +199,17 @@ def test_attention_q8k_pair_rounding_bit_identical(torch_cuda, qctx, monkeypatch
     bit-identical block outputs, with the pair's maxima tied across the two
     heads with opposite signs in every query (the first head must win). Hidden
     4096, 32 heads, 2048 tokens over 256: the 8-wave form. The 1024^2 case of
-    the gate_up test above covers the untied full size."""
-    cfg, b, s, p = dict(hidden=4096, heads=32, head_dim=128, mlp=4096), 1, 2048, 256
+    the gate_up test above covers the untied full size. 8 heads at 5392 tokens: in
+    place of the paired kernel the last round of query tiles is split over the
+    keys, which would not pay without the rounding; and 2048 tokens over a prefix
+    of 251 keys, which has no paired kernel. The reference divides the work alike
+    in both."""
+    cfg, b, s, p = dict(hidden=4096, heads=32, head_dim=128, mlp=4096), 1, 2048, 251 if case == "odd_prefix" else 256
+    if case == "split_over_keys":
+        cfg, s, p = dict(hidden=1024, heads=8, head_dim=128, mlp=1024), 5392, 64
     w, x, mod, pe, kpre, vpre = make_case(23, cfg, b, s, p, synth.Q4_K, synth.Q6_K)
-    _tied_heads(w, kpre, vpre, cfg["heads"])
+    if case == "heads_tied":
+        _tied_heads(w, kpre, vpre, cfg["heads"])
     fused, _ = run_block(torch_cuda, qctx, cfg, w, x, mod, pe, kpre, vpre)
     monkeypatch.setenv("QIMM_SEPARATE_ROUNDING", "1")
     separate, _ = run_block(torch_cuda, qctx, cfg, w, x, mod, pe, kpre, vpre)
