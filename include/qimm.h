@@ -81,14 +81,24 @@ int qimm_stream_synchronize(qimm_ctx *ctx, void *stream);
 
 /* ---------------- quantized weights ---------------- */
 
+/* Whether the weights uploaded through ctx from here on (by themselves or with a
+ * block or a model) keep their values as bf16 rows beside the codes: 2 bytes a
+ * value, for which the products of many tokens run 1.1 to 1.5 times faster (f32
+ * sums in another order). AUTO, the default, keeps them as long as at least half
+ * of the device memory stays free; NEVER leaves the memory to the caller; ALWAYS
+ * fails the upload (QIMM_ERR_OOM) where they do not fit. With NEVER or ALWAYS the
+ * kernels that a weight takes do not depend on what else is on the device. No
+ * counterpart in the reference. */
+typedef enum { QIMM_BF16_ROWS_AUTO = 0, QIMM_BF16_ROWS_NEVER = 1, QIMM_BF16_ROWS_ALWAYS = 2 } qimm_bf16_rows;
+int qimm_ctx_set_bf16_rows(qimm_ctx *ctx, int mode);
+
 /* Upload one GGUF tensor [rows = out features, cols = in features], GGML
  * blocks running along cols, exactly as candle's quantized VarBuilder hands
  * it to QMatMul::from_arc (src/quantized_transformer.rs:31-33). bytes must be
  * rows * cols / block_size * block_bytes. The library owns the device copy
  * and may re-stride blocks for aligned loads; values are never changed. Beside
- * the blocks of a quantized tensor it keeps their values as bf16 rows (2 bytes
- * a value) for the products of many tokens, as long as at least half of the
- * device memory stays free; qimm_weight_device_bytes counts both. */
+ * the blocks of a quantized tensor it may keep their values as bf16 rows
+ * (qimm_ctx_set_bf16_rows); qimm_weight_device_bytes counts both. */
 int qimm_weight_upload(qimm_ctx *ctx, int ggml_type, int64_t rows, int64_t cols,
                        const void *host_bytes, size_t nbytes, qimm_weight **out);
 int qimm_weight_free(qimm_weight *w);

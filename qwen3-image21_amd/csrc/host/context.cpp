@@ -108,6 +108,14 @@ int qimm_ctx_destroy(qimm_ctx *ctx) {
     return QIMM_OK;
 }
 
+int qimm_ctx_set_bf16_rows(qimm_ctx *ctx, int mode) {
+    if (!ctx) return QIMM_ERR_ARG;
+    if (mode != QIMM_BF16_ROWS_AUTO && mode != QIMM_BF16_ROWS_NEVER && mode != QIMM_BF16_ROWS_ALWAYS)
+        return set_err(ctx, QIMM_ERR_ARG, "bf16 rows: unknown mode");
+    ctx->bf16_rows = mode;
+    return QIMM_OK;
+}
+
 const char *qimm_last_error(const qimm_ctx *ctx) {
     if (!ctx) return "null context";
     return ctx->err.c_str();

@@ -19,6 +19,7 @@ struct qimm_ctx {
     // Growable f32 scratch for the split-K partial sums of the short-M GEMM.
     void *ws_part = nullptr;
     size_t ws_part_bytes = 0;
+    int bf16_rows = QIMM_BF16_ROWS_AUTO;  // of the weights uploaded next
 };
 
 struct qimm_weight {

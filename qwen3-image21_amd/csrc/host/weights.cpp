@@ -62,20 +62,24 @@ static inline float f16_to_f32(uint16_t h) {
 // the products of many tokens: a matrix kernel over bf16 rows runs 1.38-1.52
 // PFLOP/s, one that decodes beside its MFMAs 1.10-1.18, while a few tokens are
 // bound by the weight bytes and keep reading the codes. The copy takes 2 bytes
-// a value (a 32-layer model of hidden 4096: 14 GB of the card's 288), and is
-// made only while at least half of the device memory stays free after it;
-// without it (or if its allocation fails) the decoding kernels take every size.
-void keep_bf16_rows(qimm_weight *w) {
+// a value (a 32-layer model of hidden 4096: 14 GB of the card's 288); unless the
+// context says otherwise it is made only while at least half of the device memory
+// stays free after it, and without it (or if its allocation fails) the decoding
+// kernels take every size.
+hipError_t keep_bf16_rows(qimm_weight *w) {
     if (w->gw.fmt == qimm::WF_BF16) {
         w->gw.bf16 = (const uint16_t *)w->dev;
-        return;
+        return hipSuccess;
     }
-    if (w->rows % 256 || w->cols % 128) return;  // shapes its kernel does not take
+    const int mode = w->ctx->bf16_rows;
+    // rows % 256, cols % 128: shapes its kernel does not take
+    if (mode == QIMM_BF16_ROWS_NEVER || w->rows % 256 || w->cols % 128) return hipSuccess;
     const size_t bytes = (size_t)w->rows * (size_t)w->cols * 2;
     size_t avail = 0, total = 0;
-    if (hipMemGetInfo(&avail, &total) != hipSuccess || avail < bytes || avail - bytes < total / 2) {
+    if (mode == QIMM_BF16_ROWS_AUTO &&
+        (hipMemGetInfo(&avail, &total) != hipSuccess || avail < bytes || avail - bytes < total / 2)) {
         (void)hipGetLastError();
-        return;
+        return hipSuccess;
     }
     hipError_t e = hipMalloc(&w->dev_bf16, bytes);
     if (e == hipSuccess) e = qimm::launch_weight_rows_bf16(w->gw, (uint16_t *)w->dev_bf16, nullptr);
@@ -84,10 +88,11 @@ void keep_bf16_rows(qimm_weight *w) {
         (void)hipGetLastError();
         if (w->dev_bf16) (void)hipFree(w->dev_bf16);
         w->dev_bf16 = nullptr;
-        return;
+        return mode == QIMM_BF16_ROWS_ALWAYS ? e : hipSuccess;
     }
     w->gw.bf16 = (const uint16_t *)w->dev_bf16;
     w->dev_bytes += bytes;
+    return hipSuccess;
 }
 
 // Re-lay one tensor (rows of GGUF blocks) into the device format the GEMM
@@ -190,7 +195,10 @@ int upload_weight_rows(qimm_ctx *ctx, int type, int64_t rows, int64_t cols, cons
     w->gw.k = cols;
     w->gw.q = (const uint8_t *)w->dev;
     w->gw.scales = (const uint16_t *)w->dev_scales;
-    keep_bf16_rows(w);
+    if (const hipError_t kept = keep_bf16_rows(w); kept != hipSuccess) {
+        qimm_weight_free(w);
+        return hip_err(ctx, kept, "weight upload: bf16 rows");
+    }
     *out = w;
     return QIMM_OK;
 }

@@ -35,6 +35,7 @@ SIGNATURES = [
     ("qimm_status_string", C.c_char_p, [_i32]),
     ("qimm_ctx_create", _i32, [_i32, C.POINTER(_vp)]),
     ("qimm_ctx_destroy", _i32, [_vp]),
+    ("qimm_ctx_set_bf16_rows", _i32, [_vp, _i32]),
     ("qimm_last_error", C.c_char_p, [_vp]),
     ("qimm_malloc", _i32, [_vp, C.c_size_t, C.POINTER(_vp)]),
     ("qimm_free", _i32, [_vp, _vp]),
@@ -145,6 +146,8 @@ class GemmRoute(C.Structure):
                 ("scratch", _i64)]
 
 
+# qimm_bf16_rows
+BF16_ROWS_AUTO, BF16_ROWS_NEVER, BF16_ROWS_ALWAYS = 0, 1, 2
 # qimm_gemm_kernel
 GEMM_STREAM, GEMM_128, GEMM_LARGE, GEMM_WIDE, GEMM_BF16_ROWS = 1, 2, 3, 4, 5
 
@@ -206,6 +209,10 @@ class Context:
         if rc != OK:
             msg = self.lib.qimm_last_error(self.h)
             raise QimmError(f"{what} -> {status_name(rc)}: {msg.decode() if msg else ''}")
+
+    def set_bf16_rows(self, mode: int):
+        """Whether weights uploaded from here on keep bf16 rows (BF16_ROWS_AUTO / NEVER / ALWAYS)."""
+        self.check(self.lib.qimm_ctx_set_bf16_rows(self.h, mode), "qimm_ctx_set_bf16_rows")
 
     def close(self):
         if getattr(self, "h", None):

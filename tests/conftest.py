@@ -30,3 +30,15 @@ def qctx(torch_cuda):
     yield ctx
     torch_cuda.cuda.synchronize()
     ctx.close()
+
+
+@pytest.fixture(scope="session")
+def qctx_codes(torch_cuda):
+    """A context whose quantized weights keep their codes alone: the decoding kernels take
+    every product, as on a card without room for bf16 rows."""
+    import qimm
+    ctx = qimm.Context(0)
+    ctx.set_bf16_rows(qimm.BF16_ROWS_NEVER)
+    yield ctx
+    torch_cuda.cuda.synchronize()
+    ctx.close()

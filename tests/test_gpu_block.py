@@ -74,11 +74,14 @@ def run_modes(torch, qctx, cfg, w, x, mod, pe, kpre=None, vpre=None, alias=False
                  for act in (qimm.ACT_CANDLE, qimm.ACT_BF16))
 
 
-def check_modes(cfg, w, x, mod, pe, kpre, vpre, runs, want_kv=False):
+def oracle_modes(cfg, w, x, mod, pe, kpre, vpre):
+    return tuple(O.block_forward(cfg, w, x, mod, pe, kpre, vpre, mode=m) for m in (O.CANDLE, O.EXACT))
+
+
+def check_modes(cfg, w, x, mod, pe, kpre, vpre, runs, want_kv=False, refs=None):
     """Both modes' outputs (and own k / v) against the oracle's matching modes."""
     (got_c, kv_c), (got_b, kv_b) = runs
-    ref, kr, vr = O.block_forward(cfg, w, x, mod, pe, kpre, vpre, mode=O.CANDLE)
-    ref_e, kre, vre = O.block_forward(cfg, w, x, mod, pe, kpre, vpre, mode=O.EXACT)
+    (ref, kr, vr), (ref_e, kre, vre) = refs or oracle_modes(cfg, w, x, mod, pe, kpre, vpre)
     hid = cfg["hidden"]
     check_block(*(a.reshape(-1, hid) for a in (got_c, got_b, ref, ref_e, x)))
     if want_kv:
@@ -339,32 +342,48 @@ def test_block_hidden4096_short_m(torch_cuda, qctx, b, s, p, mlp):
 @pytest.mark.parametrize("b,s,p,mlp,attn_type,down_type", [
     (1, 1028, 16, 1024, synth.Q4_K, synth.Q6_K),  # a 4-row last tile row
     (2, 520, 8, 1024, synth.Q4_K, synth.Q6_K),    # batch boundary inside the third 256-row tile
+    (2, 523, 8, 1024, synth.Q8_0, synth.Q8_0),    # V^T rows of 523 tokens, stored 528 apart
+    (1, 2100, 0, 384, synth.Q8_0, synth.Q8_0),    # down over K = 384, half a super-block over
     (1, 1024, 0, 2048, synth.Q8_0, synth.Q8_0),   # four full tile rows, no prefix
     (1, 2820, 0, 4096, synth.Q4_K, synth.Q6_K)])  # out, gate_up and down on 256 x 256 tiles too
-def test_block_hidden4096_large_m(torch_cuda, qctx, b, s, p, mlp, attn_type, down_type):
-    """Hidden 4096 (32 heads) at M >= 1024 tokens, where the q/k/v projection
-    has enough 256 x 256 tiles for the large-M GEMM: its fused q/k/v epilogue
-    over 32 heads (head = column / 128 across 48 column tiles, V written
-    transposed) and the XCD-aware tile order, with partial tiles and a batch
-    boundary inside a tile; at 2820 tokens (12 tile rows) also its residual
-    (out, Q6_K down) and SwiGLU epilogues, on a 4-row last tile row. The
-    products with fewer tiles take the 128 x 128 kernel. Output, k and v against
-    both oracle modes. Short MLPs keep the oracle quick."""
+def test_block_hidden4096_large_m(torch_cuda, qctx, qctx_codes, b, s, p, mlp, attn_type, down_type):
+    """Hidden 4096 (32 heads) at M >= 1024 tokens, over bf16 rows and with the
+    codes alone, where the q/k/v projection has enough 256 x 256 tiles for the
+    decoding large-M kernel: the fused q/k/v epilogues over 32 heads (head =
+    column / 128 across 48 column tiles, V written transposed) and the XCD-aware
+    tile order, with partial tiles and a batch boundary inside a tile; at 2820
+    tokens (12 tile rows) also the residual (out, Q6_K down) and SwiGLU
+    epilogues, on a 4-row last tile row; at 2100 tokens the four-wave kernel's
+    residual epilogue for the codes alone. Output, k and v against both oracle
+    modes. Short MLPs keep the oracle quick."""
     cfg = dict(hidden=4096, heads=32, head_dim=128, mlp=mlp)
+    cus, m = torch_cuda.cuda.get_device_properties(0).multi_processor_count, b * s
+    assert qimm.qmatmul_route(attn_type, 12288, 4096, m, cus).kernel == qimm.GEMM_BF16_ROWS
+    assert qimm.qmatmul_route(attn_type, 12288, 4096, m, cus, False).kernel == qimm.GEMM_WIDE
+    if m > 2048:
+        large = qimm.GEMM_WIDE if mlp % 256 == 0 else qimm.GEMM_LARGE
+        assert qimm.qmatmul_route(down_type, 4096, mlp, m, cus, False).kernel == large
     w, x, mod, pe, kpre, vpre = make_case(61 + b + s, cfg, b, s, p, attn_type, down_type)
-    runs = run_modes(torch_cuda, qctx, cfg, w, x, mod, pe, kpre, vpre, want_kv=True)
-    check_modes(cfg, w, x, mod, pe, kpre, vpre, runs, want_kv=True)
+    refs = oracle_modes(cfg, w, x, mod, pe, kpre, vpre)
+    for ctx in (qctx, qctx_codes):
+        runs = run_modes(torch_cuda, ctx, cfg, w, x, mod, pe, kpre, vpre, want_kv=True)
+        check_modes(cfg, w, x, mod, pe, kpre, vpre, runs, want_kv=True, refs=refs)
 
 
-def test_block_hidden4096_large_m_bf16_weights(torch_cuda, qctx):
-    """Float-stored (bf16) weights at 2820 tokens, hidden 4096, MLP 4096: the
-    large-M GEMM's bf16 form, whose weight tile goes global -> LDS by direct
-    loads like the activations, under its fused q/k/v, residual and SwiGLU
-    epilogues (12 tile rows, a 4-row last one). Candle multiplies float-stored
-    weights in plain f32 (no int8 activations), so exact mode alone is the
-    reference here."""
-    cfg = dict(hidden=4096, heads=32, head_dim=128, mlp=4096)
-    b, s, p = 1, 2820, 0
+@pytest.mark.parametrize("s,mlp", [(2820, 4096), (2100, 192)])
+def test_block_hidden4096_large_m_bf16_weights(torch_cuda, qctx, s, mlp):
+    """Float-stored (bf16) weights, hidden 4096: the kernel over bf16 rows under
+    its fused q/k/v, residual and SwiGLU epilogues (2820 tokens, MLP 4096: 12 tile
+    rows, a 4-row last one), and the down projection of an MLP of 192 (an odd
+    number of 64-k steps) in the four-wave kernel's bf16 form, whose weight tile
+    goes global -> LDS by direct loads like the activations. Candle multiplies
+    float-stored weights in plain f32 (no int8 activations), so exact mode alone
+    is the reference here."""
+    cfg = dict(hidden=4096, heads=32, head_dim=128, mlp=mlp)
+    cus = torch_cuda.cuda.get_device_properties(0).multi_processor_count
+    down = qimm.qmatmul_route(synth.BF16, 4096, mlp, s, cus).kernel
+    assert down == (qimm.GEMM_BF16_ROWS if mlp % 128 == 0 else qimm.GEMM_LARGE)
+    b, p = 1, 0
     w, x, mod, pe, kpre, vpre = make_case(67, cfg, b, s, p, synth.BF16, synth.BF16)
     got, (k, v) = run_block(torch_cuda, qctx, cfg, w, x, mod, pe, kpre, vpre, want_kv=True)
     ref_e, kre, vre = O.block_forward(cfg, w, x, mod, pe, kpre, vpre, mode=O.EXACT)
@@ -448,16 +467,20 @@ def test_block_reserve_covers_smaller_forwards(torch_cuda):
 
 
 @pytest.mark.parametrize("case", ["config1_128x128", "wide_ragged", "two_k_shares"])
-def test_hidden_q8_0_rounding_in_gate_up_epilogue_bit_identical(torch_cuda, qctx, monkeypatch, case):
+@pytest.mark.parametrize("rows_kept", [True, False])
+def test_hidden_q8_0_rounding_in_gate_up_epilogue_bit_identical(torch_cuda, qctx, qctx_codes, monkeypatch, case, rows_kept):
     """Q8_0 down weights in candle mode: the Q8_0 rounding of the SwiGLU hidden
     state (the down projection's input, one scale per 32 columns of a token row)
     done by the gate_up kernel's epilogue against the same rounding as the
     rows-quantizer pass (QIMM_SEPARATE_ROUNDING=1): bit-identical block outputs.
-    Cases: config 1 (MLP 9216 at 256 tokens over 64: the undivided 128x128
-    kernel, four lanes per block), hidden 1024 / MLP 4096 at 1100 tokens (the
-    256x256 kernel, two waves per block, a last token tile of 76 rows), and the
-    same block at 256 tokens (two K shares: the f32 state and the rows quantizer
-    on both sides)."""
+    Cases: config 1 (MLP 9216 at 256 tokens over 64), hidden 1024 / MLP 4096 at
+    1100 tokens (a last token tile of 76 rows), and the same block at 256 tokens
+    (two K shares: the f32 state and the rows quantizer on both sides); over bf16
+    rows, whose epilogue rounds a block across four lanes, and with the codes
+    alone: the undivided 128x128 kernel (four lanes per block) and the 256x256
+    kernel (two waves per block)."""
+    if not rows_kept:
+        qctx = qctx_codes
     if case == "config1_128x128":
         cfg, b, s, p = dict(hidden=3072, heads=24, head_dim=128, mlp=9216), 1, 256, 64
     else:

@@ -83,14 +83,15 @@ def test_block_1024_q4km_full_size(torch_cuda, qctx):
                                                      (synth.Q4_K, synth.Q6_K, 1, 4160),
                                                      (synth.Q8_0, synth.Q8_0, 1, 4102),
                                                      (synth.Q4_K, synth.Q6_K, 2, 2050)])
-def test_block_4352_tokens_tail_rows(torch_cuda, qctx, attn_type, down_type, b, s):
+def test_block_4352_tokens_tail_rows(torch_cuda, qctx, qctx_codes, attn_type, down_type, b, s):
     """4352 token rows at hidden 4096 (17 rows of 256x256 tiles): q/k/v makes
     816 tiles and out and down 272 for 256 CUs, so their last 256 token rows
     run as a 256-token product of their own (the 128x128 or split path; the
     gated residual on rows shifted by 4096, the q/k/v outputs, V^T and RoPE rows
     shifted to the tail's sequence and position: sequence 0 from position 4096,
     or with two sequences of 2176 tokens sequence 1 from position 1920), the
-    rest as whole rounds; with 4160 tokens the last 64 rows take the short-M
+    rest as whole rounds; over bf16 rows the tails come from the same counts of
+    256-token tiles, and both are run; with 4160 tokens the last 64 rows take the short-M
     kernels (the gated residual and the f32 hidden state with its rows pass;
     q/k/v keeps them; with 4102 tokens, a token count that is not a multiple of
     the LayerNorm's four rows per workgroup, its last workgroup repeats the last
@@ -103,19 +104,23 @@ def test_block_4352_tokens_tail_rows(torch_cuda, qctx, attn_type, down_type, b, 
     m = b * s
     print(f"case: block hidden 4096, {b} x {s} tokens over {p}, types {attn_type}/{down_type}", flush=True)
     w, x, mod, pe, kpre, vpre = make_case(6, CFG4, b, s, p, attn_type, down_type)
-    got, (k, v) = run_block(torch_cuda, qctx, CFG4, w, x, mod, pe, kpre, vpre, want_kv=True)
-    assert np.isfinite(got).all()
+    cus = torch_cuda.cuda.get_device_properties(0).multi_processor_count
+    for rows_kept in (True, False):
+        assert qimm.qmatmul_route(attn_type, 4096, 4096, m, cus, rows_kept).tail == m - 4096
+    runs = [run_block(torch_cuda, ctx, CFG4, w, x, mod, pe, kpre, vpre, want_kv=True) for ctx in (qctx, qctx_codes)]
     rng = np.random.default_rng(41)
     seam = np.arange(s - 4, s + 4) if b > 1 else np.arange(0)
     rows = np.unique(np.concatenate([sampled_rows(rng, m), rng.choice(np.arange(4096, m), min(48, m - 4096), replace=False),
                                      seam]))
     ref, kr, vr = O.block_forward_rows(CFG4, w, x, mod, pe, rows, kpre, vpre, mode=O.CANDLE)
-    g = got.reshape(m, -1)[rows]
-    c, mr = cos_sim(g, ref), max_abs_rel(g, ref)
-    print(f"sampled rows: cos {c:.7f} mar {mr:.2e}", flush=True)
-    assert c >= 0.9999 and mr <= 2e-2
-    kv_close(k, kr)
-    kv_close(v, vr)
+    for got, (k, v) in runs:
+        assert np.isfinite(got).all()
+        g = got.reshape(m, -1)[rows]
+        c, mr = cos_sim(g, ref), max_abs_rel(g, ref)
+        print(f"sampled rows: cos {c:.7f} mar {mr:.2e}", flush=True)
+        assert c >= 0.9999 and mr <= 2e-2
+        kv_close(k, kr)
+        kv_close(v, vr)
 
 
 def _q4k_negated(rows):
@@ -145,10 +150,12 @@ def _tied_gate_up(w, mlp):
 
 
 @pytest.mark.parametrize("case", ["1024x1024", "ragged_ties", "eight_row_tail"])
-def test_hidden_rounding_in_gate_up_epilogue_bit_identical(torch_cuda, qctx, monkeypatch, case):
+@pytest.mark.parametrize("rows_kept", [True, False])
+def test_hidden_rounding_in_gate_up_epilogue_bit_identical(torch_cuda, qctx, qctx_codes, monkeypatch, case, rows_kept):
     """The candle-mode Q8_K rounding of the SwiGLU hidden state, done by the
-    large-M gate_up kernel's epilogue (one workgroup per pair of 256-row tiles,
-    the 256 hidden columns of a Q8_K block), against the same rounding as its
+    large-M gate_up kernel's epilogue (over bf16 rows tiles of 512 weight rows,
+    with the codes alone one workgroup per pair of 256-row tiles: the 256 hidden
+    columns of a Q8_K block), against the same rounding as its
     own pass after the GEMM (QIMM_SEPARATE_ROUNDING=1): bit-identical block
     outputs. Cases: the 1024^2 Q4_K_M block (4096 tokens, MLP 12288: 16 token
     tiles x 48 tile pairs), and hidden 1024 / MLP 4096 at 1100 tokens (a last
@@ -161,6 +168,8 @@ def test_hidden_rounding_in_gate_up_epilogue_bit_identical(torch_cuda, qctx, mon
         cfg, b, s, p = CFG4, 1, 4096, 256
     else:
         cfg, b, s, p = dict(hidden=1024, heads=8, head_dim=128, mlp=4096), 1, 1100 if case == "ragged_ties" else 2056, 64
+    if not rows_kept:
+        qctx = qctx_codes
     print(f"case: {case}, hidden {cfg['hidden']}, MLP {cfg['mlp']}, {s} tokens", flush=True)
     w, x, mod, pe, kpre, vpre = make_case(21, cfg, b, s, p, synth.Q4_K, synth.Q6_K)
     if case == "ragged_ties":

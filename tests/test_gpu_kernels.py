@@ -77,10 +77,8 @@ def _gemm_case(torch, qctx, t, m, n, k, seed, out_type=synth.F32, std=0.02):
                                    (16, 384, 4096), (33, 256, 1024), (64, 128, 8192),
                                    (130, 384, 1024), (300, 128, 4096),
                                    (600, 512, 1024), (1024, 256, 768),
-                                   # 256x256 kernels (more 128x128 tiles than two per CU): the
-                                   # eight-wave kernel for the quantized formats, one super-block and
-                                   # four (every Q6_K scale-pair and half position, negative scales);
-                                   # bf16 weights take the four-wave kernel's direct global->LDS path
+                                   # bf16 rows, one super-block and four (the values of every Q6_K
+                                   # scale-pair and half position, negative scales)
                                    (2304, 4096, 256), (2304, 4096, 1024)])
 def test_qmatmul_matches_bf16_weight_products(torch_cuda, qctx, t, m, n, k):
     """Products of the bf16 activations and the weights each path multiplies:
@@ -135,6 +133,58 @@ def test_qmatmul_bf16_rows(torch_cuda, qctx, t, m, n, k, route):
     scale = np.abs(a) @ np.abs(Wb).T
     assert np.isfinite(got).all()
     assert np.all(np.abs(got[rows] - a @ Wb.T) <= 2e-4 * scale + 1e-6)
+
+
+@pytest.mark.parametrize("t,m,n,k,kernel", [
+    # the eight-wave 256x256 kernel: one super-block and four
+    *[(t, 2304, 4096, k, qimm.GEMM_WIDE) for t in (synth.Q8_0, synth.Q4_K, synth.Q6_K) for k in (256, 1024)],
+    (synth.Q8_0, 2304, 4096, 384, qimm.GEMM_LARGE),  # half a super-block over: the four-wave kernel
+    (synth.Q8_0, 2304, 4096, 64, qimm.GEMM_LARGE),   # a single k step
+    (synth.BF16, 2304, 4096, 192, qimm.GEMM_LARGE),  # bf16 weights of an odd number of 64-k steps
+    *[(t, 600, 512, 1024, qimm.GEMM_128) for t in (synth.Q8_0, synth.Q4_K, synth.Q6_K)],
+])
+def test_qmatmul_codes_alone(torch_cuda, qctx_codes, t, m, n, k, kernel):
+    """Products of many rows without bf16 rows beside the codes: each decoding kernel against
+    the products of the bf16 activations and the bf16-rounded weights."""
+    cus = torch_cuda.cuda.get_device_properties(0).multi_processor_count
+    assert qimm.qmatmul_route(t, n, k, m, cus, bf16_rows=False).kernel == kernel
+    got, a, w = _gemm_case(torch_cuda, qctx_codes, t, m, n, k, seed=m + n + k + t)
+    Wb = O.bf16_round(O.dequantize(t, w, n * k).reshape(n, k)).astype(np.float64)
+    a = a.astype(np.float64)
+    assert np.all(np.abs(got - a @ Wb.T) <= 2e-4 * (np.abs(a) @ np.abs(Wb).T) + 1e-6)
+
+
+def test_bf16_rows_modes(torch_cuda):
+    """NEVER keeps the codes alone although there is room, ALWAYS keeps the rows with less than
+    half of the memory free, AUTO decides by the room: the bytes say which, and ALWAYS gives
+    AUTO's product with room bit for bit."""
+    torch = torch_cuda
+    m, n, k = 300, 512, 1024
+    rng = np.random.default_rng(78)
+    _, w, _, _ = synth.weight(rng, synth.Q4_K, n, k)
+    a_dev, _ = bf16_dev(torch, rng.standard_normal((m, k)).astype(np.float32))
+    ctx = qimm.Context(0)
+    with pytest.raises(qimm.QimmError, match="QIMM_ERR_ARG"):
+        ctx.set_bf16_rows(3)
+    sizes, ys = {}, {}
+    for mode, room in ((qimm.BF16_ROWS_AUTO, True), (qimm.BF16_ROWS_NEVER, True), (qimm.BF16_ROWS_ALWAYS, False)):
+        torch.cuda.empty_cache()
+        free, total = torch.cuda.mem_get_info()
+        hold = torch.empty(0 if room else max(free - total // 2 + (1 << 30), 0), dtype=torch.uint8, device="cuda")
+        ctx.set_bf16_rows(mode)
+        W = ctx.upload(synth.Q4_K, n, k, w.tobytes())
+        del hold
+        torch.cuda.empty_cache()
+        y = torch.empty((m, n), dtype=torch.float32, device="cuda")
+        ctx.qmatmul(W, a_dev.data_ptr(), m, k, y.data_ptr(), synth.F32, stream(torch))
+        sizes[mode], ys[mode] = W.device_bytes(), host(y)
+        W.free()
+    ctx.close()
+    codes = n * k // 256 * 144
+    assert sizes == {qimm.BF16_ROWS_AUTO: codes + 2 * n * k, qimm.BF16_ROWS_NEVER: codes,
+                     qimm.BF16_ROWS_ALWAYS: codes + 2 * n * k}
+    assert np.array_equal(ys[qimm.BF16_ROWS_AUTO], ys[qimm.BF16_ROWS_ALWAYS])
+    assert max_abs_rel(ys[qimm.BF16_ROWS_NEVER], ys[qimm.BF16_ROWS_AUTO]) <= 1e-5
 
 
 def test_no_room_for_bf16_rows(torch_cuda, qctx):
@@ -291,13 +341,19 @@ def test_qmatmul_full_qkv_shape_sampled_rows(torch_cuda, qctx):
 @pytest.mark.parametrize("m,n,k,t,out", [(4352, 4096, 4096, synth.Q4_K, synth.BF16),   # tail: split 128x128
                                          (4136, 4096, 4096, synth.Q4_K, synth.F32),    # tail: 40-row streaming
                                          (4352, 4096, 2048, synth.Q8_0, synth.BF16)])
-def test_qmatmul_large_m_tail_rows(torch_cuda, qctx, m, n, k, t, out):
+@pytest.mark.parametrize("rows_kept", [True, False])
+def test_qmatmul_large_m_tail_rows(torch_cuda, qctx, qctx_codes, m, n, k, t, out, rows_kept):
     """Large-M products whose last 256x256 tile row would run as a nearly empty
-    wave hand those rows to the shorter-M paths (plain outputs): sampled head
+    wave hand those rows to the shorter-M paths (plain outputs), over bf16 rows
+    and with the codes alone: sampled head
     rows and every tail row match the products of the bf16 activations and
     the weights each path multiplies (bf16-rounded, or exact on the Q4_K
     code-product path), and the seam rows are continuous."""
     torch = torch_cuda
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    r = qimm.qmatmul_route(t, n, k, m, cus, rows_kept)
+    assert r.kernel == (qimm.GEMM_BF16_ROWS if rows_kept else qimm.GEMM_WIDE) and r.tail == m - 4096
+    qctx = qctx if rows_kept else qctx_codes
     rng = np.random.default_rng(m + k + t)
     _, w, _, _ = synth.weight(rng, t, n, k)
     W = qctx.upload(t, n, k, w.tobytes())
