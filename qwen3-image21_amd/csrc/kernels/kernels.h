@@ -82,11 +82,12 @@ struct GemmWeight {
 };
 
 // y = A[M,K] (bf16, row stride lda) x W[N,K]^T with the epilogue selected by epi.
-// Short M streams the weights (launch_qgemm_stream). Above it, weights with bf16
-// rows take launch_qgemm_bf16 or the 128x128 kernel, whichever is estimated
-// faster; without bf16 rows the 256x256 kernels take what qgemm_large_fits (at
-// least 512 rows, and more 128x128 tiles than one wave of two workgroups per
-// CU), the 128x128 kernel the rest.
+// Short M streams the weights (launch_qgemm_stream). Above it, the 128x128 kernel
+// takes what its two workgroups per CU hold in one wave or what is below 512 rows,
+// and launch_qgemm_bf16, for weights with bf16 rows, what it is estimated to do
+// faster; larger products (qgemm_large_fits) run over bf16 rows where there are
+// some (bf16-stored weights of short K in the four-wave 256x256 kernel), else in
+// the decoding 256x256 kernels.
 hipError_t launch_qgemm(const GemmWeight &w, const uint16_t *a, int64_t m, int64_t lda,
                         int epi, const EpiParams &ep, hipStream_t stream);
 // How launch_qgemm takes a product: the kernel (qimm_gemm_kernel's values), its shares

@@ -552,10 +552,18 @@ namespace {
 // kernel (whose cost estimate, fitted at 256 and 384 tokens, is 1.1 times short
 // above, for Q6_K 1.3 times: 4096 x 12288 at 300 / 512 / 1024 tokens 70 / 74 /
 // 130 us estimated, 83-88 / 97-103 / 180 measured). Below, few tokens are bound by the weight
-// bytes, and the 128x128 kernel reads the codes. splits 0: no.
+// bytes, and the 128x128 kernel reads the codes. Products that the 128x128 kernel
+// does not take (qgemm_large_fits): a quantized weight runs over its bf16 rows
+// whatever the estimates (against the decoding 256x256 kernels, K = 256: Q8_0 8192
+// x 256 at 8448 tokens 90 -> 72 us, Q4_K at 16384 146 -> 131; K = 128 at 4299 tokens
+// 41 -> 34), a bf16-stored one in the four-wave 256x256 kernel where the 128x128
+// kernel's estimate, which stands in for that kernel's, is the lower one: short K,
+// whose few steps do not pay for this kernel's longer prologue (12288 x 128 at 3072
+// tokens 33 us against 36, 12288 x 256 at 16384 177 against 210). splits 0: no.
 Bf16Plan bf16_plan(const GemmWeight &w, int64_t m, int64_t lda, bool may_split) {
     if (!qgemm_bf16_fits(w) || lda > ((int64_t)1 << 22) || qgemm_stream_fits(w, m)) return {0, 0, 0.0};
     const Bf16Plan p = qgemm_bf16_plan(w, m, may_split);
+    if (qgemm_large_fits(w, m) && w.fmt != WF_BF16) return p;
     const MidCost mid = mid_cost(w, m);
     const double mid_us = mid.us * (w.fmt == WF_Q6_K ? 1.3 : m > 384 ? 1.1 : 1.0);
     return mid_us > 0.0 && mid_us <= p.us ? Bf16Plan{0, 0, mid_us} : p;

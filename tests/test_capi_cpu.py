@@ -84,5 +84,10 @@ def test_qmatmul_route_codes():
     assert qimm.qmatmul_route(qimm.Q4_K, 4096, 4096, 16, 256).kernel == qimm.GEMM_STREAM
     assert qimm.qmatmul_route(qimm.Q4_K, 4096, 4096, 4352, 256).kernel == qimm.GEMM_BF16_ROWS
     assert qimm.qmatmul_route(qimm.Q4_K, 4096, 4096, 4352, 256, bf16_rows=False).kernel == qimm.GEMM_WIDE
+    # so do quantized weights of short K with rows: they are not left to the decoding kernels
+    for t, m, n, k in ((qimm.Q8_0, 3072, 12288, 128), (qimm.Q8_0, 8448, 8192, 256), (qimm.Q4_K, 16384, 8192, 256)):
+        assert qimm.qmatmul_route(t, n, k, m, 256).kernel == qimm.GEMM_BF16_ROWS
+    # bf16-stored ones take the four-wave kernel there
+    assert qimm.qmatmul_route(qimm.BF16, 12288, 128, 3072, 256).kernel == qimm.GEMM_LARGE
     # float weights are bf16 rows themselves
     assert qimm.qmatmul_route(qimm.BF16, 4096, 4096, 4352, 256, bf16_rows=False).kernel == qimm.GEMM_BF16_ROWS
