@@ -370,6 +370,19 @@ def test_block_hidden4096_large_m(torch_cuda, qctx, qctx_codes, b, s, p, mlp, at
         check_modes(cfg, w, x, mod, pe, kpre, vpre, runs, want_kv=True, refs=refs)
 
 
+def test_block_bf16_weights_hidden256_large_m(torch_cuda, qctx):
+    """Float-stored (bf16) weights, hidden 256, MLP 12288, 2112 tokens: gate_up (24576 x
+    256) in the four-wave kernel with its SwiGLU epilogue, a 64-row last tile row."""
+    cfg = dict(hidden=256, heads=2, head_dim=128, mlp=12288)
+    cus = torch_cuda.cuda.get_device_properties(0).multi_processor_count
+    assert qimm.qmatmul_route(synth.BF16, 24576, 256, 2112, cus).kernel == qimm.GEMM_LARGE
+    w, x, mod, pe, kpre, vpre = make_case(71, cfg, 1, 2112, 8, synth.BF16, synth.BF16)
+    got, _ = run_block(torch_cuda, qctx, cfg, w, x, mod, pe, kpre, vpre)
+    ref_e, _, _ = O.block_forward(cfg, w, x, mod, pe, kpre, vpre, mode=O.EXACT)
+    check(got, ref_e, x)
+    check(got, ref_e, x, exact=True)
+
+
 @pytest.mark.parametrize("s,mlp", [(2820, 4096), (2100, 192)])
 def test_block_hidden4096_large_m_bf16_weights(torch_cuda, qctx, s, mlp):
     """Float-stored (bf16) weights, hidden 4096: the kernel over bf16 rows under

@@ -112,6 +112,7 @@ BF16_ROWS_CASES = [
     (synth.Q4_K, 1025, 4096, 1024, (1, 0, 0)),   # nine tiles of 128, one token in the last
     (synth.Q4_K, 2049, 4096, 1024, (1, 9, 0)),   # tiles of 256 alone, one token in the last
     (synth.Q6_K, 4299, 4096, 256, (1, 2, 0)),    # both tile sizes in one launch
+    (synth.Q8_0, 3072, 12288, 128, (1, 8, 0)),   # two k steps in tiles of 256 too
     (synth.Q6_K, 4299, 4096, 4096, (1, 16, 203)),  # one full round, then a tail of its own
 ]
 
