@@ -644,12 +644,16 @@ Bf16Plan qgemm_bf16_plan(const GemmWeight &w, int64_t m, bool may_split) {
     // the time at which the last of n1 tiles of 256 tokens, then n2 of 128, ends
     auto span = [&](int64_t n1, int64_t n2) {
         const double c1 = round_us(steps, false, n1 + n2, cus), c2 = round_us(steps, true, n1 + n2, cus);
-        const int64_t late = n1 % cus;  // CUs that run one large tile more
+        const int64_t late = n1 % cus, early = cus - late;  // CUs that run one large tile more, the others
         const double t0 = (double)(n1 / cus) * c1, t1 = t0 + c1;
-        int64_t x = 0, y = 0;  // small tiles per early and per late CU
-        while (x * (cus - late) + y * late < n2) {
-            if (late == 0 || t0 + (double)(x + 1) * c2 <= t1 + (double)(y + 1) * c2) x++;
-            else y++;
+        // small tiles per early (x) and per late CU (y), each round where it ends first:
+        // the early ones take c1 / c2 rounds ahead, then the two in turn, late first
+        int64_t x = (n2 + early - 1) / early, y = 0;
+        const int64_t lead = late ? (int64_t)(c1 / c2) + 1 : x;
+        if (x > lead) {
+            const int64_t rest = n2 - lead * early, q = rest / cus, r = rest % cus;
+            y = q + (r > 0);
+            x = lead + q + (r > late);
         }
         return std::max(late ? t1 + (double)y * c2 : t0, t0 + (double)x * c2);
     };

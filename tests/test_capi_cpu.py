@@ -73,6 +73,56 @@ def test_bf16_rows_cases_take_the_paths_they_name(t, m, n, k, route):
     assert bf16_rows_route(t, m, n, k, 256) == (True, route)
 
 
+def test_plan_of_mixed_tiles_follows_the_rounds():
+    """The tiles of 256 tokens that the plan picks, against a plan that places the tiles round
+    by round (the estimate of qgemm_bf16.hip, 256 compute units): odd and large token counts,
+    few and many weight tiles."""
+    cus = 256
+
+    def round_us(steps, small, wgs):
+        f = min(1.0, wgs / cus)
+        return 6.0 + steps * (0.61 + 0.26 * f if small else 1.08 + 0.42 * f)
+
+    def span(steps, n1, n2):
+        c1, c2 = round_us(steps, False, n1 + n2), round_us(steps, True, n1 + n2)
+        late, t0 = n1 % cus, n1 // cus * c1
+        t1, x, y = t0 + c1, 0, 0
+        while x * (cus - late) + y * late < n2:
+            if late == 0 or t0 + (x + 1) * c2 <= t1 + (y + 1) * c2:
+                x += 1
+            else:
+                y += 1
+        return max(t1 + y * c2 if late else t0, t0 + x * c2)
+
+    for n, k in ((24576, 4096), (12288, 4096), (4096, 12288), (9216, 3072)):
+        for m in (2304, 2817, 3072, 3289, 4095, 4097, 4352, 5000, 6889, 8448, 9001, 13799):
+            full, nt, steps = (m + 255) // 256, n // 256, k // 64
+            best, us = full, span(steps, full * nt, 0)
+            for h in range(full):
+                t = span(steps, h * nt, (m - 256 * h + 127) // 128 * nt)
+                if t < us * 0.995:
+                    best, us = h, t
+            r = qimm.qmatmul_route(qimm.Q4_K if k != 12288 else qimm.Q6_K, n, k, m, cus)
+            assert r.kernel == qimm.GEMM_BF16_ROWS
+            if r.tail == 0:
+                assert r.large_tiles == best, (n, k, m)
+
+
+def test_plan_of_many_tokens_is_quick():
+    """A plan is made at each launch: its cost grows with the tokens at most (it used to place
+    every round of tiles, 9 ms at 200000 tokens)."""
+    import time
+    qimm.qmatmul_route(qimm.Q4_K, 24576, 4096, 4096, 256)
+    t = min(_timed(lambda: qimm.qmatmul_route(qimm.Q4_K, 24576, 4096, 200000, 256), time) for _ in range(5))
+    assert t < 1e-3, t
+
+
+def _timed(f, time):
+    t0 = time.perf_counter()
+    f()
+    return time.perf_counter() - t0
+
+
 def test_qmatmul_route_codes():
     lib = qimm.load()
     r = qimm.GemmRoute()
