@@ -574,6 +574,13 @@ size_t bf16_workspace(const GemmWeight &w, int64_t m, const Bf16Plan &p) {
 }
 // f32 rows rounded in a pass of their own, in us
 double quant_pass_us(const GemmWeight &w, int64_t m) { return 5.0 + (double)m * (double)(w.n / 2) * 6.0 / 4.5e6; }
+// a product of up to 64 rows in the streaming kernels, in us: 5 and the weight bytes
+// at 4.7 (16 rows) to 2.2 TB/s (64), Q6_K at three quarters of that (Q4_K 24576 x
+// 4096 at 16 / 64 rows 17 / 29 us, 4096 x 4096 at 16 7; Q6_K 4096 x 12288 18 / 27)
+double stream_us(const GemmWeight &w, int64_t m) {
+    const double bytes = w.fmt == WF_Q4_K ? 144.0 / 256 : w.fmt == WF_Q6_K ? 224.0 / 256 : w.fmt == WF_Q8_0 ? 34.0 / 32 : 2.0;
+    return 5.0 + (double)w.n * (double)w.k * bytes * 1e-6 * (0.13 + 0.005 * (double)m) * (w.fmt == WF_Q6_K ? 1.3 : 1.0);
+}
 // Rows of a bf16-rows product handed to a product of their own: those after the
 // last full round of 256-token tiles (4299 tokens x N = 4096: 256 tiles for 256
 // CUs, then 203 rows), where the two together are estimated faster. 0 = none.
@@ -584,7 +591,7 @@ int64_t bf16_tail_rows(const GemmWeight &w, int64_t m, int64_t lda, bool q8k, do
     const Bf16Plan ph = bf16_plan(w, 256 * h, lda, false), pt = bf16_plan(w, tail, lda, true);
     if (!ph.splits) return 0;
     const double head_us = q8k ? std::min(qgemm_bf16_q8k_us(w, 256 * h), ph.us + quant_pass_us(w, 256 * h)) : ph.us;
-    const double tail_us = pt.splits || pt.us > 0.0 ? pt.us + (q8k ? quant_pass_us(w, tail) : 0.0) : 25.0;
+    const double tail_us = (pt.splits || pt.us > 0.0 ? pt.us : stream_us(w, tail)) + (q8k ? quant_pass_us(w, tail) : 0.0);
     return head_us + tail_us + 3.0 < whole_us ? tail : 0;
 }
 
