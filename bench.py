@@ -169,7 +169,7 @@ def main():
         log("bench: no profiled steps, stage report skipped")
     else:
         log(f"bench: stage medians sum to {sum(stages.values()):.3f} ms (timed step {ms_step:.3f} ms)")
-        kernels, roofline = stage_report(stages, att_flop, synth)
+        kernels, roofline = stage_report(stages, att_flop, qimm, synth, compute_units(torch))
 
     block_flop = att_flop + 2.0 * S_IMG * HID * (3 * HID + HID + 2 * MLP) + 2.0 * S_IMG * MLP * HID
 
@@ -392,7 +392,18 @@ def stage_profile(blocks, step, nsteps, warm=8):
             for k, v in per.items()}
 
 
-def stage_report(stages, att_flop, synth):
+def compute_units(torch):
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
+def weight_read(qimm, synth, t, n, k, m, cus):
+    """The bytes of a weight that the product of m rows reads once, and the kernel that reads
+    them: the bf16 rows an upload keeps (2 bytes a value, with room on the card) or the codes."""
+    kernel = qimm.qmatmul_route(t, n, k, m, cus).kernel
+    return (2 * n * k if kernel == qimm.GEMM_BF16_ROWS else n * synth.row_bytes(t, k)), kernel
+
+
+def stage_report(stages, att_flop, qimm, synth, cus):
     """Per-kernel ms, TFLOP/s and roofline fraction from the stage times of the
     block step; the dominant kernel's roofline with its measured HBM traffic."""
     log("bench: stages " + ", ".join(f"{k} {v:.3f}" for k, v in stages.items()) + " ms")
@@ -400,11 +411,11 @@ def stage_report(stages, att_flop, synth):
     kernels = {"attention": {"ms": stages["attention"], "gflop": att_flop / 1e9}}
     for name, (n, k) in gemm.items():
         kernels[name] = {"ms": stages[name], "gflop": 2.0 * S_IMG * n * k / 1e9}
-    qk4 = synth.row_bytes(synth.Q4_K, HID)
-    kernels["qkv"]["weight_bytes"] = 3 * HID * qk4
-    kernels["out_proj"]["weight_bytes"] = HID * qk4
-    kernels["gate_up"]["weight_bytes"] = 2 * MLP * qk4
-    kernels["down"]["weight_bytes"] = HID * synth.row_bytes(synth.Q6_K, MLP)
+    family = {"attention": "attn_fast_kernel"}
+    for name, (n, k) in gemm.items():
+        t = synth.Q6_K if name == "down" else synth.Q4_K
+        kernels[name]["weight_bytes"], kernel = weight_read(qimm, synth, t, n, k, S_IMG, cus)
+        family[name] = {qimm.GEMM_BF16_ROWS: "qgemm_bf16_kernel", qimm.GEMM_WIDE: "qgemm_wide_kernel"}.get(kernel, "qgemm")
     for kname, kd in kernels.items():
         kd["tflops"] = kd["gflop"] / kd["ms"]
         kd["frac_bf16_peak"] = kd["tflops"] / PEAK_BF16_TFLOPS
@@ -413,7 +424,7 @@ def stage_report(stages, att_flop, synth):
         log(f"bench: {kname}: {kd['ms']:.3f} ms, {kd['tflops']:.1f} TFLOP/s")
     dom_name = max(kernels, key=lambda n: kernels[n]["ms"])
     dom = kernels[dom_name]
-    traffic = measured_traffic(dom_name)
+    traffic = measured_traffic(dom_name, family[dom_name])
     roofline = {"kernel": dom_name, "bound": "mfma", "achieved": round(dom["tflops"], 2),
                 "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(dom["tflops"] / PEAK_BF16_TFLOPS, 4),
                 "traffic": traffic["bytes"] if traffic else None, "flop_per_launch": dom["gflop"] * 1e9}
@@ -465,7 +476,8 @@ def q8_gemm_sets(ctx, torch, np, qimm, synth, stream, token_counts=(4352, 256, 6
     activations ~ N(0, 1) of 4352 tokens (the image + prefix rows of a joint
     pass) and of 256, 64 and 16 tokens (the weight-bandwidth regime), bf16
     output. Every call reads its weights from
-    HBM (rotating copies past the last-level cache). Device time per call from
+    HBM (rotating copies past the last-level cache): the bf16 rows or the codes,
+    whichever the kernel of that size reads. Device time per call from
     HIP events on the launch stream."""
     sets = {"qkv": (3 * HID, HID), "out": (HID, HID), "up": (16384, HID), "down": (HID, 16384)}
     out = {}
@@ -489,8 +501,10 @@ def q8_gemm_sets(ctx, torch, np, qimm, synth, stream, token_counts=(4352, 256, 6
             torch.cuda.synchronize()
             ms = e0.elapsed_time(e1) / iters
             tflops = 2.0 * m * n * k / ms / 1e9
-            gbps = wbytes / ms / 1e6
+            rbytes, kernel = weight_read(qimm, synth, synth.Q8_0, n, k, m, compute_units(torch))
+            gbps = rbytes / ms / 1e6
             out[f"{name}_m{m}"] = {"ms": round(ms, 4), "tflops": round(tflops, 1),
+                                   "weights": "bf16 rows" if kernel == qimm.GEMM_BF16_ROWS else "codes",
                                    "frac_bf16_peak": round(tflops / PEAK_BF16_TFLOPS, 4),
                                    "weight_gbps": round(gbps, 1), "frac_hbm": round(gbps / PEAK_HBM_GBPS, 4)}
             log(f"bench: Q8_0 {name} {n}x{k} at {m} tokens: {ms:.3f} ms, {tflops:.0f} TFLOP/s, {gbps:.0f} GB/s")
@@ -796,14 +810,17 @@ def torch_gemm_bar(torch, stream, iters=10):
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_block_q4km_1024.json")
 
 
-def measured_traffic(kernel):
+def measured_traffic(kernel, family):
     """HBM bytes per launch of `kernel` from the committed rocprofv3 --pmc
     summary (FETCH_SIZE and WRITE_SIZE passes, each scaled by what the counter
-    reads for a plain copy of known size), or None when it holds no figure."""
+    reads for a plain copy of known size), or None when it holds no figure for a
+    kernel of the family that runs here."""
     try:
         with open(TRAFFIC_FILE) as f:
             data = json.load(f)
         k = data["kernels"][kernel]
+        if not k["kernel"].startswith(family):
+            return None
         return {"bytes": int(k["traffic_bytes"]), "source": os.path.relpath(TRAFFIC_FILE, ROOT)}
     except (OSError, KeyError, ValueError):
         return None

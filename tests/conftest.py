@@ -6,7 +6,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PKG = os.path.join(ROOT, "qwen3-image21_amd")
 ORACLE = os.path.join(ROOT, "oracle")
-for p in (PKG, ORACLE, os.path.join(ROOT, "tests")):
+for p in (ROOT, PKG, ORACLE, os.path.join(ROOT, "tests")):
     if p not in sys.path:
         sys.path.insert(0, p)
 

@@ -123,6 +123,19 @@ def _timed(f, time):
     return time.perf_counter() - t0
 
 
+def test_bench_counts_the_weight_bytes_the_kernels_read():
+    """bench.py's weight bytes and traffic are those of the kernels that run: the bf16 rows at
+    the block step's 4096 tokens, the codes at 16; no traffic figure of another kernel."""
+    import bench
+    import synth
+    n, k = 2 * bench.MLP, bench.HID
+    assert bench.weight_read(qimm, synth, synth.Q4_K, n, k, bench.S_IMG, 256) == (2 * n * k, qimm.GEMM_BF16_ROWS)
+    assert bench.weight_read(qimm, synth, synth.Q4_K, n, k, 16, 256) == (n * k // 256 * 144, qimm.GEMM_STREAM)
+    t = bench.measured_traffic("gate_up", "qgemm_bf16_kernel")
+    assert t and t["bytes"] > 2 * n * k
+    assert bench.measured_traffic("gate_up", "no_such_kernel") is None
+
+
 def test_qmatmul_route_codes():
     lib = qimm.load()
     r = qimm.GemmRoute()
