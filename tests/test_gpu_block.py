@@ -120,7 +120,7 @@ def check(got, ref, x, exact=False):
                                                  (synth.Q6_K, synth.Q4_K)])
 @pytest.mark.parametrize("b,s,p", [(1, 16, 8), (2, 24, 16),  # M <= 64: split-K weight-streaming GEMM
                                    (1, 96, 40), (2, 64, 64), (1, 130, 0),
-                                   # M >= 512 takes the 256x256 GEMM: partial tiles, a batch
+                                   # more than one tile of tokens: partial tiles, a batch
                                    # boundary inside a tile, S % 4 != 0, and sequences shorter
                                    # than a tile (three in one tile)
                                    (1, 520, 24), (2, 300, 16), (1, 514, 0), (3, 200, 8)])
@@ -517,7 +517,7 @@ def test_attention_q8_0_rounding_in_epilogue_bit_identical(torch_cuda, qctx, mon
     (QIMM_SEPARATE_ROUNDING=1): bit-identical block outputs. Cases: config 1
     (hidden 3072, 24 heads, MLP 9216, 256 tokens over 64: the 4-wave fast
     kernel) and a prefix and token count that are not multiples of 8 (the
-    any-length kernel)."""
+    exact form of the softmax)."""
     if case == "config1_fast_4wave":
         cfg, b, s, p = dict(hidden=3072, heads=24, head_dim=128, mlp=9216), 1, 256, 64
     else:

@@ -424,7 +424,7 @@ def _attention_case(torch, qctx, b, h, sq, p, so, seed, qmul=1.0):
 
 @pytest.mark.parametrize("b,h,sq,p,so,qmul", [
     (1, 2, 128, 64, 128, 1.0),    # aligned
-    (1, 2, 200, 70, 200, 1.0),    # ragged query tile, unaligned prefix (per-element V^T path)
+    (1, 2, 200, 70, 200, 1.0),    # ragged query tile, a prefix that ends inside a V^T chunk
     (2, 3, 64, 256, 96, 1.0),     # batch 2, prefix longer than own; own tail window slides back
     (1, 1, 33, 0, 45, 1.0),       # no prefix, odd lengths
     (1, 2, 16, 8, 8, 1.0),        # tiny: both segments shorter than one 64-key block
